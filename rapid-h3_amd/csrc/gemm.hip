@@ -26,21 +26,14 @@
 // epilogue writes 8-byte bf16 vectors along n. Workgroups are mapped XCD-aware: consecutive
 // workgroup ids land on different XCDs, so the tile order is remapped to give every XCD a
 // contiguous run of tiles that walk N fastest (one activation panel stays in that XCD's L2).
-#include "rh3_common.hpp"
-#include "attn_layout.hpp"
-#include "attn_prologue.hpp"
+#include "gemm_common.hpp"
 
 namespace rh3 {
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v16f __attribute__((ext_vector_type(16)));
+using namespace gemm;
 
-enum Epi { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_GATED = 2, EPI_ACC = 3, EPI_QKV = 4, EPI_GATED_ROWS = 5 };
-
-constexpr int BM = 256, BN = 256, BK = 64;
+constexpr int BM = 256, BN = 256;
 // NW waves in a 2 (m) x NW/2 (n) grid, 128 x (512 / NW) outputs per wave. The library builds NW = 8 (GEMM_NW):
 // 2 waves per SIMD hide each other's LDS and barrier latency. (One wave per SIMD with 128 x 128 outputs, NW = 4,
 // reads a third less LDS per MFMA but measured slower; its branches below are not instantiated.)
@@ -52,95 +45,6 @@ struct Cfg {
 };
 constexpr int GROUP_M = 4;
 constexpr int TILE_BYTES = BM * BK;  // per operand per stage (BM == BN)
-
-// EPI_QKV operands (pointers into the attention workspace of the chosen numerics)
-struct QkvPrep {
-  int64_t H, Spad;           // heads, tokens padded to 128
-  int mode;                  // 0: one Q scale per (head, 128-token block); 1: per token after the H128 rotation
-  int rotate;
-  attn::RR rq, rk;           // q / k RMSNorm + RoPE (tab null: none)
-  int8_t* q8;                // [H][Spad][128]
-  float* qs;                 // mode 0: [H][Spad/128]; mode 1: [H][Spad]
-  double* kpart;             // [H][nchunk][128] channel sums of the (RMSNorm + RoPE'd) k
-  double* vsum;              // mode 1: [H][nchunk][128]
-  float* vmax;
-  float* vmin;
-};
-
-struct GemmArgs {
-  const int8_t* x;  // [M, K] int8 or e4m3 codes
-  int64_t ldx;
-  const int8_t* w;  // [N, K]
-  int64_t ldw;
-  const float* xs;
-  const float* ws;
-  const uint16_t* bias;
-  const uint16_t* gate;
-  void* out;  // bf16 out / resid / int32 acc
-  int64_t ldo;
-  int64_t M, N, K;
-  int tiles_m, tiles_n;
-  QkvPrep qp;
-  const int32_t* gidx;  // EPI_GATED_ROWS: gate table row of each output row (the gate is [R, ldg] bf16)
-  int64_t ldg;
-  int* ctr;  // persistent kernel: per-XCD tile counters (8 ints, zero at launch) or null (fixed tile shares)
-};
-
-// 16-byte chunk c (0..3) of LDS row r: rows r, r+1 share a 128-byte line; the XOR keeps 16
-// consecutive rows of one chunk column on 16 distinct 16-byte bank groups.
-__device__ __forceinline__ int swz(int r, int c) {
-  return r * BK + ((c ^ (((r >> 1) & 3) ^ ((r >> 3) & 1))) << 4);
-}
-
-// g * sigmoid(g) * u with the sigmoid's reciprocal on v_rcp_f32 (1 ulp) instead of the IEEE division
-// sequence (~10 instructions): the exp is approximate on both sides already, so the bf16 result moves by at
-// most one ulp on a small fraction of elements, the tolerance the SwiGLU epilogue is held to
-__device__ __forceinline__ float silu_mul(float g, float u) {
-  const float sig = __builtin_amdgcn_rcpf(1.0f + __expf(-g));
-  return (g * sig) * u;
-}
-
-// EPI_ACC stores the accumulator registers as they are: int32 values (int8) or fp32 bit patterns (e4m3)
-__device__ __forceinline__ int acc_bits(int v) { return v; }
-__device__ __forceinline__ int acc_bits(float v) { return __builtin_bit_cast(int, v); }
-
-template <bool FP8>
-struct Mma;
-
-template <>
-struct Mma<false> {  // int8: 2 MFMAs of k = 32 per 64-byte step, 16-byte fragments
-  typedef v16i acc_t;
-  static constexpr int KSUB = 2;
-  typedef v4i frag_t;
-  __device__ static frag_t load(const int8_t* lds, int row, int ks, int g) {
-    return *reinterpret_cast<const v4i*>(lds + swz(row, ks * 2 + g));
-  }
-  __device__ static acc_t mma(frag_t a, frag_t b, acc_t c) {
-    return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
-  }
-  __device__ static float val(const acc_t& c, int r) { return static_cast<float>(c[r]); }
-};
-
-template <>
-struct Mma<true> {  // e4m3: 1 MFMA of k = 64 per step, 32-byte fragments (two 16-byte chunks)
-  typedef v16f acc_t;
-  static constexpr int KSUB = 1;
-  typedef v8i frag_t;
-  __device__ static frag_t load(const int8_t* lds, int row, int, int g) {
-    const v4i lo = *reinterpret_cast<const v4i*>(lds + swz(row, 2 * g));
-    const v4i hi = *reinterpret_cast<const v4i*>(lds + swz(row, 2 * g + 1));
-    frag_t f;
-    f[0] = lo[0]; f[1] = lo[1]; f[2] = lo[2]; f[3] = lo[3];
-    f[4] = hi[0]; f[5] = hi[1]; f[6] = hi[2]; f[7] = hi[3];
-    return f;
-  }
-  __device__ static acc_t mma(frag_t a, frag_t b, acc_t c) {
-    // cbsz / blgp type 0 = FP8 E4M3 for both operands; zero scale operands select the unscaled form
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
-  }
-  __device__ static float val(const acc_t& c, int r) { return c[r]; }
-};
-
 
 template <bool FP8, int EPI, int NW>
 __global__ void __launch_bounds__(GEMM_NW * 64, GEMM_NW / 4) gemm_kernel(const GemmArgs a) {
@@ -964,23 +868,32 @@ __global__ void __launch_bounds__(512, 2) gemm_persistent_kernel(const GemmArgs 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no global->LDS load outlives the workgroup
 }
 
+// the rows from r0 on of a call
+GemmArgs rows_from(GemmArgs a, int64_t r0, int64_t out_elem) {
+  a.x += r0 * a.ldx;
+  if (a.xs) a.xs += r0;
+  if (a.gidx) a.gidx += r0;
+  a.out = static_cast<int8_t*>(a.out) + r0 * a.ldo * out_elem;
+  a.M -= r0;
+  return a;
+}
+
+// every row on the 256 x 256 tile
 template <bool FP8, int EPI>
-int run(GemmArgs a, hipStream_t st, const char* name) {
-  if (a.M == 0 || a.N == 0) return RH3_OK;
+int run_256(GemmArgs a, hipStream_t st, const char* name, int64_t cus, bool off32) {
   a.tiles_m = static_cast<int>((a.M + BM - 1) / BM);
   a.tiles_n = static_cast<int>((a.N + BN - 1) / BN);
   const int64_t nb = static_cast<int64_t>(a.tiles_m) * a.tiles_n;
-  RH3_REQUIRE(nb < (1ll << 31), "%s: too many tiles", name);
   if constexpr (EPI != EPI_QKV) {
     const int64_t nk = a.K / BK;
-    const int cus = device_cus();
-    // the persistent kernel's 32-bit lane offsets reach 255 rows of either operand
-    const bool off32 = 255 * a.ldx + 64 < (1ll << 32) && 255 * a.ldw + 64 < (1ll << 32);
     if (nk % 4 == 0 && nk >= 8 && cus > 0 && off32) {
       const int64_t grid = nb < cus ? nb : cus;  // one workgroup per CU (the LDS use admits no second)
-      // the counters are cleared by a fill kernel (no hipMemsetAsync: the call stays graph-safe)
       const dim3 g(static_cast<unsigned>(grid));
-      if (a.ctr != nullptr) {
+      // The tile counters pay from four rounds of tiles on: with fewer, the fill kernel before the GEMM costs more than
+      // the XCDs' imbalance (us, with / without: 756 tiles of K = 7168 320 / 306, 504 of K = 3072 116 / 98, 1,080 of
+      // K = 3072 213 / 217, 1,680 of K = 5376 515 / 536). They are cleared by that fill kernel (no hipMemsetAsync: the
+      // call stays graph-safe).
+      if (a.ctr != nullptr && nb >= 4 * cus) {
         hipLaunchKernelGGL(zero_ctr_kernel, dim3(1), dim3(64), 0, st, a.ctr);
         hipLaunchKernelGGL((gemm_persistent_kernel<FP8, EPI, true>), g, dim3(512), 0, st, a);
       } else {
@@ -992,6 +905,30 @@ int run(GemmArgs a, hipStream_t st, const char* name) {
   hipLaunchKernelGGL((gemm_kernel<FP8, EPI, GEMM_NW>), dim3(static_cast<unsigned>(nb)), dim3(GEMM_NW * 64), 0,
                      st, a);
   return launch_status(name);
+}
+
+template <bool FP8, int EPI>
+int run(GemmArgs a, hipStream_t st, const char* name) {
+  if (a.M == 0 || a.N == 0) return RH3_OK;
+  RH3_REQUIRE((a.M + BM - 1) / BM * ((a.N + BN - 1) / BN) < (1ll << 31), "%s: too many tiles", name);
+  const int64_t cus = device_cus();
+  // the 32-bit lane offsets of the persistent and small-tile kernels reach 255 rows of either operand
+  const bool off32 = 255 * a.ldx + 64 < (1ll << 32) && 255 * a.ldw + 64 < (1ll << 32);
+  if constexpr (EPI != EPI_QKV) {
+    if (off32 && cus > 0) {
+      const TilePlan p = plan_tiles(a.M, a.N, a.K, cus);
+      if (p.tile != TILE_256) {
+        if (p.head > 0) {
+          GemmArgs h = a;
+          h.M = p.head;
+          if (int e = run_256<FP8, EPI>(h, st, name, cus, off32)) return e;
+          a = rows_from(a, p.head, EPI == EPI_ACC ? 4 : 2);
+        }
+        return run_tile(FP8, EPI, p.tile, a, st, name);
+      }
+    }
+  }
+  return run_256<FP8, EPI>(a, st, name, cus, off32);
 }
 
 int check(const char* name, const void* xq, int64_t ldx, const void* wq, int64_t ldw, const void* out, int64_t ldo,

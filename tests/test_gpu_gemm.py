@@ -115,6 +115,49 @@ def test_gemm_persistent_epilogues(dev, m, n, k):
     assert og.rel_l2(got, bf16_to_f32(og.fp8_gemm(fq, xs, fwq, ws))) < 1e-2
 
 
+# shapes of each tile rule on 256 CUs: one round of 128 x 64 (odd k-step counts: the two K halves differ by one), of
+# 128 x 128, of 256 x 128 and of 256 x 192, several rounds of 256 x 192, whole 256 x 256 rounds with the last rows on
+# 128 x 64, and counted 256 x 256 tiles; ragged last rows and columns, a single row, a single k-step
+@pytest.mark.parametrize("m,n,k", [(1, 16, 64), (77, 400, 192), (129, 2064, 320), (130, 8272, 192), (129, 16528, 64),
+                                   (257, 16528, 320), (1029, 15376, 512), (1029, 15376, 1024), (4100, 15616, 512)])
+def test_gemm_tile_rules(dev, m, n, k):
+    """Every epilogue on the tile its shape is given: int8 accumulators and outputs bit-exact, SwiGLU within one bf16
+    ulp, FP8 accumulators within the fp32 rounding of a K-term sum."""
+    from rapid_h3 import gemm
+    rng = np.random.default_rng(m + 3 * n + k)
+    xq = np.clip(np.rint(rng.standard_normal((m, k)) * 30), -127, 127).astype(np.int8)
+    wq = np.clip(np.rint(rng.standard_normal((n, k)) * 30), -127, 127).astype(np.int8)
+    xs = (rng.random((m, 1)) * 1e-3 + 1e-4).astype(np.float32)
+    ws = (rng.random((1, n)) * 1e-3 + 1e-4).astype(np.float32)
+    bias, gate, resid = _bf(rng.standard_normal(n)), _bf(rng.standard_normal((3, n))), _bf(rng.standard_normal((m, n)))
+    rows = rng.integers(0, 3, m).astype(np.int32)
+    xt, wt, xst, wst, gt = (to_dev(t, dev) for t in (xq, wq, xs, ws, gate))
+    acc = og.int8_acc(xq, wq)
+    assert np.array_equal(to_np(gemm.int8_gemm_acc(xt, wt)), acc)
+    y = og.dequant(acc, xs, ws)
+    yb = (y + bf16_to_f32(bias).reshape(1, -1)).astype(np.float32)
+    assert np.array_equal(to_np(gemm.int8_gemm(xt, xst, wt, wst, bias=to_dev(bias, dev))), f32_to_bf16(yb))
+    y16 = f32_to_bf16(y)
+
+    def gated(g):
+        return f32_to_bf16(og.fma_f32(bf16_to_f32(y16), np.broadcast_to(bf16_to_f32(g), y.shape), bf16_to_f32(resid)))
+    rt = to_dev(resid, dev)
+    gemm.int8_gemm_gated_residual(xt, xst, wt, wst, gt[1], rt)
+    assert np.array_equal(to_np(rt), gated(gate[1:2]))
+    rt = to_dev(resid, dev)
+    gemm.int8_gemm_gated_residual_rows(xt, xst, wt, wst, gt, to_dev(rows, dev), rt)
+    assert np.array_equal(to_np(rt), gated(gate[rows]))
+    d = _bf16_ulps(to_np(gemm.int8_gemm_swiglu(xt, xst, wt, wst)), og.swiglu_from_interleaved(y16))
+    assert d.max() <= 1 and (d > 0).mean() < 0.01
+    # codes of magnitude 2^-2..2^1 with 3-bit mantissas: every product is exact in fp32, a K-term fp32 sum in any order
+    # is within K 2^-24 of the sum of magnitudes
+    fq, fwq = (rng.integers(0x28, 0x44, size=t, dtype=np.uint8) | (rng.integers(0, 2, size=t, dtype=np.uint8) << 7)
+               for t in ((m, k), (n, k)))
+    a, b = og.fp8_e4m3_to_f32(fq).astype(np.float64), og.fp8_e4m3_to_f32(fwq).astype(np.float64)
+    got = to_np(gemm.fp8_gemm_acc(to_dev(fq, dev, "fp8"), to_dev(fwq, dev, "fp8"))).astype(np.float64)
+    assert np.all(np.abs(got - a @ b.T) <= k * 2.0 ** -24 * (np.abs(a) @ np.abs(b).T))
+
+
 @pytest.mark.parametrize("m,n,k", [(4500, 4112, 512), (9000, 8200, 256), (700, 784, 1024), (300, 264, 512)])
 def test_gemm_tile_counters(dev, m, n, k):
     """The persistent kernel with per-XCD tile counters (ctr, the Python layer's default) and with the fixed tile
