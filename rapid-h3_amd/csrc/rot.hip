@@ -15,9 +15,10 @@
 // Weights (kernels.py:52-72, quantize_weight mode int8_rot): w @ blockdiag(H256)^T as the fp32 rounding of
 // the exact product (float64 butterflies), then the int8_rowwise quantizer q = rint(w_rot / s).
 //
-// Layout: one wavefront per row; lane l owns the 64-column chunk 64*p + l of pass p, so the H64 part of the
-// transform runs in the lane's registers (three radix-4 stages, H4 x = sum(x) - 2 reverse(x), in float64)
-// and the four chunks of a 256-group sit in one lane quad, combined through quad DPP broadcasts.
+// Layout: activations rotate on the matrix cores, 16 groups of 256 columns per wave (see RotTable below). Weights: one
+// wavefront per row; lane l owns the 64-column chunk 64*p + l of pass p, so the H64 part of the transform runs in the
+// lane's registers (three radix-4 stages, H4 x = sum(x) - 2 reverse(x), in float64) and the four chunks of a 256-group sit
+// in one lane quad, combined through quad DPP broadcasts.
 #include "rh3_common.hpp"
 
 namespace rh3 {
@@ -62,10 +63,10 @@ __device__ __forceinline__ float silu_mul_f(float g, float u) {
 
 // one radix-4 stage of H64 on the elements i, i+S, i+2S, i+3S of every group (exact in float64 for
 // values within 2^38 of each other)
-template <int S>
-__device__ __forceinline__ void h4_stage(double (&d)[64]) {
+template <int S, int N>
+__device__ __forceinline__ void h4_stage(double (&d)[N]) {
 #pragma unroll
-  for (int g = 0; g < 16; ++g) {
+  for (int g = 0; g < N / 4; ++g) {
     const int i = (g / S) * 4 * S + (g % S);
     const double x0 = d[i], x1 = d[i + S], x2 = d[i + 2 * S], x3 = d[i + 3 * S];
     const double t = ((x0 + x1) + x2) + x3;
@@ -78,17 +79,13 @@ __device__ __forceinline__ void h4_stage(double (&d)[64]) {
 }
 
 __device__ __forceinline__ void h64(double (&d)[64]) {
-  h4_stage<1>(d);
-  h4_stage<4>(d);
-  h4_stage<16>(d);
+  h4_stage<1, 64>(d);
+  h4_stage<4, 64>(d);
+  h4_stage<16, 64>(d);
 }
 
 // lane q of every quad receives lane CTRL[2q+1:2q] of the quad (DPP quad_perm; every source lane is inside
 // the quad, so bound_ctrl never applies)
-template <int CTRL>
-__device__ __forceinline__ float quad_f(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
-}
 template <int CTRL>
 __device__ __forceinline__ double quad_d(double v) {
   const uint64_t u = __double_as_longlong(v);
@@ -97,83 +94,160 @@ __device__ __forceinline__ double quad_d(double v) {
   return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
 }
 
-// 8 consecutive modulation-table values at element i (VEC: 16-byte loads, the caller checked alignment)
-template <typename TabT, bool VEC>
-__device__ __forceinline__ void tab8(const void* p, int64_t i, float* t) {
-  if (VEC && sizeof(TabT) == 4) {
-    const float4* q = reinterpret_cast<const float4*>(static_cast<const float*>(p) + i);
-    const float4 u0 = q[0], u1 = q[1];
-    t[0] = u0.x; t[1] = u0.y; t[2] = u0.z; t[3] = u0.w; t[4] = u1.x; t[5] = u1.y; t[6] = u1.z; t[7] = u1.w;
-  } else if (VEC) {
-    unpack8(*reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p) + i), t);
-  } else {
+// ---------------------------------------------------------------- activations on the matrix cores
+typedef float v4f_t __attribute__((ext_vector_type(4)));
+typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
+typedef short v2s_t __attribute__((ext_vector_type(2)));
+typedef unsigned short v2us_t __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ v4f_t mfma_bf16(const uint4 a, const uint4 b, v4f_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf_t, a), __builtin_bit_cast(v8bf_t, b), c, 0, 0, 0);
+}
+
+// A 64-lane wave rotates 16 groups of 256 columns at once: H64 of the four 64-column chunks of a group on
+// v_mfma_f32_16x16x32_bf16 with the group as the matrix column (lane l: group n = l & 15, quarter g = l >> 4), H64 / 8
+// as the constant left operand. In chunk c the lane holds the 16 columns 64 c + 16 g + 8 t + e (t = 0, 1 the two MFMAs
+// of k = 32) and receives the outputs 64 c + 16 T + 4 g + r (T = 0..3 the 16-row tiles of H64, r = 0..3).
+//
+// The sums must be exact before their one rounding to fp32. With E the largest exponent of the group, the bf16 values
+// split into hi (exponent >= E - 10) and lo (the rest, exponent >= E - 21): each part's values are multiples of one
+// power of two, 2^17 (plus 64 terms) below its largest, so every partial sum of the 64 terms fits 24 bits and the fp32
+// accumulation is exact in any order; z = hi + lo is then the correctly rounded sum. A chunk with a nonzero value below
+// 2^(E - 21), or a group whose exponents leave that window of normal numbers (E < 48, E > 245, infinities and NaN
+// among them), takes the float64 butterflies instead (h64_slow): about 1 in 50 of the wave's chunks for normal values
+// with 1 % of the channels x20, 1 in 1000 for normal values.
+//
+// What bounds it: VALU issue (72 % busy at 145,152 x 3072 with RMSNorm + modulation, 4 waves per SIMD), then HBM. With the
+// butterflies of all chunks in float64 a row of 3072 took 1,035 VALU instructions per wave (a third of them float64), now
+// about 500. Measured at 145,152 x 3072: RMSNorm + modulation 0.498 -> 0.397 ms; head-major 22,332 x 7168 0.132 ->
+// 0.102 ms = 4.7 TB/s. The operand table stays in LDS: in registers (32 of them) only 3 waves fit a SIMD (0.495 ms), and a
+// workgroup that walks several tiles spills (0.79 ms).
+//
+// H64 / 8 as that operand: H4[a][b] = -1 where b = 3 - a, +1 elsewhere; row i = 16 T + (l & 15) and column
+// k = 16 g + 8 t + e in base 4, for every lane. A table rather than 32 words computed by each wave (a tenth of its
+// instructions).
+struct RotTable {
+  uint32_t w[8][64][4];   // [4 t + T][lane]: the bf16 pairs e = 0..7
+};
+constexpr RotTable make_rot_table() {
+  RotTable r{};
+  for (int T = 0; T < 4; ++T)
+    for (int t = 0; t < 2; ++t)
+      for (int l = 0; l < 64; ++l)
+        for (int e = 0; e < 8; ++e) {
+          const int i0 = l & 3, i1 = (l >> 2) & 3, g = l >> 4;
+          const uint32_t neg = static_cast<uint32_t>(((e & 3) == 3 - i0) ^ ((e >> 2) + 2 * t == 3 - i1) ^ (g == 3 - T));
+          r.w[4 * t + T][l][e >> 1] |= (0x3e00u | (neg << 15)) << (16 * (e & 1));
+        }
+  return r;
+}
+__device__ constexpr RotTable ROT_TABLE = make_rot_table();
+
+__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(v2us_t, a), __builtin_bit_cast(v2us_t, b)));
+}
+__device__ __forceinline__ uint32_t pk_min_u16(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(v2us_t, a), __builtin_bit_cast(v2us_t, b)));
+}
+__device__ __forceinline__ uint32_t pk_sub_u16(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, static_cast<v2us_t>(__builtin_bit_cast(v2us_t, a) - __builtin_bit_cast(v2us_t, b)));
+}
+// 0xffff in each half whose 16 bits are negative
+__device__ __forceinline__ uint32_t pk_neg_mask(uint32_t a) {
+  return __builtin_bit_cast(uint32_t, static_cast<v2s_t>(__builtin_bit_cast(v2s_t, a) >> 15));
+}
+// the largest of the four lanes l & 15 (+ 16, 32, 48)
+__device__ __forceinline__ uint32_t max_quarters(uint32_t v) {
+  auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  v = max(r[0], r[1]);
+  r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return max(r[0], r[1]);
+}
+
+// one chunk in float64, every sum in the order of h64: radix-4 stages at strides 1 and 4 on the lane's 16 columns, the
+// third across the four quarters by lane shuffles, each result rounded once and then scaled by 1/8 (the rounding of the
+// unscaled sum, overflow to infinity included)
+__device__ __forceinline__ void h64_slow(const uint32_t (&w)[8], float (&z)[16], int lane) {
+  double d[16];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) t[e] = tab_at<TabT>(p, i + e);
+  for (int i = 0; i < 8; ++i) {
+    d[2 * i] = static_cast<double>(__uint_as_float(w[i] << 16));
+    d[2 * i + 1] = static_cast<double>(__uint_as_float(w[i] & 0xffff0000u));
+  }
+  h4_stage<1, 16>(d);
+  h4_stage<4, 16>(d);
+  const int n = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    double x[4] = {0, 0, 0, 0};   // element 4 g + r of the four quarters
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const double v = __shfl(d[4 * i + r], 16 * k + n, 64);
+        x[k] = g == i ? v : x[k];
+      }
+    const double t = ((x[0] + x[1]) + x[2]) + x[3];
+#pragma unroll
+    for (int T = 0; T < 4; ++T) z[4 * T + r] = static_cast<float>(fma(-2.0, x[3 - T], t)) * 0.125f;
   }
 }
 
-// prologue values of the 8 columns c..c+7 of row m (the plain row, silu(g) * u, or the head-major gather)
-template <int KIND>
-__device__ __forceinline__ void prologue8(const RotArgs& a, int64_t m, int64_t c, float* v) {
-  if (KIND == ROT_HEADS) {
-    unpack8(*reinterpret_cast<const uint4*>(a.x + (c >> 7) * a.ld_head + m * a.ldx + (c & 127)), v);
-  } else if (KIND == ROT_SWIGLU) {
-    const uint16_t* p = a.x + m * a.ldx + c;
-    float g[8], u[8];
-    unpack8(*reinterpret_cast<const uint4*>(p), g);
-    unpack8(*reinterpret_cast<const uint4*>(p + a.K), u);
+// The rotation of the lane's group, raw[c][4 t + p] = the chunk's bf16 pairs: y[4 q + T][r] = twice output
+// 64 q + 16 T + 4 g + r (the reference's final halving is folded into the quantization scale, rot_scale). The H4
+// combine of the four chunks is in the reference's order.
+__device__ __forceinline__ void rot_group(const uint4* tab, const uint32_t (&raw)[4][8], int lane, float (&y)[16][4]) {
+  uint32_t mx = 0;
+  uint32_t mn[4];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = silu_mul_f(g[e], u[e]);
-  } else {
-    unpack8(*reinterpret_cast<const uint4*>(a.x + m * a.ldx + c), v);
+  for (int c = 0; c < 4; ++c) {
+    mn[c] = 0xffffffffu;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t t = raw[c][i] & 0x7fff7fffu;
+      mx = pk_max_u16(mx, t);
+      mn[c] = pk_min_u16(mn[c], pk_sub_u16(t, 0x00010001u));   // zeros wrap to 0xffff
+    }
   }
-}
-
-// The fp32 H4 combine of four chunk values z of a lane quad, before the halving: lane q computes
-// t_q = ((sA A + sB B) + sC C) + sD D with (A, B, C, D) its quad's z in the order of the reference's formula for y_q
-// (lanes 0-2: z0, z1, z2, z3; lane 3: z1, z2, z3, z0) and the lane's signs times a power of two (the H64
-// normalization 1/8, applied here instead of to each z). The first term is one v_mul_f32 and each further term one
-// v_fmac_f32 whose first operand arrives through a DPP quad permutation; the products with +-2^-k are exact, so each
-// step is the reference's add or subtract of the scaled z rounded once, and scaling by a power of two commutes with
-// the rounding. Four elements per block; s_nop 1 gives the DPP reads of z the two wait states a VALU write needs
-// before them.
-__device__ __forceinline__ void quad_combine4(const float* z, float sa, float sb, float sc, float sd, float* t) {
-  asm volatile(
-      "s_nop 1\n\t"
-      "v_mul_f32_dpp %0, %4, %11 quad_perm:[0,0,0,1] row_mask:0xf bank_mask:0xf\n\t"
-      "v_mul_f32_dpp %1, %5, %11 quad_perm:[0,0,0,1] row_mask:0xf bank_mask:0xf\n\t"
-      "v_mul_f32_dpp %2, %6, %11 quad_perm:[0,0,0,1] row_mask:0xf bank_mask:0xf\n\t"
-      "v_mul_f32_dpp %3, %7, %11 quad_perm:[0,0,0,1] row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %0, %4, %8 quad_perm:[1,1,1,2] row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %1, %5, %8 quad_perm:[1,1,1,2] row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %2, %6, %8 quad_perm:[1,1,1,2] row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %3, %7, %8 quad_perm:[1,1,1,2] row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %0, %4, %9 quad_perm:[2,2,2,3] row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %1, %5, %9 quad_perm:[2,2,2,3] row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %2, %6, %9 quad_perm:[2,2,2,3] row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %3, %7, %9 quad_perm:[2,2,2,3] row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %0, %4, %10 quad_perm:[3,3,3,0] row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %1, %5, %10 quad_perm:[3,3,3,0] row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %2, %6, %10 quad_perm:[3,3,3,0] row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %3, %7, %10 quad_perm:[3,3,3,0] row_mask:0xf bank_mask:0xf"
-      : "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3])
-      : "v"(z[0]), "v"(z[1]), "v"(z[2]), "v"(z[3]), "v"(sb), "v"(sc), "v"(sd), "v"(sa));
-}
-
-// H64 of the lane's chunk d (bf16 values, exact in float64), rounded once to fp32, then the fp32 H4 combine of
-// the quad's four chunks in the reference's order. The H64 normalization 1/8 rides on the combine's signs: fp32(d)/8
-// is fp32(d/8) (a power-of-two scaling commutes with the rounding; below 2^-126, where the two could differ, every
-// code is 0 and the scale sits at its 1e-12 floor either way; |d| stays below 2^128 for inputs below 2^122, the
-// range in which t = 2 y below is finite too). t = 2 y: the reference's final halving is folded
-// into the quantization scale (rot_scale), which gives the same scale and codes (see there).
-__device__ __forceinline__ void rot_combine(double (&d)[64], float sb, float sc, float sd, float (&t)[64]) {
-  h64(d);
-  float z[64];
+  const uint32_t amax = max_quarters(max(mx >> 16, mx & 0xffffu)), eb = amax & 0x7f80u;
+  const uint32_t thr1 = eb - (10u << 7), thr2 = eb - (21u << 7);   // used only where E >= 48
+  const bool off = amax != 0 && (eb < (48u << 7) || eb > (245u << 7));
+  const uint32_t p1 = amax != 0 ? thr1 * 0x00010001u : 0u;
+  float z[4][16];
 #pragma unroll
-  for (int i = 0; i < 64; ++i) z[i] = static_cast<float>(d[i]);
-  const float qb = sb * 0.125f, qc = sc * 0.125f, qd = sd * 0.125f;
+  for (int c = 0; c < 4; ++c) {
+    const uint32_t m = min(mn[c] >> 16, mn[c] & 0xffffu);   // the least nonzero magnitude - 1 (0xffff: all zero)
+    if (__builtin_amdgcn_ballot_w64(off || (amax != 0 && m + 1 < thr2)) != 0) {
+      h64_slow(raw[c], z[c], lane);
+    } else {
+      uint32_t hi[8], lo[8];
 #pragma unroll
-  for (int i = 0; i < 64; i += 4) quad_combine4(z + i, 0.125f, qb, qc, qd, t + i);
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t s = pk_neg_mask(pk_sub_u16(raw[c][i] & 0x7fff7fffu, p1));
+        lo[i] = raw[c][i] & s;
+        hi[i] = raw[c][i] & ~s;
+      }
+      const uint4 h0 = make_uint4(hi[0], hi[1], hi[2], hi[3]), h1 = make_uint4(hi[4], hi[5], hi[6], hi[7]);
+      const uint4 l0 = make_uint4(lo[0], lo[1], lo[2], lo[3]), l1 = make_uint4(lo[4], lo[5], lo[6], lo[7]);
+#pragma unroll
+      for (int T = 0; T < 4; ++T) {
+        const v4f_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        const uint4 a0 = tab[T * 64 + lane], a1 = tab[(4 + T) * 64 + lane];
+        const v4f_t zh = mfma_bf16(a1, h1, mfma_bf16(a0, h0, zero));
+        const v4f_t zl = mfma_bf16(a1, l1, mfma_bf16(a0, l0, zero));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z[c][4 * T + r] = zh[r] + zl[r];
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const float s01 = z[0][i] + z[1][i];
+    y[i >> 2][i & 3] = (s01 + z[2][i]) - z[3][i];
+    y[4 + (i >> 2)][i & 3] = (s01 - z[2][i]) + z[3][i];
+    y[8 + (i >> 2)][i & 3] = ((z[0][i] - z[1][i]) + z[2][i]) + z[3][i];
+    y[12 + (i >> 2)][i & 3] = ((z[1][i] + z[2][i]) + z[3][i]) - z[0][i];
+  }
 }
 
 // Row scale and quantization multiplier from the largest |t| (t = 2 y). With y = t / 2 the reference computes
@@ -187,220 +261,230 @@ __device__ __forceinline__ float rot_scale(float amax_t, float* inv_half) {
   return s;
 }
 
-// y = the rotated values (times 2) of chunk ch. A lane past the row (valid false; its whole quad is past it) works on
-// chunk 0 of its row instead, an in-bounds read whose results the caller discards.
-template <int KIND>
-__device__ __forceinline__ void rot_act_chunk(const RotArgs& a, int64_t m, int64_t ch, bool valid, float sb, float sc,
-                                              float sd, float (&y)[64]) {
-  double d[64];
-  const int64_t c0 = valid ? ch * 64 : 0;
+// A workgroup of 4 waves holds 64 groups: the K / 256 groups of each of its rows (rot_rows of them), 16 groups per wave.
+constexpr int ROT_GROUPS = 64;
+// row absmax over the waves that share it, then the codes: rint(t * inv_half) by the magic-number add of pack4_codes
+// (|t * inv_half| < 127.5 < 2^22), a 4 x 4 transpose over the quarters (lane g then holds columns 64 q + 16 g .. +15)
+// and 16-byte stores
+__device__ __forceinline__ void rot_row_max(const float (&y)[16][4], uint32_t* rowmax, int row, bool valid, int lane) {
+  float am = 0.0f;
 #pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    float v[8];
-    prologue8<KIND>(a, m, c0 + 8 * t, v);
-    if constexpr (KIND == ROT_SWIGLU) {
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) {  // bf16 round to nearest even (v_cvt_pk_bf16_f32), back to fp32 exactly
-        const uint32_t pk = pk_bf16_hw(v[e], v[e + 1]);
-        d[8 * t + e] = static_cast<double>(__uint_as_float(pk << 16));
-        d[8 * t + e + 1] = static_cast<double>(__uint_as_float(pk & 0xffff0000u));
-      }
-    } else {  // the plain and head-major values are bf16 already: the rounding would give them back unchanged
-#pragma unroll
-      for (int e = 0; e < 8; ++e) d[8 * t + e] = static_cast<double>(v[e]);
-    }
+  for (int i = 0; i < 16; ++i) {
+    am = max3_abs(am, y[i][0], y[i][1]);
+    am = max3_abs(am, y[i][2], y[i][3]);
   }
-  rot_combine(d, sb, sc, sd, y);
+  const uint32_t ab = max_quarters(__float_as_uint(am));   // am >= 0 and never NaN: the bits order like the values
+  if (valid && lane < 16) atomicMax(rowmax + row, ab);
 }
-
-// codes rint(t * inv_half) of the 64 values of a chunk: pack4_codes rounds to nearest even by its magic-number add
-// (|t * inv_half| < 127.5 < 2^22) and packs the low bytes
-__device__ __forceinline__ void store64(int8_t* q, const float (&t)[64], float inv_half) {
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    float n[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) n[e] = t[8 * k + e] * inv_half;
-    *reinterpret_cast<uint2*>(q + 8 * k) = make_uint2(pack4_codes(n), pack4_codes(n + 4));
-  }
-}
-
-// NP = passes of 64 chunks (K <= 4096 * NP). With one pass the rotated values stay in registers between
-// the absmax and the quantization; with more, the values of passes 0..NP-2 wait in LDS (64 floats per
-// lane, lane-interleaved float4s, a private region per wave) until the row scale is known.
-template <int NP> constexpr int rot_waves() { return NP <= 2 ? 4 : 2; }
-
-template <int KIND, int NP>
-__global__ void __launch_bounds__(64 * rot_waves<NP>()) rot_quant_kernel(const RotArgs a) {
-  constexpr int W = rot_waves<NP>();
-  __shared__ float4 stash[NP > 1 ? W * (NP - 1) * 16 * 64 : 1];  // [wave][pass][i / 4][lane]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t m = static_cast<int64_t>(blockIdx.x) * W + wave;
-  if (m >= a.M) return;  // whole wavefront: DPP partners never leave; no workgroup barrier below
-  const int q4 = lane & 3;
-  const float sb = q4 == 2 ? -1.0f : 1.0f, sc = q4 == 1 ? -1.0f : 1.0f, sd = (q4 == 0 || q4 == 3) ? -1.0f : 1.0f;
-  static_assert(KIND != ROT_NORMMOD, "RMSNorm + modulation runs in rot_normmod_kernel");
-  const int64_t nchunks = a.K / 64;
-  float4* my = stash + wave * (NP - 1) * 16 * 64 + lane;
-  float y[64];
-  float amax = 0.0f;
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
-    const int64_t ch = 64 * p + lane;
-    rot_act_chunk<KIND>(a, m, ch, ch < nchunks, sb, sc, sd, y);
-    float am = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 64; i += 2) am = max3_abs(am, y[i], y[i + 1]);
-    if (ch < nchunks) amax = fmaxf(amax, am);
-    if (p < NP - 1) {
-#pragma unroll
-      for (int t = 0; t < 16; ++t) my[(p * 16 + t) * 64] = make_float4(y[4 * t], y[4 * t + 1], y[4 * t + 2], y[4 * t + 3]);
-    }
-  }
-  amax = wave_max(amax);
+__device__ __forceinline__ void rot_store(const RotArgs& a, const float (&y)[16][4], const uint32_t* rowmax, int64_t m, int row,
+                                          int grp, bool valid, int lane) {
+  if (!valid) return;
   float inv;
-  const float s = rot_scale(amax, &inv);
-  if (lane == 0) a.s[m] = s;
-  const int64_t last = 64 * (NP - 1) + lane;
-  if (last < nchunks) store64(a.q + m * a.ldq + 64 * last, y, inv);
+  const float s = rot_scale(__uint_as_float(rowmax[row]), &inv);
+  if (grp == 0 && lane < 16) a.s[m] = s;
+  int8_t* const qp = a.q + m * a.ldq + grp * 256 + 16 * (lane >> 4);
 #pragma unroll
-  for (int p = 0; p < NP - 1; ++p) {
-    const int64_t ch = 64 * p + lane;
+  for (int q = 0; q < 4; ++q) {
+    uint32_t w[4];
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      const float4 u = my[(p * 16 + t) * 64];
-      y[4 * t] = u.x; y[4 * t + 1] = u.y; y[4 * t + 2] = u.z; y[4 * t + 3] = u.w;
+    for (int T = 0; T < 4; ++T) {
+      float n[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) n[r] = y[4 * q + T][r] * inv;
+      w[T] = pack4_codes(n);
     }
-    if (ch < nchunks) store64(a.q + m * a.ldq + 64 * ch, y, inv);
+    auto r02 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+    auto r13 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+    auto lo = __builtin_amdgcn_permlane16_swap(r02[0], r13[0], false, false);
+    auto hi = __builtin_amdgcn_permlane16_swap(r02[1], r13[1], false, false);
+    // two 8-byte halves: the alignment the entry points require of q
+    reinterpret_cast<uint2*>(qp + 64 * q)[0] = make_uint2(lo[0], lo[1]);
+    reinterpret_cast<uint2*>(qp + 64 * q)[1] = make_uint2(hi[0], hi[1]);
   }
 }
 
-// RMSNorm + modulation, rotation and INT8 with the prologue staged through LDS. Phase 1 works in the coalesced
-// layout of the sum of squares (lane l holds columns 512 j + 8 l .. +7): the row, the norm weight and both
-// modulation rows are read with whole-wave 16-byte accesses, the prologue values are computed there (the same
-// operations in the same order as the unrotated quantizer's prologue) and written to the wave's LDS region as bf16,
-// chunk-major with a 144-byte chunk pitch (lanes reading their own chunk then hit 16 distinct bank quads). Phase 2 is
-// the rotation of rot_quant_kernel with each lane's chunk read from LDS instead of gathered from global memory. A wave
-// can walk RPW consecutive rows, issuing the next row's loads before the current row's rotation; that holds the loaded
-// row through the rotation (222 registers, 2 waves per SIMD) and measured slower than one row per wave at 3 waves per
-// SIMD (0.71 vs 0.64 ms at 145,152 x 3072), so RPW is 1. A wave uses only its own LDS region (in order: a row's
-// phase-1 writes follow the previous row's phase-2 reads), so no workgroup barrier is needed.
-constexpr int STAGE_PITCH = 144;
-template <int NP> constexpr int nm_waves() { return NP == 1 ? 4 : (NP == 2 ? 2 : 1); }
-template <int NP> constexpr int nm_rows() { return 1; }
+__device__ __forceinline__ void rot_table_to(uint4* tab) {
+  const uint4* src = reinterpret_cast<const uint4*>(&ROT_TABLE);
+  tab[threadIdx.x] = src[threadIdx.x];
+  tab[256 + threadIdx.x] = src[256 + threadIdx.x];
+}
 
-template <typename TabT, int NP, bool VEC>
-__global__ void __launch_bounds__(64 * nm_waves<NP>()) rot_normmod_kernel(const RotArgs a) {
-  constexpr int W = nm_waves<NP>(), RPW = nm_rows<NP>();
-  __shared__ __attribute__((aligned(16))) uint8_t stage[W * 64 * NP * STAGE_PITCH];
-  __shared__ float4 stash[NP > 1 ? W * (NP - 1) * 16 * 64 : 1];  // [wave][pass][i / 4][lane]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t m0 = (static_cast<int64_t>(blockIdx.x) * W + wave) * RPW;
-  if (m0 >= a.M) return;  // whole wavefront: DPP partners never leave; no workgroup barrier below
-  const int nrows = static_cast<int>(min(static_cast<int64_t>(RPW), a.M - m0));
-  uint8_t* st = stage + wave * 64 * NP * STAGE_PITCH;
-  const int q4 = lane & 3;
-  const float sb = q4 == 2 ? -1.0f : 1.0f, sc = q4 == 1 ? -1.0f : 1.0f, sd = (q4 == 0 || q4 == 3) ? -1.0f : 1.0f;
-  const int64_t nchunks = a.K / 64;
-  float4* my = stash + wave * (NP - 1) * 16 * 64 + lane;
-  // the row's loads, all issued before the first product (K <= 4096 * NP, so j < 8 * NP)
-  uint4 r[8 * NP];
-  auto load_row = [&](int64_t m) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < 8 * NP; ++j) {
-      const int64_t c = 512 * j + 8 * lane;
-      r[j] = c < a.K ? *reinterpret_cast<const uint4*>(a.x + m * a.ldx + c) : make_uint4(0, 0, 0, 0);
-    }
+// the rows of a workgroup
+__host__ __device__ inline int rot_rows(int64_t K) { return static_cast<int>(ROT_GROUPS * 256 / K); }
+
+// Plain, head-major and SwiGLU rows, read straight from global memory: lane (n, g) takes 32 bytes of each 128-byte
+// chunk line of its group, four lanes a line.
+template <int KIND>
+__global__ void __launch_bounds__(256, 4) rot_quant_kernel(const RotArgs a) {
+  static_assert(KIND != ROT_NORMMOD, "RMSNorm + modulation runs in rot_normmod_kernel");
+  __shared__ uint4 tab[8 * 64];
+  __shared__ uint32_t rowmax[ROT_GROUPS];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
+  const int G = static_cast<int>(a.K >> 8), R = rot_rows(a.K);
+  const int gi = wave * 16 + n, row = gi / G, grp = gi - row * G;
+  const int64_t m0 = static_cast<int64_t>(blockIdx.x) * R, m = m0 + row;
+  const bool valid = row < R && m < a.M;
+  if (threadIdx.x < ROT_GROUPS) rowmax[threadIdx.x] = 0;
+  rot_table_to(tab);
+  __syncthreads();
+  // a lane with no group of its own works on the first group of the workgroup's first row (in bounds) and stores nothing
+  const int64_t ml = valid ? m : m0;
+  const int gl = valid ? grp : 0;
+  uint32_t raw[4][8];
+  auto load16 = [&](const uint16_t* p, uint32_t* w) __attribute__((always_inline)) {
+    const uint4 u0 = reinterpret_cast<const uint4*>(p)[0], u1 = reinterpret_cast<const uint4*>(p)[1];
+    w[0] = u0.x; w[1] = u0.y; w[2] = u0.z; w[3] = u0.w;
+    w[4] = u1.x; w[5] = u1.y; w[6] = u1.z; w[7] = u1.w;
   };
-  load_row(m0);
-  for (int ri = 0; ri < nrows; ++ri) {
-    const int64_t m = m0 + ri;
-    const int64_t trow = static_cast<int64_t>(a.idx[m]) * a.ld_tab;
-    // phase 1. Sum of squares in the order of quant.hip (lane chunks 512 j + 8 l, (j, e) sequential, butterfly)
-    float xv[8 * NP][8];
+  if constexpr (KIND == ROT_SWIGLU) {
+    const uint16_t* p = a.x + ml * a.ldx + gl * 256 + 16 * g;
+    uint32_t up[4][8];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      load16(p + 64 * c, raw[c]);
+      load16(p + 64 * c + a.K, up[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        raw[c][i] = pk_bf16_hw(silu_mul_f(__uint_as_float(raw[c][i] << 16), __uint_as_float(up[c][i] << 16)),
+                               silu_mul_f(__uint_as_float(raw[c][i] & 0xffff0000u), __uint_as_float(up[c][i] & 0xffff0000u)));
+  } else if constexpr (KIND == ROT_HEADS) {
+    const uint16_t* p = a.x + 2 * gl * a.ld_head + ml * a.ldx + 16 * g;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) load16(p + (c >> 1) * a.ld_head + 64 * (c & 1), raw[c]);
+  } else {
+    const uint16_t* p = a.x + ml * a.ldx + gl * 256 + 16 * g;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) load16(p + 64 * c, raw[c]);
+  }
+  float y[16][4];
+  rot_group(tab, raw, lane, y);
+  rot_row_max(y, rowmax, row, valid, lane);
+  __syncthreads();
+  rot_store(a, y, rowmax, m, row, grp, valid, lane);
+}
+
+// RMSNorm + modulation, rotation and INT8. Phase 1, a wave per row in the coalesced layout of the sum of squares (lane
+// l holds columns 512 j + 8 l .. +7, the order of quant.hip): the row, the norm weight and both modulation rows are
+// read with whole-wave 16-byte accesses, and the prologue values go to LDS as bf16, group-major, 16-byte unit u of
+// group i at u ^ (i & 15), so that both phases' accesses spread over the banks. Phase 2 is the rotation of
+// rot_quant_kernel from there.
+template <typename TabT, int NCH, bool VEC>
+__global__ void __launch_bounds__(256, 4) rot_normmod_kernel(const RotArgs a) {
+  extern __shared__ uint4 stage[];   // 32 units of 16 bytes per group of the workgroup's rows
+  __shared__ uint4 tab[8 * 64];
+  __shared__ uint32_t rowmax[ROT_GROUPS];
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int G = static_cast<int>(a.K >> 8), R = min(4, rot_rows(a.K));   // one row per wave
+  const int64_t m0 = static_cast<int64_t>(blockIdx.x) * R;
+  if (threadIdx.x < ROT_GROUPS) rowmax[threadIdx.x] = 0;
+  rot_table_to(tab);
+  if (wave < R && m0 + wave < a.M) {
+    // every row operand through a buffer resource (the row's base in scalar registers, its size as the range check: lanes
+    // past K read zeros), so the loop has fixed 32-bit lane offsets and no branch
+    const int64_t m = m0 + wave;
+    const int K = static_cast<int>(a.K);
+    constexpr int TB = sizeof(TabT);
+    const int64_t trow = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(a.idx[m])) * a.ld_tab;
+    auto rsrc = [](const void* p, int bytes) __attribute__((always_inline)) {
+      return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, BUF_RSRC_WORD3);
+    };
+    const __amdgpu_buffer_rsrc_t rx = rsrc(a.x + m * a.ldx, 2 * K), rw = rsrc(a.w, a.w ? 2 * K : 0);
+    const __amdgpu_buffer_rsrc_t rsc = rsrc(static_cast<const TabT*>(a.scale) + trow, TB * K);
+    const __amdgpu_buffer_rsrc_t rsh = rsrc(static_cast<const TabT*>(a.shift) + trow, TB * K);
+    auto load16 = [](const __amdgpu_buffer_rsrc_t r, int off, int s) __attribute__((always_inline)) {
+      const u32x4_t t = __builtin_amdgcn_raw_buffer_load_b128(r, off, s, 0);
+      return make_uint4(t[0], t[1], t[2], t[3]);
+    };
+    auto load_at = [&](int j) __attribute__((always_inline)) { return load16(rx, 16 * lane, 1024 * j); };
+    auto table_at = [&](const __amdgpu_buffer_rsrc_t r, const void* p, int j, float* t) __attribute__((always_inline)) {
+      if constexpr (VEC && TB == 4) {
+        const uint4 u0 = load16(r, 32 * lane, 2048 * j), u1 = load16(r, 32 * lane + 16, 2048 * j);
+        t[0] = __uint_as_float(u0.x); t[1] = __uint_as_float(u0.y); t[2] = __uint_as_float(u0.z); t[3] = __uint_as_float(u0.w);
+        t[4] = __uint_as_float(u1.x); t[5] = __uint_as_float(u1.y); t[6] = __uint_as_float(u1.z); t[7] = __uint_as_float(u1.w);
+      } else if constexpr (VEC) {
+        unpack8(load16(r, 16 * lane, 1024 * j), t);
+      } else {  // rows that are not 16-byte aligned
+        const int64_t c = 512 * j + 8 * lane;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t[e] = c < a.K ? tab_at<TabT>(p, trow + c + e) : 0.0f;
+      }
+    };
     float ss = 0.0f;
+    auto add_squares = [&](const uint4 r) __attribute__((always_inline)) {
+      float v[8];
+      unpack8(r, v);
 #pragma unroll
-    for (int j = 0; j < 8 * NP; ++j) {
-      unpack8(r[j], xv[j]);
+      for (int e = 0; e < 8; ++e) ss = fmaf(v[e], v[e], ss);  // x * x is exact (bf16 x): = ss + x * x
+    };
+    float rstd = 0.0f;
+    const bool has_w = a.w != nullptr;
+    auto modulate = [&](const uint4 r, int j) __attribute__((always_inline)) {
+      float v[8], scl[8], shf[8];
+      unpack8(r, v);
+      table_at(rsc, a.scale, j, scl);
+      table_at(rsh, a.shift, j, shf);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) ss = fmaf(xv[j][e], xv[j][e], ss);  // x * x is exact (bf16 x): = ss + x * x
-    }
-    if (ri + 1 < nrows) load_row(m + 1);
-    ss = wave_sum_tree(ss);
-    const float rstd = 1.0f / sqrtf(ss / static_cast<float>(a.K) + a.eps);
+      for (int e = 0; e < 8; ++e) v[e] = v[e] * rstd;
+      if (has_w) {
+        float wv[8];
+        unpack8(load16(rw, 16 * lane, 1024 * j), wv);
 #pragma unroll
-    for (int j = 0; j < 8 * NP; ++j) {
-      const int64_t c = 512 * j + 8 * lane;
-      if (c < a.K) {
-        float* v = xv[j];
-        float wv[8], scl[8], shf[8];
-        if (a.w) unpack8(*reinterpret_cast<const uint4*>(a.w + c), wv);
-        tab8<TabT, VEC>(a.scale, trow + c, scl);
-        tab8<TabT, VEC>(a.shift, trow + c, shf);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          float y = v[e] * rstd;
-          if (a.w) y = y * wv[e];
-          v[e] = y * (1.0f + scl[e]) + shf[e];
-        }
-        uint4 o;
-        o.x = pk_bf16_hw(v[0], v[1]);
-        o.y = pk_bf16_hw(v[2], v[3]);
-        o.z = pk_bf16_hw(v[4], v[5]);
-        o.w = pk_bf16_hw(v[6], v[7]);
-        *reinterpret_cast<uint4*>(st + (c >> 6) * STAGE_PITCH + (c & 63) * 2) = o;
+        for (int e = 0; e < 8; ++e) v[e] = v[e] * wv[e];
       }
-    }
-    // the wave's own LDS writes are complete before its lanes read each other's columns
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_wave_barrier();
-    // phase 2: lane l rotates chunk 64 p + l
-    float y[64];
-    float amax = 0.0f;
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int64_t ch = 64 * p + lane;
-      // a lane past the row (its whole quad is) reads its slot of the wave's region all the same (ch < 64 NP) and
-      // its results are discarded
-      double d[64];
-      const uint8_t* src = st + ch * STAGE_PITCH;
+      for (int e = 0; e < 8; ++e) v[e] = v[e] * (1.0f + scl[e]) + shf[e];
+      const int i = wave * G + 2 * j + (lane >> 5);
+      if (512 * j + 8 * lane < K)
+        stage[i * 32 + ((lane & 31) ^ (i & 15))] =
+            make_uint4(pk_bf16_hw(v[0], v[1]), pk_bf16_hw(v[2], v[3]), pk_bf16_hw(v[4], v[5]), pk_bf16_hw(v[6], v[7]));
+    };
+    auto finish = [&]() __attribute__((always_inline)) {
+      ss = wave_sum_tree(ss);
+      rstd = 1.0f / sqrtf(ss / static_cast<float>(a.K) + a.eps);
+    };
+    if constexpr (NCH > 0) {
+      uint4 r[NCH];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const uint4 u = *reinterpret_cast<const uint4*>(src + 16 * t);
-        const uint32_t w4[4] = {u.x, u.y, u.z, u.w};
+      for (int j = 0; j < NCH; ++j) r[j] = load_at(j);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          d[8 * t + 2 * e] = static_cast<double>(__uint_as_float(w4[e] << 16));
-          d[8 * t + 2 * e + 1] = static_cast<double>(__uint_as_float(w4[e] & 0xffff0000u));
-        }
-      }
-      rot_combine(d, sb, sc, sd, y);
-      float am = 0.0f;
+      for (int j = 0; j < NCH; ++j) add_squares(r[j]);
+      finish();
 #pragma unroll
-      for (int i = 0; i < 64; i += 2) am = max3_abs(am, y[i], y[i + 1]);
-      if (ch < nchunks) amax = fmaxf(amax, am);
-      if (p < NP - 1) {
-#pragma unroll
-        for (int t = 0; t < 16; ++t) my[(p * 16 + t) * 64] = make_float4(y[4 * t], y[4 * t + 1], y[4 * t + 2], y[4 * t + 3]);
-      }
-    }
-    amax = wave_max(amax);
-    float inv;
-    const float s = rot_scale(amax, &inv);
-    if (lane == 0) a.s[m] = s;
-    const int64_t last = 64 * (NP - 1) + lane;
-    if (last < nchunks) store64(a.q + m * a.ldq + 64 * last, y, inv);
-#pragma unroll
-    for (int p = 0; p < NP - 1; ++p) {
-      const int64_t ch = 64 * p + lane;
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        const float4 u = my[(p * 16 + t) * 64];
-        y[4 * t] = u.x; y[4 * t + 1] = u.y; y[4 * t + 2] = u.z; y[4 * t + 3] = u.w;
-      }
-      if (ch < nchunks) store64(a.q + m * a.ldq + 64 * ch, y, inv);
+      for (int j = 0; j < NCH; ++j) modulate(r[j], j);
+    } else {  // the row does not fit the registers: read twice, the second time from L2
+      const int nch = (K + 511) / 512;
+#pragma unroll 4
+      for (int j = 0; j < nch; ++j) add_squares(load_at(j));
+      finish();
+#pragma unroll 2
+      for (int j = 0; j < nch; ++j) modulate(load_at(j), j);
     }
   }
+  __syncthreads();
+  const int gi = wave * 16 + n, row = gi / G, grp = gi - row * G;
+  const int64_t m = m0 + row;
+  const bool valid = row < R && m < a.M;
+  const int il = valid ? gi : 0;   // lanes with no group of their own: group 0, nothing stored
+  float y[16][4];
+  const bool work = wave * 16 < R * G;   // the whole wave's groups may lie past the rows (it still meets the barrier)
+  if (work) {
+    uint32_t raw[4][8];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const uint4 u = stage[il * 32 + ((8 * c + 2 * g + t) ^ (il & 15))];
+        raw[c][4 * t] = u.x; raw[c][4 * t + 1] = u.y; raw[c][4 * t + 2] = u.z; raw[c][4 * t + 3] = u.w;
+      }
+    rot_group(tab, raw, lane, y);
+    rot_row_max(y, rowmax, row, valid, lane);
+  }
+  __syncthreads();
+  if (work) rot_store(a, y, rowmax, m, row, grp, valid, lane);
 }
 
 // ---------------------------------------------------------------- exact H256 rotation of weights
@@ -516,24 +600,19 @@ __global__ void __launch_bounds__(256) rot_exact_kernel(const ExactArgs a) {
 
 template <typename TabT, bool VEC>
 void launch_normmod(const RotArgs& a, hipStream_t st) {
-  if (a.K <= 4096)
-    hipLaunchKernelGGL((rot_normmod_kernel<TabT, 1, VEC>), dim3(static_cast<unsigned>((a.M + 3) / 4)), dim3(256), 0, st,
-                       a);
-  else if (a.K <= 8192)
-    hipLaunchKernelGGL((rot_normmod_kernel<TabT, 2, VEC>), dim3(static_cast<unsigned>((a.M + 1) / 2)), dim3(128), 0, st,
-                       a);
-  else
-    hipLaunchKernelGGL((rot_normmod_kernel<TabT, 4, VEC>), dim3(static_cast<unsigned>(a.M)), dim3(64), 0, st, a);
+  const int64_t R = rot_rows(a.K) < 4 ? rot_rows(a.K) : 4;
+  const dim3 grid(static_cast<unsigned>((a.M + R - 1) / R)), block(256);
+  const unsigned lds = static_cast<unsigned>(R * (a.K / 256) * 512);
+  // the 512-column chunks of a row that a lane holds (wider rows are read twice)
+  if (a.K <= 3072) hipLaunchKernelGGL((rot_normmod_kernel<TabT, 6, VEC>), grid, block, lds, st, a);
+  else if (a.K <= 6144) hipLaunchKernelGGL((rot_normmod_kernel<TabT, 12, VEC>), grid, block, lds, st, a);
+  else hipLaunchKernelGGL((rot_normmod_kernel<TabT, 0, VEC>), grid, block, lds, st, a);
 }
 
 template <int KIND>
 void launch_rot(const RotArgs& a, hipStream_t st) {
-  if (a.K <= 4096)
-    hipLaunchKernelGGL((rot_quant_kernel<KIND, 1>), dim3(static_cast<unsigned>((a.M + 3) / 4)), dim3(256), 0, st, a);
-  else if (a.K <= 8192)
-    hipLaunchKernelGGL((rot_quant_kernel<KIND, 2>), dim3(static_cast<unsigned>((a.M + 3) / 4)), dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL((rot_quant_kernel<KIND, 4>), dim3(static_cast<unsigned>((a.M + 1) / 2)), dim3(128), 0, st, a);
+  const int64_t R = rot_rows(a.K);
+  hipLaunchKernelGGL((rot_quant_kernel<KIND>), dim3(static_cast<unsigned>((a.M + R - 1) / R)), dim3(256), 0, st, a);
 }
 
 template <int KIND, typename TabT>

@@ -139,6 +139,54 @@ def test_rot_extreme_magnitudes(dev):
     _eq(q, s, eq, es)
 
 
+# rows per workgroup and row widths at their edges: 64 groups of 256 columns per workgroup (at most four rows with the
+# RMSNorm prologue, whose lanes hold 6 or 12 chunks of 512 columns or read the row twice), ragged last workgroups
+@pytest.mark.parametrize("m,k", [(1, 256), (65, 256), (5, 2816), (9, 3072), (7, 3328), (4, 6144), (5, 6400), (3, 7168),
+                                 (2, 8448), (2, 16384)])
+def test_rot_exact_window(dev, m, k):
+    """The matrix-core sums against the oracle's float64 ones, bit for bit, where a 256-group's values span the split: 1 %
+    of the columns x 2^13 (both parts used), every seventh row scaled column by column over 2^+-24 (values below the
+    window: the float64 path), rows of zeros and of one nonzero value."""
+    import torch
+    from rapid_h3 import quant
+    rng = np.random.default_rng(m + k)
+    x = rng.standard_normal((m, k))
+    x[:, rng.permutation(k)[:max(1, k // 100)]] *= 2.0 ** 13
+    x[::7] *= 2.0 ** rng.integers(-24, 25, (1, k))
+    if m > 2:
+        x[1] = 0
+        x[2] = 0
+        x[2, k // 2] = 3.0
+    xb = f32_to_bf16(x.astype(np.float32))
+    xt = to_dev(xb, dev)
+    _eq(*quant.rot_quant_rows_i8(xt), *oq.rot_quant_rows_i8(xb))
+    o = np.ascontiguousarray(xb.reshape(m, k // 128, 128).transpose(1, 0, 2))
+    _eq(*quant.rot_quant_heads_i8(to_dev(o, dev)), *oq.rot_quant_heads_i8(o))
+    w = f32_to_bf16((1 + 0.3 * rng.standard_normal(k)).astype(np.float32))
+    idx = rng.integers(0, 3, m).astype(np.int32)
+    for pad in (0, 1):   # 16-byte table rows, and rows that are not
+        tab = [(0.1 * rng.standard_normal((3, k + pad))).astype(np.float32) for _ in range(2)]
+        for wn in (w, None):
+            got = quant.norm_mod_rot_quant_rows_i8(xt, None if wn is None else to_dev(wn, dev), 1e-6, to_dev(idx, dev),
+                                                   *(to_dev(t, dev)[:, :k] for t in tab))
+            _eq(*got, *oq.norm_mod_rot_quant_rows_i8(xb, wn, 1e-6, idx, *(np.ascontiguousarray(t[:, :k]) for t in tab)))
+
+
+def test_rot_non_finite(dev):
+    """An infinity sets its row's scale to infinity and every code to 0; a NaN takes its 256-group's codes to 0 and leaves
+    the rest of the row as if the group were zero."""
+    import torch
+    from rapid_h3 import quant
+    x = torch.randn(4, 768, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16)
+    ref = x.clone()
+    x[1, 300], x[2, 300], x[3, 5] = float("inf"), float("nan"), float("-inf")
+    ref[2, 256:512] = 0
+    q, s = quant.rot_quant_rows_i8(x.to(dev))
+    eq, es = quant.rot_quant_rows_i8(ref.to(dev))
+    assert torch.equal(q[[0, 2]], eq[[0, 2]]) and torch.equal(s[[0, 2]], es[[0, 2]])
+    assert torch.isinf(s[[1, 3]]).all() and (q[[1, 3]] == 0).all()
+
+
 def test_rot_strided_rows(dev):
     from rapid_h3 import quant
     rng = np.random.default_rng(7)
