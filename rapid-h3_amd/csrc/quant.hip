@@ -79,6 +79,37 @@ __device__ __forceinline__ uint32_t fp8_e4m3(float t) {
   return code | sign;
 }
 
+// 8 e4m3 codes of clamp(x / s, +-448) (IEEE quotient) packed little-endian. Two residual steps on x * inv give the
+// correctly rounded quotient (inv = 1 / s is the correctly rounded reciprocal and no intermediate leaves the normal range
+// where the code depends on it: |x / s| >= 2^-11 with s in [2^-60, 2^60]); the hardware conversion rounds to nearest even.
+// The residual is taken as t s - x, which keeps the sign of a zero.
+// odd: the row's scale is outside that range or its absmax not finite; those rows take the division and the software
+// encoder. With those for every value the kernel ran at 3.5 TB/s, bound by VALU: 145,152 x 3072 387 -> 212 us, the int8 form's time. (A vote on
+// x * inv being near a rounding boundary, as in quant8_i8, does not pay: the quotients of two 8-bit significands are
+// exactly on one so often that two in five votes fail, 422 us.)
+__device__ __forceinline__ bool fp8_odd_row(float amax, float s) { return !(amax < INFINITY && s >= 0x1p-60f && s <= 0x1p60f); }
+__device__ __forceinline__ uint2 quant8_fp8(const float* x, float s, float inv, bool odd) {
+  if (odd) {
+    uint32_t b[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) b[e] = fp8_e4m3(fminf(fmaxf(x[e] / s, -448.0f), 448.0f));
+    return make_uint2(b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24), b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24));
+  }
+  float t[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    t[e] = x[e] * inv;
+    t[e] = fmaf(fmaf(t[e], s, -x[e]), -inv, t[e]);
+    // a NaN becomes -448 (v_med3_f32 then returns the least of the others), as fminf(fmaxf()) makes it
+    t[e] = __builtin_amdgcn_fmed3f(fmaf(fmaf(t[e], s, -x[e]), -inv, t[e]), -448.0f, 448.0f);
+  }
+  int lo = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);
+  lo = __builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], lo, true);
+  int hi = __builtin_amdgcn_cvt_pk_fp8_f32(t[4], t[5], 0, false);
+  hi = __builtin_amdgcn_cvt_pk_fp8_f32(t[6], t[7], hi, true);
+  return make_uint2(static_cast<uint32_t>(lo), static_cast<uint32_t>(hi));
+}
+
 // 16-byte row loads; STREAM: the row is read once (streaming hint), else it may be read again from L2
 template <bool STREAM>
 __device__ __forceinline__ uint4 ld_row16(const uint16_t* p) {
@@ -195,11 +226,7 @@ __global__ void __launch_bounds__(256) quant_rows_kernel(const QuantArgs a) {
     vals(j, x);
     uint2 out;
     if (FP8) {
-      uint32_t b[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) b[e] = fp8_e4m3(fminf(fmaxf(x[e] / s, -448.0f), 448.0f));
-      out.x = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
-      out.y = b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24);
+      out = quant8_fp8(x, s, inv, fp8_odd_row(amax, s));
     } else {
       out = quant8_i8(x, s, inv);
     }
@@ -448,11 +475,7 @@ __global__ void __launch_bounds__(256) quant_rows_split_kernel(const QuantArgs a
     unpack8(raw[i], x);
     uint2 out;
     if (FP8) {
-      uint32_t b[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) b[e] = fp8_e4m3(fminf(fmaxf(x[e] / s, -448.0f), 448.0f));
-      out.x = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
-      out.y = b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24);
+      out = quant8_fp8(x, s, inv, fp8_odd_row(amax, s));
     } else {
       out = quant8_i8(x, s, inv);
     }

@@ -43,6 +43,30 @@ def test_quant_rows_shapes(dev, m, k):
         assert np.array_equal(to_np(s), es), (m, k, fp8)
 
 
+@pytest.mark.parametrize("k", [8, 3072, 8192])
+def test_quant_fp8_quotients(dev, k):
+    """FP8 codes where the quotient decides them, bit for bit: row absmax of every bf16 significand (small-denominator
+    ratios hit rounding boundaries exactly), scales at the ends of the fast quotient's range and past them, zeros of both
+    signs, and rows with an infinity or a NaN (the reference's clamp takes a NaN to -448)."""
+    rng = np.random.default_rng(k)
+    x = rng.standard_normal((140, k)) * 0.2
+    x[np.arange(128), rng.integers(0, k, 128)] = np.arange(128, 256) / 256.0 * np.where(rng.random(128) < 0.5, -4, 4)
+    x[128] *= 2.0 ** -53
+    x[129] *= 2.0 ** -70
+    x[130] *= 2.0 ** 66
+    x[131] *= 2.0 ** 120
+    x[132], x[133, ::2], x[134, 1:] = 0.0, -0.0, -0.0
+    b = _bf(x)
+    b[135, 3], b[136, 3], b[137, 3], b[138] = 0x7F80, 0xFF80, 0x7FC1, 0x7FC0
+    q, s = _quant(to_dev(b, dev), fp8=True)
+    fin = np.r_[0:135, 139]
+    eq, es = oq.quantize_rows(b[fin], "fp8_rowwise")
+    assert np.array_equal(to_np(q)[fin], eq) and np.array_equal(to_np(s)[fin], es)
+    q = to_np(q)
+    assert (q[135, 3], q[136, 3], q[137, 3]) == (0xFE, 0xFE, 0xFE) and (q[138] == 0xFE).all()
+    assert np.isinf(to_np(s)[135:137]).all() and (np.delete(q[135], 3) & 0x7F == 0).all()
+
+
 def test_quant_rows_strided(dev):
     import torch
     rng = np.random.default_rng(5)
