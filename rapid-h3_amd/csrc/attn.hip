@@ -18,6 +18,7 @@
 //   K and Vt tiles (8 + 16 KiB per step) go through a 4-slot LDS ring with XOR-swizzled 16-byte chunks.
 //   With one workgroup per CU the grid runs in rounds; a last round at most half full runs as two key
 //   halves per workgroup (fp32 partials), merged by attn_combine_kernel.
+#include <algorithm>
 #include <cstdlib>
 #include <mutex>
 #include <type_traits>
@@ -169,6 +170,9 @@ struct FwdArgs {
   int npair;    // items nmain + i and nmain + npair + i run the two key halves of id nmain + i
   float* tail;  // [2][npair][FWD_BQ][TAIL_ROW] fp32 partials of the split ids
   int* ctr;     // CLAIM_COUNTERS work counters, zero at launch (claim_item)
+  // the 128-query kernel
+  const uint16_t* q;   // raw queries [Sq][H][128] when the kernel quantizes them itself
+  int64_t q_ss, q_sh;
 };
 
 // a wave-uniform float (lane 0's value), held in an SGPR
@@ -190,6 +194,10 @@ __device__ __forceinline__ int vsw(int d) { return ((d & 31) ^ ((d & 31) >> 3)) 
 // no score scan while a bound proves the running max is still good).
 constexpr int FWD_WAVES = 12, FWD_NT = FWD_WAVES * 64, FWD_BQ = FWD_WAVES * 32;
 static_assert(FWD_BQ == attn_ws::FWD_BQ, "workspace layout constants");
+// The same step on a workgroup of 4 waves (128 queries, one scale block; three such workgroups on a CU, each with a
+// 2-slot ring of its own): for calls whose items are short or few (use_small).
+constexpr int SM_WAVES = 4, SM_NT = SM_WAVES * 64, SM_BQ = SM_WAVES * 32, SM_KB = 512;
+static_assert(SM_BQ == attn_ws::SM_BQ, "workspace layout constants");
 constexpr int TAIL_ROW = attn_ws::TAIL_ROW;
 constexpr int MAGIC_I = 0x4B400000;  // bits of 1.5 * 2^23
 constexpr float MAGIC_F = 12582912.0f;
@@ -202,34 +210,91 @@ constexpr float BOUND_LOG2 = 64.0f;
 constexpr int KSLOT = STEP * D;      // K tile: 64 keys x 128 B, chunk c of row r at c ^ ((r ^ (r >> 3)) & 7)
 constexpr int VSLOT = D * STEP * 2;  // V^T tile: 128 d x 64 keys x 2 B, chunk c of row d at c ^ vsw(d)
 constexpr int NRING = 4;             // slots of the K ring and of the V^T ring
+constexpr int SM_NRING = 2;
 
 // Step j reads K(j) and V^T(j) from ring slot u = (j - j0) % 4 and first copies K(j+2), V^T(j+2) into slot
 // (u + 2) % 4, last read in step j-2 (every wave has passed the end-of-step barrier of step j-1). Steps past Sk
 // are not run; the ragged last step is a separate instantiation, so the full steps carry no key mask.
 // SPLIT: bid < npair runs the first half of the steps of id nmain + bid, bid >= npair the second half of id
 // nmain + bid - npair, and each writes its unnormalised O, running max and row sum to the tail partials.
-template <bool SPLIT>
+// SMALL: the 128-query kernel. QF: its queries come raw, one quantization block per workgroup, quantized here as
+// quant_kernel does.
+template <bool SPLIT, bool SMALL = false, bool QF = false>
 __device__ __forceinline__ void fwd_body(const FwdArgs& a, const int bid, int8_t* kring, int8_t* vring,
                                          float2* kscale) {
+  constexpr int NT = SMALL ? SM_NT : FWD_NT, BQ = SMALL ? SM_BQ : FWD_BQ, RING = SMALL ? SM_NRING : NRING;
+  static_assert(!(SMALL && SPLIT), "the 128-query kernel runs whole items");
   const int half = SPLIT ? bid / a.npair : 0;
   const int id = SPLIT ? a.nmain + bid - half * a.npair : bid;
   const int h = id / a.nqb, qb = id - h * a.nqb;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, g = lane >> 5;
-  const int64_t q = static_cast<int64_t>(qb) * FWD_BQ + wave * 32 + l32;
+  const int64_t q = static_cast<int64_t>(qb) * BQ + wave * 32 + l32;
+
+  // SMALL: copy c of a slot (8 rows, positions 64 c + lane) is K's for c < 8 and V^T's otherwise; wave w takes K's 2w,
+  // 2w + 1 and V^T's 4w .. 4w + 3. Row 8c + l/8 is stored with chunk l % 8 XOR (l / 8 ^ c), so the lane offsets of a wave's
+  // copies differ in the XOR with 16 i alone. The first tiles are on their way while the queries are read and quantized.
+  const uint32_t sk0 = static_cast<uint32_t>((lane >> 3) * 128 + (((lane & 7) ^ (((lane >> 3) ^ (2 * wave)) & 7)) << 4));
+  const uint32_t sv0 = static_cast<uint32_t>(static_cast<int>((lane >> 3) * a.Skpad * 2) + (((lane & 7) ^ ((lane >> 3) & 7)) << 4));
+  auto load_small = [&](int j) __attribute__((always_inline)) {
+    const uint32_t u = static_cast<uint32_t>(j) & (SM_NRING - 1);
+    const int64_t jj = min(j, static_cast<int>((a.Sk + STEP - 1) / STEP) - 1);   // clamped: the copy lands unread
+    const int8_t* kb = a.k8 + static_cast<int64_t>(h) * a.Skpad * D + jj * KSLOT + wave * 2048;
+    const int8_t* vb = reinterpret_cast<const int8_t*>(a.vt + static_cast<int64_t>(h) * D * a.Skpad) + jj * (STEP * 2) +
+                       static_cast<int64_t>(wave) * 64 * a.Skpad;
+    const uint32_t kd = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(kring)) + u * KSLOT + wave * 2048;
+    const uint32_t vd = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(vring)) + u * VSLOT + wave * 4096;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) lds_dma16_s(kb + i * 1024, sk0 ^ (16 * i), kd + i * 1024);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lds_dma16_s(vb + static_cast<int64_t>(i) * 16 * a.Skpad, sv0 ^ (16 * i), vd + i * 1024);
+  };
+  if constexpr (SMALL) load_small(0);
 
   // the Q operands are padded to 128 queries; a workgroup's last blocks may lie past them (then they are
   // computed on zero codes and never stored)
   const bool qin = q < a.Sqpad;
   v4i qf[4];
-  {
+  float qscale;
+  if constexpr (QF) {
+    // chunk ds of the lane: channels 32 ds + 16 g .. +15 of its query (zeros past Sq)
+    __shared__ float wmax[SM_WAVES];
+    const uint16_t* qp = a.q + (q < a.Sq ? q : a.Sq - 1) * a.q_ss + static_cast<int64_t>(h) * a.q_sh + g * 16;
+    uint4 raw[8];
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) raw[2 * ds + t] = reinterpret_cast<const uint4*>(qp + ds * 32)[t];
+    uint32_t m2 = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (q >= a.Sq) raw[i] = make_uint4(0, 0, 0, 0);
+      m2 = absmax8_bf16(m2, raw[i]);
+    }
+    const float am = wave_max(amax_of_pair(m2));
+    if (lane == 0) wmax[wave] = am;
+    __syncthreads();
+    const float bm = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    const float sc = fmaxf(bm, 1e-8f) / 127.0f, inv = 1.0f / sc;
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        float v[8];
+        unpack8(raw[2 * ds + t], v);
+        const uint2 c = quant8_i8(v, sc, inv);
+        qf[ds][2 * t] = static_cast<int>(c.x);
+        qf[ds][2 * t + 1] = static_cast<int>(c.y);
+      }
+    qscale = uniform(sc * a.scale_log2);
+  } else {
     const int8_t* qp = a.q8 + (static_cast<int64_t>(h) * a.Sqpad + q) * D + g * 16;
 #pragma unroll
     for (int ds = 0; ds < 4; ++ds) qf[ds] = qin ? *reinterpret_cast<const v4i*>(qp + ds * 32) : v4i{0, 0, 0, 0};
+    // a wave's 32 queries lie in one 128-query scale block, all below Sqpad or all past it: the scale is uniform
+    qscale = uniform((qin ? a.qs[static_cast<int64_t>(h) * (a.Sqpad / BLK) + (q >> 7)] : 0.0f) * a.scale_log2);
   }
-  // a wave's 32 queries lie in one 128-query scale block, all below Sqpad or all past it: the scale is uniform
-  const float qscale = uniform((qin ? a.qs[static_cast<int64_t>(h) * (a.Sqpad / BLK) + (q >> 7)] : 0.0f) * a.scale_log2);
   // |q8 . k8| <= |q8| |k8|: the wave's largest query norm (each lane's 64 codes plus the partner lane's 64),
   // pushed up past the roundings of the bound below, times the query scale
   float qbound;
@@ -245,7 +310,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, const int bid, int8_t
     qbound = uniform(qscale * (sqrtf(static_cast<float>(n2)) * 1.0001f));
   }
   const int nkb = static_cast<int>(a.Skpad / BLK);
-  for (int i = tid; i < nkb; i += FWD_NT) {
+  for (int i = tid; i < nkb; i += NT) {
     const float ksc = a.ks[static_cast<int64_t>(h) * nkb + i];
     kscale[i] = make_float2(ksc, ksc * a.kn[static_cast<int64_t>(h) * nkb + i]);
   }
@@ -419,22 +484,27 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, const int bid, int8_t
   // j+2 right after B_(j-1), into the slot last read in step j-2; before B_j it waits for its copies of step j+1
   // (vmcnt(2) leaves the two issued in step j in flight), so slot j+1 is complete past B_j.
   auto barrier = [&]() __attribute__((always_inline)) {
-    asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+    // SMALL copies one step ahead, into the slot of the step before: its last reads must have returned, too
+    if constexpr (SMALL) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
   auto step = [&](const int j, auto tail) __attribute__((always_inline)) {
-    const uint32_t slot = static_cast<uint32_t>(j - j0) & (NRING - 1);
+    const uint32_t slot = static_cast<uint32_t>(j - j0) & (RING - 1);
     const float2 kk = kscale[j >> 1];
-    load_step(j + 2);
+    if constexpr (SMALL) load_small(j + 1);
+    else load_step(j + 2);
     qk(slot);
     softmax(j, tail, kk);
     pv(slot);
     barrier();
   };
 
-  load_step(j0);
-  load_step(j0 + 1);
+  if constexpr (!SMALL) {
+    load_step(j0);
+    load_step(j0 + 1);
+  }
   // vmcnt(0) through the builtin, so the compiler also sees the Q loads above as complete and adds no
   // wait of its own inside the loop (gfx9 s_waitcnt: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8])
   __builtin_amdgcn_s_waitcnt(0x0f70);
@@ -447,7 +517,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, const int bid, int8_t
   const float lt = lrow + __shfl_xor(lrow, 32, 64);
   if constexpr (SPLIT) {
     if (q < a.Sq) {
-      float* tp = a.tail + ((static_cast<int64_t>(half) * a.npair + (id - a.nmain)) * FWD_BQ + wave * 32 + l32) * TAIL_ROW;
+      float* tp = a.tail + ((static_cast<int64_t>(half) * a.npair + (id - a.nmain)) * BQ + wave * 32 + l32) * TAIL_ROW;
 #pragma unroll
       for (int db = 0; db < 4; ++db)
 #pragma unroll
@@ -459,6 +529,34 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, const int bid, int8_t
     return;
   }
   const float il = 1.0f / lt;
+  if constexpr (SMALL) {
+    // The wave's 32 rows go through its 8 KiB of the idle ring (row r at 256 r, 16-byte chunk c at c ^ (r & 15)), so that a
+    // store instruction writes four whole rows; straight from the accumulators it writes 8 bytes to each of 32 rows. Every
+    // wave is past the last step's barrier with no copy in flight; a wave's LDS accesses execute in order.
+    const uint32_t st = kring_lds + wave * 8192;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq) {
+        const int c = db * 4 + rq;   // channels 8c + 4g .. +3
+        lds_write8(st + l32 * 256 + ((c ^ (l32 & 15)) << 4) + 8 * g,
+                   make_uint2(pk_bf16(o[db][4 * rq + 0] * il, o[db][4 * rq + 1] * il),
+                              pk_bf16(o[db][4 * rq + 2] * il, o[db][4 * rq + 3] * il)));
+      }
+    asm volatile("" ::: "memory");
+    const int64_t q0 = static_cast<int64_t>(qb) * BQ + wave * 32;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = 4 * i + (lane >> 4), c = lane & 15;
+      const v4i w = lds_read16(st + r * 256 + ((c ^ (r & 15)) << 4));
+      if (q0 + r < a.Sq) {   // two 8-byte stores, the alignment the entry points require of out
+        uint2* op = reinterpret_cast<uint2*>(a.out + (q0 + r) * a.o_ss + static_cast<int64_t>(h) * a.o_sh + 8 * c);
+        op[0] = make_uint2(static_cast<uint32_t>(w[0]), static_cast<uint32_t>(w[1]));
+        op[1] = make_uint2(static_cast<uint32_t>(w[2]), static_cast<uint32_t>(w[3]));
+      }
+    }
+    return;
+  }
   if (q < a.Sq) {
     uint16_t* op = a.out + q * a.o_ss + static_cast<int64_t>(h) * a.o_sh;
 #pragma unroll
@@ -493,6 +591,16 @@ __global__ void __launch_bounds__(FWD_NT, 1) attn_fwd_kernel(const FwdArgs a) {
     fwd_body<false>(a, item, ring, ring + NRING * KSLOT, kscale);
   else
     fwd_body<true>(a, item - a.nmain, ring, ring + NRING * KSLOT, kscale);
+}
+
+// The 128-query kernel: workgroup b of n takes item b % 8 * n / 8 + b / 8, so that the workgroups of one XCD read few heads.
+template <bool QF>
+__global__ void __launch_bounds__(SM_NT, 3) attn_fwd_small_kernel(const FwdArgs a) {
+  __shared__ __attribute__((aligned(16))) int8_t ring[SM_NRING * (KSLOT + VSLOT)];
+  __shared__ float2 kscale[SM_KB];
+  const int n = gridDim.x, b = blockIdx.x, x = b % 8;
+  const int item = x * (n / 8) + min(x, n % 8) + b / 8;
+  fwd_body<false, true, QF>(a, item, ring, ring + SM_NRING * KSLOT, kscale);
 }
 
 // Merge of the two key halves of a split workgroup: m = max(m0, m1), O = (O0 2^(m0-m) + O1 2^(m1-m)) / l with
@@ -565,8 +673,9 @@ int prepass(const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* k, in
     // a fill kernel, not hipMemsetAsync, so the call stays safe inside a captured HIP graph
     hipLaunchKernelGGL(zero_kernel, dim3((H * D + 255) / 256), dim3(256), 0, st, w.kmean, H * D);
   }
-  launch_quant(dim3(H, sqp / BLK), st, q, q_ss, q_sh, Sq, sqp, rq, static_cast<const float*>(nullptr), w.q8, w.qs,
-               nullptr);
+  if (!w.rawq)  // else the main kernel quantizes the queries itself
+    launch_quant(dim3(H, sqp / BLK), st, q, q_ss, q_sh, Sq, sqp, rq, static_cast<const float*>(nullptr), w.q8, w.qs,
+                 nullptr);
   if (staged)
     launch_quant(dim3(H, skp / BLK), st, w.vt, D, skp * D, Sk, skp, RR{nullptr, nullptr, 0.f, 0}, mean, w.k8, w.ks,
                  w.kn);
@@ -576,8 +685,49 @@ int prepass(const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* k, in
   return launch_status("attention prepass");
 }
 
+// Whether a call runs on the 128-query kernel. Both forms are modelled in us from their measured rounds: n steps of 64 keys
+// take 12 + 2.0 n in a full round of the 384-query kernel (10 + 1.75 n when some CUs have no item, half of a round when a last
+// one is split in keys) and 8 + 2.15 n in a full round of three 128-query workgroups per CU, 6 + 0.95 n or 6 + 1.42 n when
+// the fullest CU holds only one or two. The small form wins where items are short (its prologues and epilogues overlap
+// another workgroup's steps) or where its finer items fill the last round better; long items cost it 5 % (every wave
+// reads K and V^T from LDS for 32 queries either way, but each is copied there three times as often). Measured main
+// kernel (us, 384 / 128 queries): 1,024 tokens x 24 heads 39 / 20, 1,560 x 24 54 / 39, 2,816 x 24 86 / 92, 4,096 x 24
+// 186 / 148, 5,583 x 24 290 / 301, 1,560 x 56 92 / 61, 72,216 queries x 512 keys x 24 heads 502 / 402 (qf: it also quantizes
+// the queries itself, which the pre-pass takes 180 us for there), 11,000 x 24 986 / 1,052.
+bool use_small(int64_t Sq, int64_t Sk, int64_t H, bool qf) {
+  const int64_t cus = device_cus();
+  if (cus <= 0 || pad(Sk) / BLK > SM_KB) return false;
+  const double n = static_cast<double>((Sk + STEP - 1) / STEP);
+  const int64_t big = (Sq + FWD_BQ - 1) / FWD_BQ * H, small = (Sq + SM_BQ - 1) / SM_BQ * H;
+  if (small >= (int64_t{1} << 31)) return false;
+  const int64_t bf = big / cus, br = big % cus, sf = small / (3 * cus), sr = (small % (3 * cus) + cus - 1) / cus;
+  double tb = static_cast<double>(bf) * (12 + 2.0 * n);
+  if (br > 0) tb += bf == 0 ? 10 + 1.75 * n : 2 * br <= cus && n >= 8 ? 10 + n : 12 + 2.0 * n;
+  if (qf) tb += 6 + static_cast<double>(Sq * H) * (180.0 / (72216.0 * 24.0));   // the pre-pass over the queries
+  const double part[4] = {0, 6 + 0.95 * n, 6 + 1.42 * n, 6 + 2.05 * n};
+  const double ts = static_cast<double>(sf) * (8 + 2.15 * n) + part[sr];
+  return ts < tb;
+}
+
+// one-call attention without RMSNorm + RoPE: hand the raw queries to the 128-query kernel where it runs
+void raw_queries(Work& w, const uint16_t* q, int64_t q_ss, int64_t q_sh, int64_t Sq, int64_t Sk, int64_t H) {
+  if (!use_small(Sq, Sk, H, true)) return;
+  w.rawq = q;
+  w.rq_ss = q_ss;
+  w.rq_sh = q_sh;
+}
+
 int forward(const Work& w, int64_t Sq, int64_t Sk, int64_t H, float scale, uint16_t* out, int64_t o_ss,
             int64_t o_sh, hipStream_t st) {
+  if (use_small(Sq, Sk, H, w.rawq != nullptr)) {
+    const int nqb = static_cast<int>((Sq + SM_BQ - 1) / SM_BQ);
+    const FwdArgs f{w.q8, w.qs, w.k8, w.ks, w.kn, w.vt, out, o_ss, o_sh, Sq, Sk, pad(Sq), pad(Sk),
+                    scale * 1.4426950408889634f, nqb, 0, 0, nullptr, nullptr, w.rawq, w.rq_ss, w.rq_sh};
+    const dim3 g(static_cast<unsigned>(H * nqb));
+    if (w.rawq) hipLaunchKernelGGL(attn_fwd_small_kernel<true>, g, dim3(SM_NT), 0, st, f);
+    else hipLaunchKernelGGL(attn_fwd_small_kernel<false>, g, dim3(SM_NT), 0, st, f);
+    return launch_status("attention forward");
+  }
   const int64_t nwg = attn_ws::fwd_blocks(Sq, H);
   RH3_REQUIRE(nwg < (int64_t{1} << 30) / FWD_NT, "attention forward: %lld workgroups exceed the grid limit",
               (long long)nwg);
@@ -706,8 +856,9 @@ extern "C" int rh3_int8_attention_noalloc(const uint16_t* q, int64_t q_ss, int64
               (long long)need, (long long)NOALLOC_SCRATCH_BYTES);
   void* base = nullptr;
   if (int e = scratch_of(stream, &base)) return e;
-  const Work w = layout(base, Sq, Sk, H, false);
+  Work w = layout(base, Sq, Sk, H, false);
   const RR none{nullptr, nullptr, 0.f, 0};
+  raw_queries(w, q, q_ss, q_sh, Sq, Sk, H);
   if (int e = prepass(q, q_ss, q_sh, k, k_ss, k_sh, v, v_ss, v_sh, Sq, Sk, H, none, none, smooth_k, w, stream))
     return e;
   return forward(w, Sq, Sk, H, scale, out, o_ss, o_sh, stream);
@@ -803,10 +954,11 @@ extern "C" int rh3_int8_attention(const uint16_t* q, int64_t q_ss, int64_t q_sh,
   if (int e = check_qkv("int8_attention", q, q_ss, q_sh, k, k_ss, k_sh, v, v_ss, v_sh, Sq, Sk, H)) return e;
   RH3_REQUIRE(out && (reinterpret_cast<uintptr_t>(out) & 7) == 0 && o_ss % 4 == 0 && o_sh % 4 == 0,
               "int8_attention: out must be 8-byte aligned with strides multiple of 4");
-  const Work w = layout(workspace, Sq, Sk, H);
+  Work w = layout(workspace, Sq, Sk, H);
   RH3_REQUIRE(workspace && aligned16(workspace) && workspace_bytes >= w.bytes,
               "int8_attention: workspace %lld bytes < required %lld", (long long)workspace_bytes, (long long)w.bytes);
   const RR none{nullptr, nullptr, 0.f, 0};
+  raw_queries(w, q, q_ss, q_sh, Sq, Sk, H);
   if (int e = prepass(q, q_ss, q_sh, k, k_ss, k_sh, v, v_ss, v_sh, Sq, Sk, H, none, none, smooth_k, w, stream))
     return e;
   return forward(w, Sq, Sk, H, scale, out, o_ss, o_sh, stream);

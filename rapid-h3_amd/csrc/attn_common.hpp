@@ -145,6 +145,11 @@ __device__ __forceinline__ v4i lds_read16(uint32_t addr) {
   return *reinterpret_cast<lds_v4i*>(static_cast<uintptr_t>(addr));
 }
 
+__device__ __forceinline__ void lds_write8(uint32_t addr, uint2 v) {
+  typedef __attribute__((address_space(3))) u32x2_t lds_u2;
+  *reinterpret_cast<lds_u2*>(static_cast<uintptr_t>(addr)) = u32x2_t{v.x, v.y};
+}
+
 // max of lane l and lane l ^ 32 (v_permlane32_swap exchanges the wave's halves)
 __device__ __forceinline__ int max_halves(int v) {
   const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);

@@ -19,6 +19,7 @@ __host__ __device__ inline int64_t nchunks(int64_t s) { return (s + CHUNK - 1) /
 
 // per-128-block recipe (bf16 P.V)
 constexpr int FWD_BQ = 384;     // queries per main-kernel workgroup
+constexpr int SM_BQ = 128;      // queries per workgroup of the 128-query kernel
 constexpr int TAIL_MAX = 128;   // most (head, query block) workgroups whose keys the main kernel splits in two
 constexpr int TAIL_ROW = D + 4; // floats per query of a split partial: O[128], running max, row sum, 2 unused
 
@@ -31,6 +32,9 @@ struct Work {
   float* tail;  // [2][npair][FWD_BQ][TAIL_ROW] partials of the split last round; null when not reserved
   int* ctr;     // the main kernel's work counter (cleared before each launch)
   int64_t bytes;
+  // not part of the layout: the raw queries, when the main kernel quantizes them itself (the Q region then stays unused)
+  const uint16_t* rawq = nullptr;
+  int64_t rq_ss = 0, rq_sh = 0;
 };
 
 // split false: no room for the split-last-round partials (the main kernel then runs every workgroup whole)

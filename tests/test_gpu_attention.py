@@ -114,6 +114,38 @@ def test_attention_ragged(dev, sq, sk, h):
     assert rel_l2(out, ref) < GUARD
 
 
+@pytest.mark.parametrize("sq,sk,h", [(1, 64, 2), (127, 63, 3), (128, 65, 2), (385, 128, 2), (300, 1000, 3), (9000, 129, 24)])
+def test_attention_128_query_kernel(dev, sq, sk, h):
+    """The 128-query kernel, which quantizes the queries of a one-call attention itself: at the edges of its query
+    blocks and key steps, and over many rounds of workgroups per CU, the one call and the split pair (whose pre-pass
+    quantizes them) agree bit for bit; sampled rows against the oracle."""
+    import torch
+    from rapid_h3 import attention
+    rng = np.random.default_rng(sq + 3 * sk + h)
+    q, k, v = (_bf(rng.standard_normal((n, h, 128)) + off) for n, off in
+               ((sq, 0.0), (sk, 2.0 * rng.standard_normal((1, h, 128))), (sk, 0.0)))
+    qt, kt, vt = (to_dev(t, dev) for t in (q, k, v))
+    pad = torch.full((sq + 1, h + 1, 136), 7.0, dtype=torch.bfloat16, device=dev)
+    out = attention.attention(qt, kt, vt, out=pad[:sq, :h, 4:132])      # 8-byte aligned rows
+    assert torch.equal(out, attention.forward(attention.prepass(qt, kt, vt), sq))
+    assert (pad[sq] == 7).all() and (pad[:, h] == 7).all() and (pad[:, :, :4] == 7).all() and (pad[:, :, 132:] == 7).all()
+    rows = np.arange(sq) if sq < 1000 else np.sort(rng.choice(sq, 200, replace=False))
+    q8, qs, k8, ks, _ = oa.prepass(q, k)
+    ref = oa.attention_from_codes(q8, qs, k8, ks, v, 128 ** -0.5, rows=rows)
+    assert rel_l2(bf16_to_f32(to_np(out[torch.from_numpy(rows).to(dev)])), ref[:len(rows)]) < GUARD
+
+
+def test_attention_query_kernels_agree(dev):
+    """2,816 queries of 24 heads fill the chip with 384-query workgroups; the first 1,024 of them alone run on the
+    128-query kernel: the same rows, bit for bit (on 256 CUs; elsewhere both may run on one kernel)."""
+    import torch
+    from rapid_h3 import attention
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn(2816, 24, 128, generator=g).to(torch.bfloat16).to(dev) for _ in range(3))
+    whole = attention.attention(q, k, v)
+    assert torch.equal(attention.attention(q[:1024], k, v), whole[:1024])
+
+
 def test_attention_strided_out(dev):
     """q/k/v as views of one [S, 3*H*128] qkv buffer; output into a head-major [1, H, S, D] buffer
     through out=o[0].transpose(0, 1) (the _fused_block call, __init__.py:283-291)."""
