@@ -14,7 +14,7 @@
 //   vq_kernel      per (128-key tile, head): int8 V codes rint((v - vmean) / vscale) (attn_int8.cu:452-475),
 //                  transposed to [H][128][Skpad] in the key order of the P.V operand, and the tile's P.V
 //                  accumulator start 1.5*2^23 bits + 128 * (sum of its codes) per channel
-// Main kernel: per (256-query block, head) workgroup of 8 waves, 32 queries per wave, 128-key tiles.
+// Main kernel: per (128-query block, head) workgroup of 4 waves, 32 queries per wave, 128-key tiles.
 //   S^T = K8 . Q8^T on v_mfma_i32_32x32x32_i8 (keys on rows, queries on lanes), the accumulator starting at
 //   the bits of 1.5*2^23 so that t = fma(float bits, s_j, b_j) is the dequantized score in one instruction;
 //   tile max tm, n = max(m, tm), a = 2^((m - n) c), ts = 2^((tm - n) c); P = rint(2^(fma(t, c, log2 255 - tm c)))
@@ -362,7 +362,12 @@ struct U8Args {
   int* ctr;  // work counter, zero at launch: a starting workgroup takes item ctr++
 };
 
-constexpr int U8_WAVES = 8, U8_NT = U8_WAVES * 64, U8_BQ = U8_WAVES * 32;
+// 4 waves (one per SIMD) of 32 queries, two workgroups on a CU: VALU and matrix work of a wave do not overlap, so what fills
+// the matrix pipe during one workgroup's softmax is the other workgroup, which no barrier ties to it. (One workgroup of
+// 8 waves, half of them held half a tile behind by its barriers, ran 384.8 us against 334.1 for 5,583 tokens x 24 heads,
+// 4.49 against 4.27 ms for 22,332 and 43.9 against 43.1 ms for 72,216, same bits; its 256-query items also filled the last
+// round worse.)
+constexpr int U8_WAVES = 4, U8_NT = U8_WAVES * 64, U8_BQ = U8_WAVES * 32;
 
 typedef __attribute__((address_space(3))) const v4i lds_v4i_u8;
 typedef __attribute__((address_space(3))) const float lds_f32_u8;
@@ -374,8 +379,8 @@ __device__ __forceinline__ float max3f(float a, float b, float c) {
   return r;
 }
 
-// Tile j reads K(j), V^T(j) and its side record from ring slot j % 4 and first loads tile j + 2 into slot
-// (j + 2) % 4, whose last reader ran before the barrier that ended tile j - 1 (see the barrier comment).
+// Tile j reads K(j), V^T(j) and its side record from ring slot j % 2 and first loads tile j + 1 into the other slot, whose
+// last reads returned before the barrier that ended tile j - 1.
 // A slot holds K: 128 keys x 128 B (chunk c of row r at c ^ ((r ^ (r >> 3)) & 7)), V^T: 128 channels x 128
 // keys (the same swizzle), then the 2 KiB side record. Padded keys carry b = -inf, so every tile runs unmasked.
 // BK (configs 60-61, attn_fwd6 :1786-1962): one K scale kb per 128-key tile (the first float of the side record)
@@ -388,10 +393,10 @@ __device__ __forceinline__ float max3f(float a, float b, float c) {
 // round to nearest even), l += P unquantized, and O^T += V^T . P^T on v_mfma_scale_f32_32x32x64_f8f6f4 (e4m3 V
 // from vq_kernel<true>) straight into the fp32 accumulators: no per-tile fold.
 template <int MODE, int MAXG = 128>
-__global__ void __launch_bounds__(U8_NT, 1) attn_u8_kernel(const U8Args a) {
+__global__ void __launch_bounds__(U8_NT, 2) attn_u8_kernel(const U8Args a) {
   constexpr bool BK = MODE == 1;
   constexpr int KB = TILE * D, VB = D * TILE, SLOT = KB + VB + SIDE;
-  __shared__ __attribute__((aligned(16))) int8_t ring[4 * SLOT];
+  __shared__ __attribute__((aligned(16))) int8_t ring[2 * SLOT];
   // the workgroup runs the item it takes from one work counter when it starts (a fast XCD takes more; see the
   // launch), the (head, query block) pair h * nqb + qb. Per-XCD shares (claim_item) measured 1.6 % slower here
   // (180.3 vs 177.4 ms at C4), so this kernel keeps the single counter.
@@ -419,30 +424,27 @@ __global__ void __launch_bounds__(U8_NT, 1) attn_u8_kernel(const U8Args a) {
   const float c = (qin ? a.qs[static_cast<int64_t>(h) * a.Sqpad + q] : 0.0f) * a.scale_log2;
   const float ib = (a.nbias > 0 && c > 0.0f) ? a.bias_log2 / c : 0.0f;
 
-  // global -> LDS copies (lane l of a wave writes LDS base + 16 l; the swizzle is applied on the global side):
-  // K and V^T positions p = 64 w + lane and 512 + 64 w + lane (rows p / 8 and p / 8 + 64, same swizzle) for
-  // every wave, the 128 side chunks by waves 0 and 1. Waves 0-1 issue 5 copies per tile, waves 2-7 issue 4.
+  // global -> LDS copies (lane l of a wave writes LDS base + 16 l; the swizzle is applied on the global side): copy c of K
+  // and of V^T fills rows 8 c .. 8 c + 7 of the slot, row 8 c + l / 8 stored with chunk l % 8 XOR (l / 8 ^ c) & 7; wave w takes
+  // copies 4 w .. 4 w + 3 of each, whose lane offsets differ in the XOR with 16 i alone, and waves 0 and 1 a side half
   const int8_t* kbase = a.k8 + static_cast<int64_t>(h) * a.Skpad * D;
   const int8_t* vbase = a.vt + static_cast<int64_t>(h) * D * a.Skpad;
   const int8_t* sbase = a.side + static_cast<int64_t>(h) * ntiles * SIDE;
-  const int p0 = wave * 64 + lane, row0 = p0 >> 3, pc0 = p0 & 7, sw0 = (pc0 ^ ((row0 ^ (row0 >> 3)) & 7)) << 4;
-  const int8_t* ksrc = kbase + row0 * D + sw0;
-  const int8_t* vsrc = vbase + static_cast<int64_t>(row0) * a.Skpad + sw0;
-  const int8_t* ssrc = sbase + p0 * 16;  // waves 0, 1 only
-  const int64_t vhalf = 64 * a.Skpad;
+  const uint32_t sx = ((lane & 7) ^ (((lane >> 3) ^ (4 * wave)) & 7)) << 4;
+  const uint32_t ko = (lane >> 3) * D + sx, vo = static_cast<uint32_t>((lane >> 3) * a.Skpad) + sx;
   const uint32_t ring_lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(ring));
-  const uint32_t kdst = ring_lds + wave * 1024, vdst = kdst + KB, sdst = ring_lds + KB + VB + wave * 1024;
-  const bool side_wave = wave < 2;
   auto load_tile = [&](int j) __attribute__((always_inline)) {
-    const uint32_t so = static_cast<uint32_t>(j & 3) * SLOT;
-    j = min(j, ntiles - 1);  // clamped: every tile issues the same copies; a copy past the end lands unread
-    const int8_t* kp = ksrc + static_cast<int64_t>(j) * KB;
-    const int8_t* vp = vsrc + static_cast<int64_t>(j) * TILE;
-    lds_dma16(kp, kdst + so);
-    lds_dma16(kp + 64 * D, kdst + so + 8192);
-    lds_dma16(vp, vdst + so);
-    lds_dma16(vp + vhalf, vdst + so + 8192);
-    if (side_wave) lds_dma16(ssrc + static_cast<int64_t>(j) * SIDE, sdst + so);
+    const uint32_t so = static_cast<uint32_t>(j & 1) * SLOT;
+    j = min(j, ntiles - 1);  // clamped: a copy past the end lands unread
+    const int8_t* kp = kbase + static_cast<int64_t>(j) * KB + wave * 4096;
+    const int8_t* vp = vbase + static_cast<int64_t>(j) * TILE + static_cast<int64_t>(wave) * 32 * a.Skpad;
+    const uint32_t kd = ring_lds + so + wave * 4096;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lds_dma16_s(kp + i * 1024, ko ^ (16 * i), kd + i * 1024);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lds_dma16_s(vp + static_cast<int64_t>(i) * 8 * a.Skpad, vo ^ (16 * i), kd + KB + i * 1024);
+    if (wave < 2)
+      lds_dma16_s(sbase + static_cast<int64_t>(j) * SIDE + wave * 1024, lane * 16, ring_lds + so + KB + VB + wave * 1024);
   };
 
   // lane parts of the LDS reads inside a slot. K fragment (kb, ds): row 32 kb + l32, chunk 2 ds + g, stored at
@@ -482,7 +484,7 @@ __global__ void __launch_bounds__(U8_NT, 1) attn_u8_kernel(const U8Args a) {
   // S^T of tile j: lane (l32, g) of s[kb] holds query l32 and keys 32 kb + 8 (r / 4) + 4 g + r % 4
   v16i s[4];
   auto qk = [&](const int j) __attribute__((always_inline)) {
-    const uint32_t so = static_cast<uint32_t>(j & 3) * SLOT;
+    const uint32_t so = static_cast<uint32_t>(j & 1) * SLOT;
     uint32_t ka[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) ka[i] = koff[i] + so;
@@ -498,7 +500,7 @@ __global__ void __launch_bounds__(U8_NT, 1) attn_u8_kernel(const U8Args a) {
   };
 
   auto softmax_pv = [&](const int j) __attribute__((always_inline)) {
-    const uint32_t so = static_cast<uint32_t>(j & 3) * SLOT;
+    const uint32_t so = static_cast<uint32_t>(j & 1) * SLOT;
     // exponent of P: 2^(fma(t, cx, bb)); u8: t the dequantized score, cx = c; BK: t the accumulator bits, cx = c kb
     float t[4][16];
     float cx, bb, al, ts;
@@ -624,7 +626,7 @@ __global__ void __launch_bounds__(U8_NT, 1) attn_u8_kernel(const U8Args a) {
   };
 
   auto softmax_pv_f8 = [&](const int j) __attribute__((always_inline)) {
-    const uint32_t so = static_cast<uint32_t>(j & 3) * SLOT;
+    const uint32_t so = static_cast<uint32_t>(j & 1) * SLOT;
     float t[4][16];
     // t of blocks kb0 .. kb1 - 1 (MAXG 64: per 64-key chunk, so that only one chunk's scores are live at a time)
     auto dequant = [&](const int kb0, const int kb1) __attribute__((always_inline)) {
@@ -700,60 +702,55 @@ __global__ void __launch_bounds__(U8_NT, 1) attn_u8_kernel(const U8Args a) {
     }
   };
 
-  // Barrier B_j ends the use of ring slot j. Leading waves reach B_j after softmax_pv(j), lagging waves after
-  // qk(j), so between B_(j-1) and B_j a lagging wave runs softmax_pv(j-1) while a leading wave runs qk(j). Each
-  // wave issues its copies of tile j+2 right after B_(j-1), into slot (j+2) % 4, whose last reader
-  // (softmax_pv(j-2) of a lagging wave) ran before B_(j-1); before B_j it waits for its copies of tile j+1
-  // (vmcnt(n) leaves the n issued after B_(j-1) in flight), so slot j+1 is complete past B_j.
-  const bool lag = (wave >> 2) == 1;  // waves 4-7 (one per SIMD) run half a tile behind
-  auto barrier = [&]() __attribute__((always_inline)) {
-    if (side_wave) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-  };
-
   load_tile(0);
-  load_tile(1);
   // vmcnt(0) through the builtin, so the compiler also sees the Q loads above as complete and adds no wait of
   // its own inside the loop (gfx9 s_waitcnt: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8])
   __builtin_amdgcn_s_waitcnt(0x0f70);
   __syncthreads();
-  if (lag) load_tile(2);
   for (int j = 0; j < ntiles; ++j) {
-    if (!lag) load_tile(j + 2);
+    load_tile(j + 1);
     qk(j);
-    if (lag) {
-      barrier();
-      load_tile(j + 3);
-    }
     if constexpr (MODE == 2) softmax_pv_f8(j);
     else softmax_pv(j);
-    if (!lag) barrier();
+    // the copies of tile j + 1 have landed and every read of tile j has returned, for every wave past the barrier
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no global->LDS copy outlives the workgroup
 
   const float lt = lrow + __shfl_xor(lrow, 32, 64);
   const float il = 1.0f / lt;
-  if (q < a.Sq) {
-    uint16_t* op = a.out + q * a.o_ss + static_cast<int64_t>(h) * a.o_sh;
-    const float* vs = a.vscale + h * D;
-    const float* vm = a.vmean + h * D;
+  // The wave's 32 rows go through 8 KiB of the idle ring (row r at 256 r, 16-byte chunk c at c ^ (r & 15)), so that a store
+  // instruction writes four whole rows; straight from the accumulators it writes 8 bytes to each of 32. Every wave is past
+  // the last tile's barrier with no copy in flight; a wave's LDS accesses execute in order.
+  const float* vs = a.vscale + h * D;
+  const float* vm = a.vmean + h * D;
+  const uint32_t st = ring_lds + wave * 8192;
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+  for (int db = 0; db < 4; ++db)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int d = db * 32 + 8 * i + 4 * g;
-        float4 s4 = *reinterpret_cast<const float4*>(vs + d);
-        if constexpr (MODE == 2) {  // the e4m3 V codes were stretched by 448 / 127 (attn_int8.cu:2642)
-          s4.x = s4.x * V_UNSTRETCH; s4.y = s4.y * V_UNSTRETCH; s4.z = s4.z * V_UNSTRETCH; s4.w = s4.w * V_UNSTRETCH;
-        }
-        const float4 m4 = *reinterpret_cast<const float4*>(vm + d);
-        uint2 w;
-        w.x = pack_bf2(fmaf(o[db][4 * i + 0] * il, s4.x, m4.x), fmaf(o[db][4 * i + 1] * il, s4.y, m4.y));
-        w.y = pack_bf2(fmaf(o[db][4 * i + 2] * il, s4.z, m4.z), fmaf(o[db][4 * i + 3] * il, s4.w, m4.w));
-        *reinterpret_cast<uint2*>(op + d) = w;
+    for (int i = 0; i < 4; ++i) {
+      const int d = db * 32 + 8 * i + 4 * g, cc = db * 4 + i;
+      float4 s4 = *reinterpret_cast<const float4*>(vs + d);
+      if constexpr (MODE == 2) {  // the e4m3 V codes were stretched by 448 / 127 (attn_int8.cu:2642)
+        s4.x = s4.x * V_UNSTRETCH; s4.y = s4.y * V_UNSTRETCH; s4.z = s4.z * V_UNSTRETCH; s4.w = s4.w * V_UNSTRETCH;
       }
+      const float4 m4 = *reinterpret_cast<const float4*>(vm + d);
+      lds_write8(st + l32 * 256 + ((cc ^ (l32 & 15)) << 4) + 8 * g,
+                 make_uint2(pack_bf2(fmaf(o[db][4 * i + 0] * il, s4.x, m4.x), fmaf(o[db][4 * i + 1] * il, s4.y, m4.y)),
+                            pack_bf2(fmaf(o[db][4 * i + 2] * il, s4.z, m4.z), fmaf(o[db][4 * i + 3] * il, s4.w, m4.w))));
+    }
+  asm volatile("" ::: "memory");
+  const int64_t q0 = static_cast<int64_t>(qb) * U8_BQ + wave * 32;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int r = 4 * i + (lane >> 4), cc = lane & 15;
+    const v4i w = lds_read16(st + r * 256 + ((cc ^ (r & 15)) << 4));
+    if (q0 + r < a.Sq) {   // two 8-byte stores, the alignment the entry points require of out
+      uint2* op = reinterpret_cast<uint2*>(a.out + (q0 + r) * a.o_ss + static_cast<int64_t>(h) * a.o_sh + 8 * cc);
+      op[0] = make_uint2(static_cast<uint32_t>(w[0]), static_cast<uint32_t>(w[1]));
+      op[1] = make_uint2(static_cast<uint32_t>(w[2]), static_cast<uint32_t>(w[3]));
+    }
   }
 }
 
