@@ -38,18 +38,17 @@ constexpr int BLK = 128;     // quantization block and attention tile (tokens)
 // rows in L2), 256 threads: wave w handles tokens w*32 .. w*32+31 of the block, 4 per pass
 // knorm (K only, may be null): per block, an upper bound of the largest L2 norm of a token's 128 int8 codes,
 // which lets the main kernel bound every logit of the block without scanning its scores
-__global__ void __launch_bounds__(256) quant_kernel(const uint16_t* __restrict__ x, int64_t x_ss, int64_t x_sh,
-                                                    int64_t S, int64_t Spad, RR rr, const float* __restrict__ mean,
-                                                    int8_t* __restrict__ codes, float* __restrict__ scales,
-                                                    float* __restrict__ knorm) {
-  __shared__ float wmax[4];
-  __shared__ int wnorm[4];
-  const int h = blockIdx.x, blk = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// mean: the head's row (global memory or LDS), or null
+__device__ __forceinline__ void quant_block(const uint16_t* __restrict__ x, int64_t x_ss, int64_t x_sh, int64_t S,
+                                            int64_t Spad, const RR& rr, const float* mean, int8_t* __restrict__ codes,
+                                            float* __restrict__ scales, float* __restrict__ knorm, int h, int blk,
+                                            float* wmax, int* wnorm) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, sub = lane >> 4;
   float mv[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   if (mean) {
-    const float4 a = *reinterpret_cast<const float4*>(mean + h * D + 8 * l16);
-    const float4 b = *reinterpret_cast<const float4*>(mean + h * D + 8 * l16 + 4);
+    const float4 a = *reinterpret_cast<const float4*>(mean + 8 * l16);
+    const float4 b = *reinterpret_cast<const float4*>(mean + 8 * l16 + 4);
     mv[0] = a.x; mv[1] = a.y; mv[2] = a.z; mv[3] = a.w; mv[4] = b.x; mv[5] = b.y; mv[6] = b.z; mv[7] = b.w;
   }
   float w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -108,6 +107,16 @@ __global__ void __launch_bounds__(256) quant_kernel(const uint16_t* __restrict__
   }
 }
 
+__global__ void __launch_bounds__(256) quant_kernel(const uint16_t* __restrict__ x, int64_t x_ss, int64_t x_sh,
+                                                    int64_t S, int64_t Spad, RR rr, const float* __restrict__ mean,
+                                                    int8_t* __restrict__ codes, float* __restrict__ scales,
+                                                    float* __restrict__ knorm) {
+  __shared__ float wmax[4];
+  __shared__ int wnorm[4];
+  quant_block(x, x_ss, x_sh, S, Spad, rr, mean ? mean + blockIdx.x * D : nullptr, codes, scales, knorm, blockIdx.x,
+              blockIdx.y, wmax, wnorm);
+}
+
 void launch_quant(dim3 grid, hipStream_t st, const uint16_t* x, int64_t x_ss, int64_t x_sh, int64_t S, int64_t Spad,
                   const RR& rr, const float* mean, int8_t* codes, float* scales, float* knorm) {
   hipLaunchKernelGGL(quant_kernel, grid, dim3(256), 0, st, x, x_ss, x_sh, S, Spad, rr, mean, codes, scales, knorm);
@@ -122,12 +131,13 @@ __device__ __forceinline__ int perm32(int p) {
 }
 
 // grid (H, Skpad/64) (heads fastest, so a block's token rows are read together), 256 threads
-__global__ void __launch_bounds__(256) vt_kernel(const uint16_t* __restrict__ v, int64_t v_ss, int64_t v_sh,
-                                                 int64_t S, int64_t Spad, uint16_t* __restrict__ vt) {
+constexpr int VT_LDS = 64 * (D + 8) * 2;
+__device__ __forceinline__ void vt_slab(const uint16_t* __restrict__ v, int64_t v_ss, int64_t v_sh, int64_t S, int64_t Spad,
+                                        uint16_t* __restrict__ vt, int h, int blk, uint16_t* tile) {
   constexpr int T = 64, P = D + 8;
-  __shared__ uint16_t tile[T * P];
-  const int h = blockIdx.x, tid = threadIdx.x;
-  const int64_t s0 = static_cast<int64_t>(blockIdx.y) * T;
+  static_assert(VT_LDS == T * P * 2, "tile");
+  const int tid = threadIdx.x;
+  const int64_t s0 = static_cast<int64_t>(blk) * T;
   for (int i = tid; i < T * D / 8; i += 256) {
     const int r = i / (D / 8), c8 = (i % (D / 8)) * 8;
     uint4 val = make_uint4(0, 0, 0, 0);
@@ -151,6 +161,68 @@ __global__ void __launch_bounds__(256) vt_kernel(const uint16_t* __restrict__ v,
     pk.w = o[6] | (static_cast<uint32_t>(o[7]) << 16);
     *reinterpret_cast<uint4*>(vt + (static_cast<int64_t>(h) * D + d) * Spad + s0 + pc) = pk;
   }
+}
+
+__global__ void __launch_bounds__(256) vt_kernel(const uint16_t* __restrict__ v, int64_t v_ss, int64_t v_sh,
+                                                 int64_t S, int64_t Spad, uint16_t* __restrict__ vt) {
+  __shared__ __attribute__((aligned(16))) uint16_t tile[VT_LDS / 2];
+  vt_slab(v, v_ss, v_sh, S, Spad, vt, blockIdx.x, blockIdx.y, tile);
+}
+
+// ------------------------------------------------------------------ the pre-pass of a short call in two launches
+// A: K statistics, the Q quantizer and the V relayout, which do not depend on each other; B: the K quantizer, each workgroup
+// folding its head's kmean itself (float64 sums of bf16 values: exact in any order). At 1,560 tokens x 24 heads the five
+// launches they replace (or six) took 45 us, more of it launch gaps and half-empty grids than work; now 31. From 16
+// statistics chunks on the fold would cost more than a launch, and K's staged rows (prepass) save its second prologue.
+constexpr int PRE_CHUNKS = 16;
+struct PreArgs {
+  const uint16_t *q, *k, *v;
+  int64_t q_ss, q_sh, k_ss, k_sh, v_ss, v_sh;
+  int64_t Sq, Sk, sqp, skp;
+  int H, nchunk, smooth_k;
+  RR rq, rk;
+  attn_ws::Work w;
+  unsigned nk, nq;   // workgroups of the K statistics and of the Q quantizer
+};
+
+__global__ void __launch_bounds__(256) pre_a_kernel(const PreArgs a) {
+  __shared__ __attribute__((aligned(16))) int8_t lds[VT_LDS];
+  static_assert(VT_LDS >= STATS_LDS, "shared by the parts");
+  unsigned b = blockIdx.x;
+  if (b < a.nk) {
+    if (a.rk.tab) stats_chunk<true>(a.k, a.k_ss, a.k_sh, a.Sk, a.rk, a.w.part, nullptr, 0, b % a.H, b / a.H, a.nchunk, lds);
+    else stats_chunk<false>(a.k, a.k_ss, a.k_sh, a.Sk, a.rk, a.w.part, nullptr, 0, b % a.H, b / a.H, a.nchunk, lds);
+    return;
+  }
+  b -= a.nk;
+  if (b < a.nq) {
+    float* wmax = reinterpret_cast<float*>(lds);
+    quant_block(a.q, a.q_ss, a.q_sh, a.Sq, a.sqp, a.rq, nullptr, a.w.q8, a.w.qs, nullptr, b % a.H, b / a.H, wmax,
+                reinterpret_cast<int*>(wmax + 4));
+    return;
+  }
+  b -= a.nq;
+  vt_slab(a.v, a.v_ss, a.v_sh, a.Sk, a.skp, a.w.vt, b % a.H, b / a.H, reinterpret_cast<uint16_t*>(lds));
+}
+
+__global__ void __launch_bounds__(256) pre_b_kernel(const PreArgs a) {
+  __shared__ double red[2][D];
+  __shared__ __attribute__((aligned(16))) float mean[D];
+  __shared__ float wmax[4];
+  __shared__ int wnorm[4];
+  const int h = blockIdx.x, d = threadIdx.x % D, j = threadIdx.x / D;
+  double t = 0.0;
+  if (a.smooth_k)
+    for (int c = j; c < a.nchunk; c += 2) t += a.w.part[(static_cast<int64_t>(h) * a.nchunk + c) * D + d];
+  red[j][d] = t;
+  __syncthreads();
+  if (j == 0) {
+    mean[d] = a.smooth_k ? static_cast<float>((red[0][d] + red[1][d]) / static_cast<double>(a.Sk)) : 0.0f;
+    if (blockIdx.y == 0) a.w.kmean[h * D + d] = mean[d];
+  }
+  __syncthreads();
+  quant_block(a.k, a.k_ss, a.k_sh, a.Sk, a.skp, a.rk, a.smooth_k ? mean : nullptr, a.w.k8, a.w.ks, a.w.kn, h, blockIdx.y, wmax,
+              wnorm);
 }
 
 // ------------------------------------------------------------------ main kernel
@@ -661,6 +733,16 @@ int prepass(const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* k, in
   const int64_t sqp = pad(Sq), skp = pad(Sk);
   const int nchunk = static_cast<int>((Sk + CHUNK - 1) / CHUNK);
   const float* mean = nullptr;
+  if (nchunk <= PRE_CHUNKS) {
+    PreArgs a{q, k, v, q_ss, q_sh, k_ss, k_sh, v_ss, v_sh, Sq, Sk, sqp, skp, static_cast<int>(H), nchunk, smooth_k, rq, rk, w,
+              0, 0};
+    const unsigned heads = static_cast<unsigned>(H);
+    a.nk = smooth_k ? heads * nchunk : 0;
+    a.nq = w.rawq ? 0 : heads * static_cast<unsigned>(sqp / BLK);   // raw queries: the main kernel quantizes them itself
+    hipLaunchKernelGGL(pre_a_kernel, dim3(a.nk + a.nq + heads * static_cast<unsigned>(skp / 64)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(pre_b_kernel, dim3(heads, static_cast<unsigned>(skp / BLK)), dim3(256), 0, st, a);
+    return launch_status("attention prepass");
+  }
   // With smoothing and the RMSNorm + RoPE prologue, the statistics pass already computes every K row's prologue:
   // it stores those rows (bf16, [H][Skpad][128]) in the V^T region, which vt_kernel fills only afterwards, and the K
   // quantizer reads them back without running the prologue a second time (the same values, so the same codes).

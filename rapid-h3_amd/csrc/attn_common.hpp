@@ -26,12 +26,13 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 // L2), STATS_NT threads = 16 token slots x 16 lanes. A row and its rope-table row are loaded together; rows past
 // S read row S - 1 and are not added, so no lane-divergent branch stands between the loads.
 constexpr int STATS_NT = 256;
+constexpr int STATS_LDS = 16 * D * 8;   // red
 template <bool RRON>
-__global__ void __launch_bounds__(STATS_NT) stats_kernel(const uint16_t* __restrict__ k, int64_t k_ss, int64_t k_sh,
-                                                    int64_t S, RR rr, double* __restrict__ part,
-                                                    uint16_t* __restrict__ kn, int64_t kn_sh) {
-  __shared__ double red[16][D];
-  const int h = blockIdx.x, c = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+__device__ __forceinline__ void stats_chunk(const uint16_t* __restrict__ k, int64_t k_ss, int64_t k_sh, int64_t S,
+                                            const RR& rr, double* __restrict__ part, uint16_t* __restrict__ kn,
+                                            int64_t kn_sh, int h, int c, int nchunk, void* lds) {
+  double(*red)[D] = static_cast<double(*)[D]>(lds);
+  const int tid = threadIdx.x, lane = tid & 63;
   const int slot = tid >> 4, l16 = tid & 15;
   double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   float w[8];
@@ -64,8 +65,15 @@ __global__ void __launch_bounds__(STATS_NT) stats_kernel(const uint16_t* __restr
   if (tid < D) {
     double t = 0.0;
     for (int i = 0; i < 16; ++i) t += red[i][tid];
-    part[(static_cast<int64_t>(h) * gridDim.y + c) * D + tid] = t;
+    part[(static_cast<int64_t>(h) * nchunk + c) * D + tid] = t;
   }
+}
+template <bool RRON>
+__global__ void __launch_bounds__(STATS_NT) stats_kernel(const uint16_t* __restrict__ k, int64_t k_ss, int64_t k_sh,
+                                                    int64_t S, RR rr, double* __restrict__ part,
+                                                    uint16_t* __restrict__ kn, int64_t kn_sh) {
+  __shared__ double red[16][D];
+  stats_chunk<RRON>(k, k_ss, k_sh, S, rr, part, kn, kn_sh, blockIdx.x, blockIdx.y, gridDim.y, red);
 }
 
 // the K statistics of one launch: stats_kernel with or without the RMSNorm + RoPE prologue; with the prologue and
@@ -107,14 +115,12 @@ __device__ __forceinline__ int claim_item(int* ctr, int nmain, int ntail, int bi
 }
 constexpr int64_t CLAIM_COUNTERS = 9;
 
-// grid (H), KMEAN_NT threads: group j of 128 channels sums chunks j, j + 8, ..., then the 8 groups
+// KMEAN_NT threads: group j of 128 channels sums chunks j, j + 8, ... (p: the head's partials of channel d), then the 8
+// groups; kmean: the head's row
 constexpr int KMEAN_NT = 1024;
-__global__ void __launch_bounds__(KMEAN_NT) kmean_kernel(const double* __restrict__ part, int nchunk, int64_t S,
-                                                         float* __restrict__ kmean) {
+__device__ __forceinline__ void kmean_fold(const double* __restrict__ p, int nchunk, int64_t S, float* __restrict__ kmean, int d,
+                                           int j, double (*red)[D]) {
   constexpr int G = KMEAN_NT / D;
-  __shared__ double red[G][D];
-  const int h = blockIdx.x, d = threadIdx.x % D, j = threadIdx.x / D;
-  const double* p = part + static_cast<int64_t>(h) * nchunk * D + d;
   double t0 = 0.0, t1 = 0.0;
   int c = j;
   for (; c + G < nchunk; c += 2 * G) {
@@ -128,8 +134,14 @@ __global__ void __launch_bounds__(KMEAN_NT) kmean_kernel(const double* __restric
     double t = 0.0;
 #pragma unroll
     for (int i = 0; i < G; ++i) t += red[i][d];
-    kmean[h * D + d] = static_cast<float>(t / static_cast<double>(S));
+    kmean[d] = static_cast<float>(t / static_cast<double>(S));
   }
+}
+__global__ void __launch_bounds__(KMEAN_NT) kmean_kernel(const double* __restrict__ part, int nchunk, int64_t S,
+                                                         float* __restrict__ kmean) {
+  __shared__ double red[KMEAN_NT / D][D];
+  const int h = blockIdx.x, d = threadIdx.x % D, j = threadIdx.x / D;
+  kmean_fold(part + static_cast<int64_t>(h) * nchunk * D + d, nchunk, S, kmean + h * D, d, j, red);
 }
 
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));

@@ -118,12 +118,15 @@ __device__ __forceinline__ void rope_tab8(const RR& rr, int l16, int64_t s, floa
   }
 }
 
-// rope_tab8 with no lane-dependent branch (lanes past rot load pair 0 of the row and ignore it), as raw bf16
-// words, so that a kernel can issue the row and table loads of several tokens before any arithmetic
+// rope_tab8 with no lane-dependent branch, as raw bf16 words, so that a kernel can issue the row and table loads of several
+// tokens before any arithmetic; lanes past rot read eight pairs of the identity rotation
+alignas(16) __device__ constexpr uint16_t ROPE_IDENTITY[32] = {
+    0x3f80, 0, 0, 0x3f80, 0x3f80, 0, 0, 0x3f80, 0x3f80, 0, 0, 0x3f80, 0x3f80, 0, 0, 0x3f80,
+    0x3f80, 0, 0, 0x3f80, 0x3f80, 0, 0, 0x3f80, 0x3f80, 0, 0, 0x3f80, 0x3f80, 0, 0, 0x3f80};
 __device__ __forceinline__ void rope_tab8_raw(const RR& rr, int l16, int64_t s, uint4* raw) {
   const int hr = rr.rot >> 1, c0 = 8 * l16;
-  const int i0 = c0 < hr ? c0 : (c0 < rr.rot ? c0 - hr : 0);
-  const uint16_t* t = rr.tab + (s * hr + i0) * 4;
+  const int i0 = c0 < hr ? c0 : c0 - hr;
+  const uint16_t* t = c0 < rr.rot ? rr.tab + (s * hr + i0) * 4 : ROPE_IDENTITY;
 #pragma unroll
   for (int q = 0; q < 4; ++q) raw[q] = *reinterpret_cast<const uint4*>(t + 8 * q);
 }
@@ -160,12 +163,19 @@ __device__ __forceinline__ void rms_rope8_pre(float* x, int lane, const RR& rr, 
   }
 }
 
+// two floats rounded to bf16 (one conversion for the pair)
+__device__ __forceinline__ void round_bf2(float& a, float& b) {
+  const uint32_t p = pack_bf2(a, b);
+  a = __uint_as_float(p << 16);
+  b = __uint_as_float(p & 0xffff0000u);
+}
+
 // rms_rope8_pre on the raw table words of rope_tab8_raw, with no lane-dependent branch. With a, b the pair of the
 // reference's formula, a first-half lane computes round_bf(a t00 + b t01) = round_bf(fma(y, t00, py t01)) and a
 // second-half lane round_bf(a t10 + b t11) = round_bf(fma(y, t11, py t10)) (a = py, b = y there): every product of
 // bf16 values is exact in fp32, so both forms round alike. Each lane therefore needs one coefficient pair (A, B):
-// (t00, t01) from the pair's first word, (t11, t10) from its second word, (1, 0) past rot; v_perm_b32 with
-// per-lane selectors moves the right bf16 halves into place, one instruction per coefficient.
+// (t00, t01) from the pair's first word, (t11, t10) from its second word ((1, 0) past rot, from the identity pairs);
+// v_perm_b32 with per-lane selectors moves the right bf16 halves into place, one instruction per coefficient.
 __device__ __forceinline__ void rms_rope8_raw(float* x, int lane, const RR& rr, const float* w, const uint4* rt) {
   const int l16 = lane & 15;
   float ss = 0.0f;
@@ -175,23 +185,25 @@ __device__ __forceinline__ void rms_rope8_raw(float* x, int lane, const RR& rr, 
   const float r = 1.0f / sqrtf(ss / 128.0f + rr.eps);
   float y[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) y[e] = round_bf((r * x[e]) * w[e]);
-  const int hr = rr.rot >> 1;
-  const int c0 = 8 * l16;
-  const bool first = c0 < hr, rotl = c0 < rr.rot;
+  for (int e = 0; e < 8; e += 2) {
+    y[e] = (r * x[e]) * w[e];
+    y[e + 1] = (r * x[e + 1]) * w[e + 1];
+    round_bf2(y[e], y[e + 1]);
+  }
+  const bool first = 8 * l16 < rr.rot >> 1;
   float py[8];
   rope_partner8(y, py, lane, rr.rot);
   // v_perm_b32(hi, lo, sel): selector bytes 0-3 take lo's bytes, 4-7 hi's, 0x0c gives 0x00
-  const uint32_t sela = first || !rotl ? 0x01000c0cu : 0x07060c0cu;  // A: lo16(word 0) or hi16(word 1)
-  const uint32_t selb = first || !rotl ? 0x03020c0cu : 0x05040c0cu;  // B: hi16(word 0) or lo16(word 1)
+  const uint32_t sela = first ? 0x01000c0cu : 0x07060c0cu;  // A: lo16(word 0) or hi16(word 1)
+  const uint32_t selb = first ? 0x03020c0cu : 0x05040c0cu;  // B: hi16(word 0) or lo16(word 1)
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const uint4 q = rt[e >> 1];
-    const uint32_t w0 = rotl ? ((e & 1) ? q.z : q.x) : 0x00003f80u;  // (1.0, 0) past rot
-    const uint32_t w1 = (e & 1) ? q.w : q.y;
+    const uint32_t w0 = (e & 1) ? q.z : q.x, w1 = (e & 1) ? q.w : q.y;
     const float A = __uint_as_float(__builtin_amdgcn_perm(w1, w0, sela));
     const float B = __uint_as_float(__builtin_amdgcn_perm(w1, w0, selb));
-    x[e] = round_bf(fmaf(y[e], A, py[e] * B));
+    x[e] = fmaf(y[e], A, py[e] * B);
+    if (e & 1) round_bf2(x[e - 1], x[e]);
   }
 }
 
@@ -210,12 +222,11 @@ __device__ __forceinline__ void wht128_row(float* v, int l16) {
       }
   auto stage = [&](auto mc) __attribute__((always_inline)) {
     constexpr int M = decltype(mc)::value;
-    const bool hi = l16 & M;
+    // the upper lane of a pair holds hi and gets lo - hi, the lower lo + hi: the partner's value plus the own one, negated
+    // in the upper lane (exact), as one XOR and one add that reads its partner through DPP
+    const uint32_t neg = l16 & M ? 0x80000000u : 0u;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float y = xor16<M>(v[e]);
-      v[e] = hi ? y - v[e] : v[e] + y;
-    }
+    for (int e = 0; e < 8; ++e) v[e] = xor16<M>(v[e]) + __uint_as_float(__float_as_uint(v[e]) ^ neg);
   };
   stage(std::integral_constant<int, 1>{});
   stage(std::integral_constant<int, 2>{});
@@ -229,11 +240,11 @@ __device__ __forceinline__ void wht128_row(float* v, int l16) {
 __device__ __forceinline__ float row_amax16(const float* v) {
   float amax = 0.0f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[e]));
-  amax = fmaxf(amax, xor16<8>(amax));
-  amax = fmaxf(amax, xor16<4>(amax));
-  amax = fmaxf(amax, xor16<2>(amax));
-  amax = fmaxf(amax, xor16<1>(amax));
+  for (int e = 0; e < 8; e += 2) amax = max3_abs(amax, v[e], v[e + 1]);
+  amax = fmax_nc(amax, xor16<8>(amax));
+  amax = fmax_nc(amax, xor16<4>(amax));
+  amax = fmax_nc(amax, xor16<2>(amax));
+  amax = fmax_nc(amax, xor16<1>(amax));
   return amax;
 }
 
@@ -242,11 +253,11 @@ __device__ __forceinline__ float row_amax16(const float* v) {
 __device__ __forceinline__ float token_quant_row(const float* v, uint2& codes) {
   const float sc = fmaxf(row_amax16(v), 1e-8f) / 127.0f;
   const float inv = 1.0f / sc;
-  uint32_t b[8];
+  // |v * inv| <= 127 (1 + 2^-22): pack4_codes rounds to nearest even by its magic-number add and packs the low bytes
+  float n[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) b[e] = static_cast<uint32_t>(static_cast<int32_t>(rintf(v[e] * inv))) & 0xffu;
-  codes.x = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
-  codes.y = b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24);
+  for (int e = 0; e < 8; ++e) n[e] = v[e] * inv;
+  codes = make_uint2(pack4_codes(n), pack4_codes(n + 4));
   return sc;
 }
 

@@ -32,6 +32,8 @@ namespace rh3 {
 namespace {
 
 using namespace attn;
+using attn_ws::WorkU8;
+using attn_ws::layout_u8;
 
 constexpr int TILE = 128;                 // keys per tile (the tile max of the u8 P)
 constexpr int SIDE = 2048;                // bytes per (head, tile): 128 (s, b) pairs, 128 int32 starts, pad
@@ -47,12 +49,25 @@ constexpr float INV_SQRT128 = 0.08838834764831845f;  // attn_int8.cu:127
 // ------------------------------------------------------------------ V statistics
 // grid (H, nchunk) (heads fastest, so a chunk's token rows are read together), 256 threads = 16 token slots x 16
 // lanes (8 channels each)
-__global__ void __launch_bounds__(256) vstats_kernel(const uint16_t* __restrict__ v, int64_t v_ss, int64_t v_sh,
-                                                     int64_t S, double* __restrict__ vsum,
-                                                     float* __restrict__ vmax, float* __restrict__ vmin) {
-  __shared__ double red[16][D];
-  __shared__ float rmx[16][D], rmn[16][D];
-  const int h = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
+constexpr int VSTATS_LDS = 16 * D * (8 + 4 + 4);
+// max / min of three floats in one instruction (fmaxf and fminf chains get a NaN-quieting max per operand)
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+__device__ __forceinline__ float min3(float a, float b, float c) {
+  float r;
+  asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+__device__ __forceinline__ void vstats_chunk(const uint16_t* __restrict__ v, int64_t v_ss, int64_t v_sh, int64_t S,
+                                             double* __restrict__ vsum, float* __restrict__ vmax,
+                                             float* __restrict__ vmin, int h, int c, int nchunk, void* lds) {
+  double(*red)[D] = static_cast<double(*)[D]>(lds);
+  float(*rmx)[D] = reinterpret_cast<float(*)[D]>(red + 16);
+  float(*rmn)[D] = rmx + 16;
+  const int tid = threadIdx.x;
   const int slot = tid >> 4, l16 = tid & 15;
   double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   float mx[8], mn[8];
@@ -66,19 +81,28 @@ __global__ void __launch_bounds__(256) vstats_kernel(const uint16_t* __restrict_
       const int64_t s = static_cast<int64_t>(c) * CHUNK + (it0 + i) * 16 + slot;
       rx[i] = *reinterpret_cast<const uint4*>(v + (s < S ? s : S - 1) * v_ss + h * v_sh + 8 * l16);
     }
+    // max and min two rows at a time, the sums row by row
+    auto rows = [&](auto full) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (static_cast<int64_t>(c) * CHUNK + (it0 + i) * 16 + slot < S) {
-        float x[8];
+      for (int i = 0; i < 4; i += 2) {
+        const int64_t s0 = static_cast<int64_t>(c) * CHUNK + (it0 + i) * 16 + slot;
+        if (!full && s0 >= S) return;
+        const bool two = full || s0 + 16 < S;
+        float x[8], y[8];
         unpack8(rx[i], x);
+        unpack8(rx[i + 1], y);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
+          const float z = two ? y[e] : x[e];
+          mx[e] = max3(mx[e], x[e], z);
+          mn[e] = min3(mn[e], x[e], z);
           acc[e] += static_cast<double>(x[e]);
-          mx[e] = fmaxf(mx[e], x[e]);
-          mn[e] = fminf(mn[e], x[e]);
+          if (two) acc[e] += static_cast<double>(y[e]);
         }
       }
-    }
+    };
+    if (static_cast<int64_t>(c + 1) * CHUNK <= S) rows(std::true_type{});   // uniform: no row of the chunk past S
+    else rows(std::false_type{});
   }
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -95,32 +119,37 @@ __global__ void __launch_bounds__(256) vstats_kernel(const uint16_t* __restrict_
       a = fmaxf(a, rmx[i][tid]);
       b = fminf(b, rmn[i][tid]);
     }
-    const int64_t o = (static_cast<int64_t>(h) * gridDim.y + c) * D + tid;
+    const int64_t o = (static_cast<int64_t>(h) * nchunk + c) * D + tid;
     vsum[o] = t;
     vmax[o] = a;
     vmin[o] = b;
   }
 }
 
-// grid H, VFINAL_NT threads: group j of 128 channels folds chunks j, j + 8, ..., then the 8 groups (the float64
-// sums of bf16 values are exact and max / min are order-free, so the grouping does not change the result)
-constexpr int VFINAL_NT = 1024;
-__global__ void __launch_bounds__(VFINAL_NT) vfinal_kernel(const double* __restrict__ vsum,
-                                                           const float* __restrict__ vmax,
-                                                           const float* __restrict__ vmin, int nchunk, int64_t S,
-                                                           int smooth_v, float* __restrict__ vmean,
-                                                           float* __restrict__ vscale) {
-  constexpr int G = VFINAL_NT / D;
+// grid (H, 2), KMEAN_NT threads: y = 0 the K mean (kmean_kernel's fold; zeros without smoothing), y = 1 V's mean and scale:
+// group j of 128 channels folds chunks j, j + 8, ..., then the 8 groups (the float64 sums of bf16 values are exact and max /
+// min are order-free, so the grouping does not change the result). The first workgroup also clears the work counter.
+__global__ void __launch_bounds__(KMEAN_NT) kmean_vfinal_kernel(const WorkU8 w, int nchunk, int64_t S, int smooth_k, int smooth_v) {
+  constexpr int G = KMEAN_NT / D;
   __shared__ double rs[G][D];
   __shared__ float rmx[G][D], rmn[G][D];
   const int h = blockIdx.x, d = threadIdx.x % D, j = threadIdx.x / D;
+  if (blockIdx.y == 0) {
+    if (h == 0 && threadIdx.x == 0) *w.ctr = 0;
+    if (!smooth_k) {
+      if (j == 0) w.kmean[h * D + d] = 0.0f;
+      return;
+    }
+    kmean_fold(w.kpart + static_cast<int64_t>(h) * nchunk * D + d, nchunk, S, w.kmean + h * D, d, j, rs);
+    return;
+  }
   double t = 0.0;
   float a = -INFINITY, b = INFINITY;
   for (int c = j; c < nchunk; c += G) {
     const int64_t o = (static_cast<int64_t>(h) * nchunk + c) * D + d;
-    t += vsum[o];
-    a = fmaxf(a, vmax[o]);
-    b = fminf(b, vmin[o]);
+    t += w.vsum[o];
+    a = fmaxf(a, w.vmax[o]);
+    b = fminf(b, w.vmin[o]);
   }
   rs[j][d] = t;
   rmx[j][d] = a;
@@ -134,80 +163,77 @@ __global__ void __launch_bounds__(VFINAL_NT) vfinal_kernel(const double* __restr
     b = fminf(b, rmn[i][d]);
   }
   const float vm = smooth_v ? static_cast<float>(t / static_cast<double>(S)) : 0.0f;
-  vmean[h * D + d] = vm;
-  vscale[h * D + d] = fmaxf(fmaxf(a - vm, vm - b), 1e-6f) / 127.0f;
+  w.vmean[h * D + d] = vm;
+  w.vscale[h * D + d] = fmaxf(fmaxf(a - vm, vm - b), 1e-6f) / 127.0f;
 }
 
 // ------------------------------------------------------------------ per-token Q / K quantizer
-// 256 threads = 16 rows of 16 lanes; row g = blockIdx.x * 16 + tid / 16 is (token g / H, head g % H), heads
-// fastest. grid = Spad * H / 16 (Spad is a multiple of 128).
-__global__ void __launch_bounds__(256) tokq_kernel(const uint16_t* __restrict__ x, int64_t x_ss, int64_t x_sh,
-                                                   int64_t S, int64_t Spad, int64_t H, RR rr,
-                                                   const float* __restrict__ mean, int rotate,
-                                                   int8_t* __restrict__ codes, float* __restrict__ scales,
-                                                   float* __restrict__ side) {
+// 256 threads = 16 groups of 16 lanes; group i = block * 16 + tid / 16 takes the TOKQ_ROWS tokens TOKQ_ROWS (i / H) .. of head
+// i % H (heads fastest, so a workgroup's rope-table rows are shared). Bound by VALU: about 260 instructions per 8 values with
+// RMSNorm + RoPE, against 522 with one row per group (half of them addresses, norm weights and the division by H) and
+// selects in the transform.
+constexpr int TOKQ_ROWS = 4;
+__device__ __forceinline__ void tokq_rows(const uint16_t* __restrict__ x, int64_t x_ss, int64_t x_sh, int64_t S, int64_t Spad,
+                                          int H, const RR& rr, const float* __restrict__ mean, int rotate,
+                                          int8_t* __restrict__ codes, float* __restrict__ scales, float* __restrict__ side,
+                                          uint32_t block) {
   const int tid = threadIdx.x, lane = tid & 63, l16 = tid & 15;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 16 + (tid >> 4);
-  const int64_t s = row / H, h = row % H;
-  const int64_t co = (h * Spad + s) * D + 8 * l16;
-  if (s >= S) {  // uniform per 16-lane row: padded rows and keys
-    *reinterpret_cast<uint2*>(codes + co) = make_uint2(0, 0);
-    if (l16 == 0) {
-      scales[h * Spad + s] = 0.0f;
-      if (side) {
-        float* p = side + ((h * (Spad / TILE) + s / TILE) * SIDE) / 4 + 2 * (s % TILE);
-        *reinterpret_cast<float2*>(p) = make_float2(0.0f, -INFINITY);
-      }
-    }
-    return;
+  const uint32_t i = block * 16 + (tid >> 4), q4 = i / static_cast<uint32_t>(H);   // Spad * H < 2^31
+  const int h = static_cast<int>(i - q4 * H);
+  const int64_t s0 = static_cast<int64_t>(q4) * TOKQ_ROWS;
+  int8_t* co = codes + (h * Spad + s0) * D + 8 * l16;
+  float* sc_out = scales + h * Spad + s0;
+  // TOKQ_ROWS tokens lie in one tile (TILE is a multiple)
+  float2* pair = side ? reinterpret_cast<float2*>(side + (h * (Spad / TILE) + s0 / TILE) * (SIDE / 4)) + s0 % TILE : nullptr;
+  // the rows, their rope-table rows and the norm weights are loaded together, before any arithmetic (rows past S read the
+  // last one)
+  const uint16_t* xp = x + h * x_sh + 8 * l16;
+  uint4 rx[TOKQ_ROWS], rt[TOKQ_ROWS][4];
+#pragma unroll
+  for (int u = 0; u < TOKQ_ROWS; ++u) {
+    const int64_t sl = s0 + u < S ? s0 + u : S - 1;
+    rx[u] = *reinterpret_cast<const uint4*>(xp + sl * x_ss);
+    if (rr.tab) rope_tab8_raw(rr, l16, sl, rt[u]);
   }
-  // the row, the rope-table row and the norm weights are loaded together, before any arithmetic
-  const uint4 rx = *reinterpret_cast<const uint4*>(x + s * x_ss + h * x_sh + 8 * l16);
-  uint4 rt[4];
-  uint4 rw = make_uint4(0, 0, 0, 0);
-  if (rr.tab) {
-    rope_tab8_raw(rr, l16, s, rt);
-    rw = *reinterpret_cast<const uint4*>(rr.w + 8 * l16);
-  }
-  float v[8];
-  unpack8(rx, v);
-  if (rr.tab) {
-    float w[8];
-    unpack8(rw, w);
-    rms_rope8_raw(v, lane, rr, w, rt);
-  }
+  float w[8], m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (rr.tab) load8(rr.w + 8 * l16, w);
   if (mean) {
-    float m[8];
     const float4 a = *reinterpret_cast<const float4*>(mean + h * D + 8 * l16);
     const float4 b = *reinterpret_cast<const float4*>(mean + h * D + 8 * l16 + 4);
     m[0] = a.x; m[1] = a.y; m[2] = a.z; m[3] = a.w; m[4] = b.x; m[5] = b.y; m[6] = b.z; m[7] = b.w;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = v[e] - m[e];
   }
-  if (rotate) wht128_row(v, l16);
-  uint2 o;
-  const float sc = token_quant_row(v, o);
-  *reinterpret_cast<uint2*>(codes + co) = o;
-  if (l16 == 0) {
-    scales[h * Spad + s] = sc;
-    if (side) {
-      float* p = side + ((h * (Spad / TILE) + s / TILE) * SIDE) / 4 + 2 * (s % TILE);
-      *reinterpret_cast<float2*>(p) = make_float2(sc, -MAGIC_F * sc);
+#pragma unroll
+  for (int u = 0; u < TOKQ_ROWS; ++u) {
+    const bool ok = s0 + u < S;   // uniform per 16-lane row
+    float v[8];
+    unpack8(rx[u], v);
+    if (rr.tab) rms_rope8_raw(v, lane, rr, w, rt[u]);
+    if (mean) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = v[e] - m[e];
+    }
+    if (rotate) wht128_row(v, l16);
+    uint2 o;
+    const float sc = token_quant_row(v, o);
+    *reinterpret_cast<uint2*>(co + u * D) = ok ? o : make_uint2(0, 0);   // padded rows and keys: zero codes
+    if (l16 == 0) {
+      sc_out[u] = ok ? sc : 0.0f;
+      if (pair) pair[u] = ok ? make_float2(sc, -MAGIC_F * sc) : make_float2(0.0f, -INFINITY);
     }
   }
 }
+inline unsigned tokq_blocks(int64_t Spad, int64_t H) { return static_cast<unsigned>((Spad / TOKQ_ROWS * H + 15) / 16); }
 
 // ------------------------------------------------------------------ per-block K (configs 60-61)
 // grid (H, Skpad / 128) (heads fastest), 256 threads: wave w quantizes tokens 32 w .. 32 w + 31 of the block, four 16-lane rows
 // per pass. K - kmean -> [normalized H128] -> one scale per (head, 128-key block) sc = max(amax, 1e-8) / 127,
 // codes rint(x * (1 / sc)) (quant_k_block, attn_int8.cu:404-443); sc goes to kbs [H][Skpad/128] and to the first
 // float of the block's side record, where the main kernel reads it. Padded tokens are zero rows.
-__global__ void __launch_bounds__(256) blockk_kernel(const uint16_t* __restrict__ k, int64_t k_ss, int64_t k_sh,
-                                                     int64_t S, int64_t Spad, const float* __restrict__ mean,
-                                                     int rotate, int8_t* __restrict__ codes,
-                                                     float* __restrict__ kbs, float* __restrict__ side) {
-  __shared__ float wmax[4];
-  const int h = blockIdx.x, blk = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+__device__ __forceinline__ void blockk_tile(const uint16_t* __restrict__ k, int64_t k_ss, int64_t k_sh, int64_t S,
+                                            int64_t Spad, const float* __restrict__ mean, int rotate,
+                                            int8_t* __restrict__ codes, float* __restrict__ kbs, float* __restrict__ side,
+                                            int h, int blk, float* wmax) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, sub = lane >> 4;
   float m[8];
   {
@@ -274,15 +300,14 @@ __device__ __forceinline__ int perm_f8(int p) {
 
 // grid (H, Skpad / 128) (heads fastest), 256 threads. F8 (configs 50-56): e4m3 codes of ((v - vmean) / vscale) *
 // fp32(448 / 127) (attn_int8.cu:467-473) in the perm_f8 order, and no accumulator starts.
+constexpr int VQ_PITCH = D + 16;  // row pitch of the key-major code tile
 template <bool F8>
-__global__ void __launch_bounds__(256) vq_kernel(const uint16_t* __restrict__ v, int64_t v_ss, int64_t v_sh,
-                                                 int64_t S, int64_t Spad, const float* __restrict__ vmean,
-                                                 const float* __restrict__ vscale, int8_t* __restrict__ vt,
-                                                 int32_t* __restrict__ side) {
-  constexpr int P = D + 16;  // row pitch of the key-major code tile
-  __shared__ int8_t tile[TILE * P];
-  const int h = blockIdx.x, tid = threadIdx.x, l16 = tid & 15;
-  const int64_t s0 = static_cast<int64_t>(blockIdx.y) * TILE;
+__device__ __forceinline__ void vq_tile(const uint16_t* __restrict__ v, int64_t v_ss, int64_t v_sh, int64_t S, int64_t Spad,
+                                        const float* __restrict__ vmean, const float* __restrict__ vscale,
+                                        int8_t* __restrict__ vt, int32_t* __restrict__ side, int h, int blk, int8_t* tile) {
+  constexpr int P = VQ_PITCH;
+  const int tid = threadIdx.x, l16 = tid & 15;
+  const int64_t s0 = static_cast<int64_t>(blk) * TILE;
   float vm[8], vs[8], iv[8];
   {
     const float4 a = *reinterpret_cast<const float4*>(vmean + h * D + 8 * l16);
@@ -307,39 +332,126 @@ __global__ void __launch_bounds__(256) vq_kernel(const uint16_t* __restrict__ v,
         o.x = __builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], 0, false), true);
         o.y = __builtin_amdgcn_cvt_pk_fp8_f32(y[6], y[7], __builtin_amdgcn_cvt_pk_fp8_f32(y[4], y[5], 0, false), true);
       } else {
-        uint32_t b[8];
+        // rint_div with one wave vote per 8 values: |x * inv| < 128, so the product lies within 2^-15 of the IEEE quotient
+        float n[8], d = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          b[e] = static_cast<uint32_t>(static_cast<int32_t>(rint_div(x[e] - vm[e], vs[e], iv[e]))) & 0xffu;
-        o.x = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
-        o.y = b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24);
+        for (int e = 0; e < 8; ++e) x[e] = x[e] - vm[e];
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          const float t0 = x[e] * iv[e], t1 = x[e + 1] * iv[e + 1];
+          n[e] = rintf(t0);
+          n[e + 1] = rintf(t1);
+          d = max3_abs(d, t0 - n[e], t1 - n[e + 1]);
+        }
+        if (__builtin_amdgcn_ballot_w64(d > 0.5f - 0x1p-14f) != 0) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            float so = vs[e];   // opaque, so that the division's divisor-only steps stay on this path
+            asm volatile("" : "+v"(so));
+            if (fabsf(x[e] * iv[e] - n[e]) > 0.5f - 0x1p-14f) n[e] = rintf(x[e] / so);
+          }
+        }
+        o = make_uint2(pack4_codes(n), pack4_codes(n + 4));
       }
     }
     *reinterpret_cast<uint2*>(&tile[r * P + 8 * l16]) = o;
   }
   __syncthreads();
-  // V^T rows: channel d, 16 positions per store (8 stores of 16 B per row)
-  for (int i = tid; i < D * (TILE / 16); i += 256) {
-    const int d = i >> 3, pc = (i & 7) * 16;  // positions pc..pc+15 of this tile
-    uint32_t w[4] = {0, 0, 0, 0};
+  // thread i: channels 4 (i / 8) .. +3, positions 16 (i % 8) .. +15 of the tile, by 4 x 4 byte transposes (four keys' words
+  // in, four channels' out)
+  const int d0 = 4 * (tid >> 3), pc = (tid & 7) * 16;
+  uint32_t w[4][4];   // [channel][position / 4]
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int p = pc + e;
+  for (int t = 0; t < 4; ++t) {
+    uint32_t k[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int p = pc + 4 * t + e;
       const int key = F8 ? (p & ~63) + perm_f8(p & 63) : (p & ~31) + perm_u8(p & 31);
-      w[e >> 2] |= (static_cast<uint32_t>(static_cast<uint8_t>(tile[key * P + d]))) << (8 * (e & 3));
+      k[e] = *reinterpret_cast<const uint32_t*>(&tile[key * P + d0]);
     }
-    *reinterpret_cast<uint4*>(vt + (static_cast<int64_t>(h) * D + d) * Spad + s0 + pc) =
-        make_uint4(w[0], w[1], w[2], w[3]);
+    // v_perm_b32(hi, lo, sel): selector bytes 0-3 take lo's bytes, 4-7 hi's
+    const uint32_t a01 = __builtin_amdgcn_perm(k[1], k[0], 0x05010400u), a23 = __builtin_amdgcn_perm(k[3], k[2], 0x05010400u);
+    const uint32_t b01 = __builtin_amdgcn_perm(k[1], k[0], 0x07030602u), b23 = __builtin_amdgcn_perm(k[3], k[2], 0x07030602u);
+    w[0][t] = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
+    w[1][t] = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
+    w[2][t] = __builtin_amdgcn_perm(b23, b01, 0x05040100u);
+    w[3][t] = __builtin_amdgcn_perm(b23, b01, 0x07060302u);
   }
-  // accumulator starts: 1.5*2^23 bits + 128 * (sum of the tile's codes of channel d); the pad is zeroed
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    *reinterpret_cast<uint4*>(vt + (static_cast<int64_t>(h) * D + d0 + c) * Spad + s0 + pc) =
+        make_uint4(w[c][0], w[c][1], w[c][2], w[c][3]);
+  // accumulator starts: 1.5*2^23 bits + 128 * (sum of the tile's codes of channel d), over the 8 threads of a channel; the
+  // pad is zeroed
   if constexpr (F8) return;
-  int32_t* rec = side + (static_cast<int64_t>(h) * (Spad / TILE) + blockIdx.y) * (SIDE / 4);
-  if (tid < D) {
-    int sum = 0;
-    for (int k = 0; k < TILE; ++k) sum += static_cast<int8_t>(tile[k * P + tid]);
-    rec[SIDE_VINIT / 4 + tid] = MAGIC_I + 128 * sum;
+  int32_t* rec = side + (static_cast<int64_t>(h) * (Spad / TILE) + blk) * (SIDE / 4);
+  int sum[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    int t = 0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) t = __builtin_amdgcn_sdot4(static_cast<int>(w[c][u]), 0x01010101, t, false);
+    t += __builtin_amdgcn_update_dpp(0, t, 0xB1, 0xf, 0xf, true);    // lane ^ 1
+    t += __builtin_amdgcn_update_dpp(0, t, 0x4E, 0xf, 0xf, true);    // lane ^ 2
+    t += __builtin_amdgcn_update_dpp(0, t, 0x141, 0xf, 0xf, true);   // 7 - lane of the 8: the other four's sum
+    sum[c] = MAGIC_I + 128 * t;
+  }
+  if ((tid & 7) == 0) {
+    *reinterpret_cast<int4*>(rec + SIDE_VINIT / 4 + d0) = make_int4(sum[0], sum[1], sum[2], sum[3]);
+    *reinterpret_cast<int4*>(rec + SIDE_VINIT / 4 + D + d0) = make_int4(0, 0, 0, 0);
+  }
+}
+
+// ------------------------------------------------------------------ the pre-pass in three launches
+// A: K statistics (smoothing), V statistics and the Q quantizer; kmean_vfinal_kernel: their second level; B: the K quantizer
+// and the V codes. The parts of one launch do not depend on each other; run as eight launches of their own, the small ones cost
+// more in launch gaps than in work and the memory-bound ones ran beside no arithmetic. Whole pre-pass with RMSNorm + RoPE (us,
+// before and now): 1,560 tokens x 24 heads 60 and 42, 5,583 x 56 193 and 168, 22,332 x 56 670 and 611; A is bound by VALU
+// (94 % busy), B by VALU and HBM together.
+struct PreU8 {
+  const uint16_t *q, *k, *v;
+  int64_t q_ss, q_sh, k_ss, k_sh, v_ss, v_sh;
+  int64_t Sq, Sk, sqp, skp;
+  int H, nchunk, smooth_k, smooth_v, rotate;
+  RR rq, rk;
+  WorkU8 w;
+  unsigned nk, nv;   // workgroups of the first two parts (A: K and V statistics; B: nk of the K quantizer)
+};
+
+__global__ void __launch_bounds__(256) pre_a_u8_kernel(const PreU8 a) {
+  __shared__ __attribute__((aligned(16))) int8_t lds[VSTATS_LDS];
+  static_assert(VSTATS_LDS >= STATS_LDS, "shared by the parts");
+  unsigned b = blockIdx.x;
+  if (b < a.nk) {
+    if (a.rk.tab) stats_chunk<true>(a.k, a.k_ss, a.k_sh, a.Sk, a.rk, a.w.kpart, nullptr, 0, b % a.H, b / a.H, a.nchunk, lds);
+    else stats_chunk<false>(a.k, a.k_ss, a.k_sh, a.Sk, a.rk, a.w.kpart, nullptr, 0, b % a.H, b / a.H, a.nchunk, lds);
+    return;
+  }
+  b -= a.nk;
+  if (b < a.nv) {
+    vstats_chunk(a.v, a.v_ss, a.v_sh, a.Sk, a.w.vsum, a.w.vmax, a.w.vmin, b % a.H, b / a.H, a.nchunk, lds);
+    return;
+  }
+  b -= a.nv;
+  tokq_rows(a.q, a.q_ss, a.q_sh, a.Sq, a.sqp, a.H, a.rq, nullptr, a.rotate, a.w.q8, a.w.qs, nullptr, b);
+}
+
+// V: 0 int8 codes, 1 e4m3 codes; BLK: K quantized per 128-key block (configs 60-61) instead of per token
+template <bool F8, bool BLK>
+__global__ void __launch_bounds__(256) pre_b_u8_kernel(const PreU8 a) {
+  __shared__ __attribute__((aligned(16))) int8_t tile[TILE * VQ_PITCH];
+  const unsigned b = blockIdx.x;
+  if (b >= a.nk) {
+    const unsigned t = b - a.nk;
+    vq_tile<F8>(a.v, a.v_ss, a.v_sh, a.Sk, a.skp, a.w.vmean, a.w.vscale, a.w.vt, reinterpret_cast<int32_t*>(a.w.side), t % a.H,
+                t / a.H, tile);
+  } else if constexpr (BLK) {
+    blockk_tile(a.k, a.k_ss, a.k_sh, a.Sk, a.skp, a.w.kmean, a.rotate, a.w.k8, a.w.ks, reinterpret_cast<float*>(a.w.side),
+                b % a.H, b / a.H, reinterpret_cast<float*>(tile));
   } else {
-    rec[SIDE_VINIT / 4 + tid] = 0;
+    tokq_rows(a.k, a.k_ss, a.k_sh, a.Sk, a.skp, a.H, a.rk, a.smooth_k ? a.w.kmean : nullptr, a.rotate, a.w.k8, a.w.ks,
+              reinterpret_cast<float*>(a.w.side), b);
   }
 }
 
@@ -371,13 +483,6 @@ constexpr int U8_WAVES = 4, U8_NT = U8_WAVES * 64, U8_BQ = U8_WAVES * 32;
 
 typedef __attribute__((address_space(3))) const v4i lds_v4i_u8;
 typedef __attribute__((address_space(3))) const float lds_f32_u8;
-
-// max of three floats in one instruction (fmaxf chains get a NaN-quieting max inserted per operand)
-__device__ __forceinline__ float max3f(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
 
 // Tile j reads K(j), V^T(j) and its side record from ring slot j % 2 and first loads tile j + 1 into the other slot, whose
 // last reads returned before the barrier that ended tile j - 1.
@@ -562,7 +667,7 @@ __global__ void __launch_bounds__(U8_NT, 2) attn_u8_kernel(const U8Args a) {
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-      for (int r = 0; r < 16; r += 2) tm = max3f(tm, t[kb][r], t[kb][r + 1]);
+      for (int r = 0; r < 16; r += 2) tm = max3(tm, t[kb][r], t[kb][r + 1]);
     {
       const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(tm), __float_as_int(tm), false, false);
       tm = fmaxf(__int_as_float(sw[0]), __int_as_float(sw[1]));
@@ -654,7 +759,7 @@ __global__ void __launch_bounds__(U8_NT, 2) attn_u8_kernel(const U8Args a) {
 #pragma unroll
         for (int kb = 2 * cc; kb < 2 * cc + MAXG / 32; ++kb)
 #pragma unroll
-          for (int r = 0; r < 16; r += 2) tm = max3f(tm, t[kb][r], t[kb][r + 1]);
+          for (int r = 0; r < 16; r += 2) tm = max3(tm, t[kb][r], t[kb][r + 1]);
         {
           const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(tm), __float_as_int(tm), false, false);
           tm = fmaxf(__int_as_float(sw[0]), __int_as_float(sw[1]));
@@ -756,8 +861,6 @@ __global__ void __launch_bounds__(U8_NT, 2) attn_u8_kernel(const U8Args a) {
 
 // ------------------------------------------------------------------ host
 static_assert(TILE == attn_ws::BLK && SIDE == attn_ws::SIDE, "workspace layout constants");
-using attn_ws::WorkU8;
-using attn_ws::layout_u8;
 inline int64_t padk(int64_t s) { return attn_ws::pad(s); }
 
 int check_qkv_u8(const char* name, const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* k, int64_t k_ss,
@@ -782,65 +885,63 @@ int check_rr_u8(const char* name, const uint16_t* tab, int rot, const uint16_t* 
   return RH3_OK;
 }
 
+// the second level of the statistics, then the K quantizer and the V codes
+template <bool F8, bool BLK>
+int prepass_tail(PreU8& a, hipStream_t st, const char* name) {
+  hipLaunchKernelGGL(kmean_vfinal_kernel, dim3(a.H, 2), dim3(KMEAN_NT), 0, st, a.w, a.nchunk, a.Sk, a.smooth_k, a.smooth_v);
+  const unsigned tiles = static_cast<unsigned>(a.skp / TILE * a.H);
+  a.nk = BLK ? tiles : tokq_blocks(a.skp, a.H);
+  hipLaunchKernelGGL((pre_b_u8_kernel<F8, BLK>), dim3(a.nk + tiles), dim3(256), 0, st, a);
+  return launch_status(name);
+}
+template <bool F8, bool BLK>
+int prepass_all(PreU8& a, hipStream_t st, const char* name) {
+  const unsigned chunks = static_cast<unsigned>(a.nchunk) * a.H;
+  a.nk = a.smooth_k ? chunks : 0;
+  a.nv = chunks;
+  hipLaunchKernelGGL(pre_a_u8_kernel, dim3(a.nk + a.nv + tokq_blocks(a.sqp, a.H)), dim3(256), 0, st, a);
+  return prepass_tail<F8, BLK>(a, st, name);
+}
+
 int prepass_u8(const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* k, int64_t k_ss, int64_t k_sh,
                const uint16_t* v, int64_t v_ss, int64_t v_sh, int64_t Sq, int64_t Sk, int64_t H, const RR& rq,
                const RR& rk, int smooth_k, int smooth_v, int rotate, const WorkU8& w, hipStream_t st,
                bool f8 = false) {
-  const int64_t sqp = padk(Sq), skp = padk(Sk);
-  const int nchunk = static_cast<int>((Sk + CHUNK - 1) / CHUNK);
-  const float* mean = nullptr;
-  if (smooth_k) {
-    launch_stats(dim3(H, nchunk), st, k, k_ss, k_sh, Sk, rk, w.kpart);
-    hipLaunchKernelGGL(kmean_kernel, dim3(H), dim3(KMEAN_NT), 0, st, w.kpart, nchunk, Sk, w.kmean);
-    mean = w.kmean;
-  } else {
-    // a fill kernel, not hipMemsetAsync, so the call stays safe inside a captured HIP graph
-    hipLaunchKernelGGL(zero_kernel, dim3((H * D + 255) / 256), dim3(256), 0, st, w.kmean, H * D);
-  }
-  hipLaunchKernelGGL(vstats_kernel, dim3(H, nchunk), dim3(256), 0, st, v, v_ss, v_sh, Sk, w.vsum, w.vmax, w.vmin);
-  hipLaunchKernelGGL(vfinal_kernel, dim3(H), dim3(VFINAL_NT), 0, st, w.vsum, w.vmax, w.vmin, nchunk, Sk, smooth_v, w.vmean,
-                     w.vscale);
-  hipLaunchKernelGGL(tokq_kernel, dim3(sqp * H / 16), dim3(256), 0, st, q, q_ss, q_sh, Sq, sqp, H, rq,
-                     static_cast<const float*>(nullptr), rotate, w.q8, w.qs, static_cast<float*>(nullptr));
-  hipLaunchKernelGGL(tokq_kernel, dim3(skp * H / 16), dim3(256), 0, st, k, k_ss, k_sh, Sk, skp, H, rk, mean, rotate,
-                     w.k8, w.ks, reinterpret_cast<float*>(w.side));
-  if (f8)  // configs 50-56: e4m3 V codes (attn_int8.cu:2639-2642)
-    hipLaunchKernelGGL(vq_kernel<true>, dim3(H, skp / TILE), dim3(256), 0, st, v, v_ss, v_sh, Sk, skp, w.vmean,
-                       w.vscale, w.vt, reinterpret_cast<int32_t*>(w.side));
-  else
-    hipLaunchKernelGGL(vq_kernel<false>, dim3(H, skp / TILE), dim3(256), 0, st, v, v_ss, v_sh, Sk, skp, w.vmean,
-                       w.vscale, w.vt, reinterpret_cast<int32_t*>(w.side));
-  return launch_status("attention_u8 prepass");
+  PreU8 a{q, k, v, q_ss, q_sh, k_ss, k_sh, v_ss, v_sh, Sq, Sk, padk(Sq), padk(Sk), static_cast<int>(H),
+          static_cast<int>(attn_ws::nchunks(Sk)), smooth_k, smooth_v, rotate, rq, rk, w, 0, 0};
+  // configs 50-56: e4m3 V codes (attn_int8.cu:2639-2642)
+  return f8 ? prepass_all<true, false>(a, st, "attention_u8 prepass") : prepass_all<false, false>(a, st, "attention_u8 prepass");
 }
 
 // Grid of the main kernel, whose workgroups take their (head, query block) items from a work counter: the grid is
 // dealt to the XCDs in fixed shares and the XCDs run at different clocks, so the grid holds a quarter more
 // workgroups than items (room for the fastest XCD to take a quarter more than its share); the extra ones return
-// at once. gridDim.y carries H. The counter is cleared first by a fill kernel (no hipMemsetAsync: graph-safe).
-dim3 claim_grid(U8Args& f, const WorkU8& w, int64_t Sq, int64_t H, hipStream_t st) {
+// at once. gridDim.y carries H. The counter is cleared first by a fill kernel (no hipMemsetAsync: graph-safe), unless the
+// pre-pass of the same call just did.
+dim3 claim_grid(U8Args& f, const WorkU8& w, int64_t Sq, int64_t H, hipStream_t st, bool cleared) {
   f.nqb = static_cast<int>((Sq + U8_BQ - 1) / U8_BQ);
   f.ctr = w.ctr;
   const int64_t per_head = f.nqb + (f.nqb + 3) / 4;
-  hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, st, reinterpret_cast<float*>(w.ctr), int64_t{1});
+  if (!cleared) hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, st, reinterpret_cast<float*>(w.ctr), int64_t{1});
   return dim3(static_cast<uint32_t>(per_head), static_cast<uint32_t>(H));
 }
 
 // configs 50-56: the FP8 P.V main kernel; tile = the reference's BN (64 or 128 keys per running-max update)
 int forward_f8(const WorkU8& w, int64_t Sq, int64_t Sk, int64_t H, float scale, int tile, uint16_t* out, int64_t o_ss,
-               int64_t o_sh, hipStream_t st) {
+               int64_t o_sh, hipStream_t st, bool cleared = false) {
   U8Args f{w.q8, w.qs, w.k8, w.side, w.vt, w.vscale, w.vmean, out, o_ss, o_sh, Sq, Sk, padk(Sq), padk(Sk),
            scale * 1.4426950408889634f, 0, 0.0f};
-  const dim3 grid = claim_grid(f, w, Sq, H, st);  // sets f.nqb and f.ctr: before f is passed
+  const dim3 grid = claim_grid(f, w, Sq, H, st, cleared);  // sets f.nqb and f.ctr: before f is passed
   if (tile == 64) hipLaunchKernelGGL((attn_u8_kernel<2, 64>), grid, dim3(U8_NT), 0, st, f);
   else hipLaunchKernelGGL((attn_u8_kernel<2, 128>), grid, dim3(U8_NT), 0, st, f);
   return launch_status("attention_f8 forward");
 }
 
 int forward_u8(const WorkU8& w, int64_t Sq, int64_t Sk, int64_t H, float scale, int nbias, double bias, uint16_t* out,
-               int64_t o_ss, int64_t o_sh, hipStream_t st) {
+               int64_t o_ss, int64_t o_sh, hipStream_t st, bool cleared = false) {
   U8Args f{w.q8, w.qs, w.k8, w.side, w.vt, w.vscale, w.vmean, out, o_ss, o_sh, Sq, Sk, padk(Sq), padk(Sk),
            scale * 1.4426950408889634f, nbias, static_cast<float>(bias * 1.4426950408889634)};
-  const dim3 grid = claim_grid(f, w, Sq, H, st);  // sets f.nqb and f.ctr: before f is passed
+  const dim3 grid = claim_grid(f, w, Sq, H, st, cleared);  // sets f.nqb and f.ctr: before f is passed
   hipLaunchKernelGGL(attn_u8_kernel<0>, grid, dim3(U8_NT), 0, st, f);
   return launch_status("attention_u8 forward");
 }
@@ -851,32 +952,17 @@ int forward_u8(const WorkU8& w, int64_t Sq, int64_t Sk, int64_t H, float scale, 
 int prepass_bk(const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* k, int64_t k_ss, int64_t k_sh,
                const uint16_t* v, int64_t v_ss, int64_t v_sh, int64_t Sq, int64_t Sk, int64_t H, int smooth_k,
                int smooth_v, int rotate, const WorkU8& w, hipStream_t st) {
-  const int64_t sqp = padk(Sq), skp = padk(Sk);
-  const int nchunk = static_cast<int>((Sk + CHUNK - 1) / CHUNK);
   const RR none{nullptr, nullptr, 0.f, 0};
-  if (smooth_k) {
-    launch_stats(dim3(H, nchunk), st, k, k_ss, k_sh, Sk, none, w.kpart);
-    hipLaunchKernelGGL(kmean_kernel, dim3(H), dim3(KMEAN_NT), 0, st, w.kpart, nchunk, Sk, w.kmean);
-  } else {
-    hipLaunchKernelGGL(zero_kernel, dim3((H * D + 255) / 256), dim3(256), 0, st, w.kmean, H * D);
-  }
-  hipLaunchKernelGGL(vstats_kernel, dim3(H, nchunk), dim3(256), 0, st, v, v_ss, v_sh, Sk, w.vsum, w.vmax, w.vmin);
-  hipLaunchKernelGGL(vfinal_kernel, dim3(H), dim3(VFINAL_NT), 0, st, w.vsum, w.vmax, w.vmin, nchunk, Sk, smooth_v,
-                     w.vmean, w.vscale);
-  hipLaunchKernelGGL(tokq_kernel, dim3(sqp * H / 16), dim3(256), 0, st, q, q_ss, q_sh, Sq, sqp, H, none,
-                     static_cast<const float*>(nullptr), rotate, w.q8, w.qs, static_cast<float*>(nullptr));
-  hipLaunchKernelGGL(blockk_kernel, dim3(H, skp / TILE), dim3(256), 0, st, k, k_ss, k_sh, Sk, skp,
-                     static_cast<const float*>(w.kmean), rotate, w.k8, w.ks, reinterpret_cast<float*>(w.side));
-  hipLaunchKernelGGL(vq_kernel<false>, dim3(H, skp / TILE), dim3(256), 0, st, v, v_ss, v_sh, Sk, skp, w.vmean, w.vscale,
-                     w.vt, reinterpret_cast<int32_t*>(w.side));
-  return launch_status("attention_bk prepass");
+  PreU8 a{q, k, v, q_ss, q_sh, k_ss, k_sh, v_ss, v_sh, Sq, Sk, padk(Sq), padk(Sk), static_cast<int>(H),
+          static_cast<int>(attn_ws::nchunks(Sk)), smooth_k, smooth_v, rotate, none, none, w, 0, 0};
+  return prepass_all<false, true>(a, st, "attention_bk prepass");
 }
 
 int forward_bk(const WorkU8& w, int64_t Sq, int64_t Sk, int64_t H, float scale, uint16_t* out, int64_t o_ss,
-               int64_t o_sh, hipStream_t st) {
+               int64_t o_sh, hipStream_t st, bool cleared = false) {
   U8Args f{w.q8, w.qs, w.k8, w.side, w.vt, w.vscale, w.vmean, out, o_ss, o_sh, Sq, Sk, padk(Sq), padk(Sk),
            scale * 1.4426950408889634f, 0, 0.0f};
-  const dim3 grid = claim_grid(f, w, Sq, H, st);  // sets f.nqb and f.ctr: before f is passed
+  const dim3 grid = claim_grid(f, w, Sq, H, st, cleared);  // sets f.nqb and f.ctr: before f is passed
   hipLaunchKernelGGL(attn_u8_kernel<1>, grid, dim3(U8_NT), 0, st, f);
   return launch_status("attention_bk forward");
 }
@@ -970,22 +1056,9 @@ extern "C" int rh3_attention_u8_prepass_qkv(const uint16_t* k, int64_t k_ss, int
     rk = RR{tab, kw, eps, rot};
   }
   // q8, qs and the K / V channel statistics come from rh3_gemm_i8_qkv (numerics 1) on this workspace
-  const int64_t skp = padk(S);
-  const int nchunk = static_cast<int>((S + CHUNK - 1) / CHUNK);
-  const float* mean = nullptr;
-  if (smooth_k) {
-    hipLaunchKernelGGL(kmean_kernel, dim3(H), dim3(KMEAN_NT), 0, stream, w.kpart, nchunk, S, w.kmean);
-    mean = w.kmean;
-  } else {
-    hipLaunchKernelGGL(zero_kernel, dim3((H * D + 255) / 256), dim3(256), 0, stream, w.kmean, H * D);
-  }
-  hipLaunchKernelGGL(vfinal_kernel, dim3(H), dim3(VFINAL_NT), 0, stream, w.vsum, w.vmax, w.vmin, nchunk, S, smooth_v, w.vmean,
-                     w.vscale);
-  hipLaunchKernelGGL(tokq_kernel, dim3(skp * H / 16), dim3(256), 0, stream, k, k_ss, k_sh, S, skp, H, rk, mean, rotate,
-                     w.k8, w.ks, reinterpret_cast<float*>(w.side));
-  hipLaunchKernelGGL(vq_kernel<false>, dim3(H, skp / TILE), dim3(256), 0, stream, v, v_ss, v_sh, S, skp, w.vmean, w.vscale,
-                     w.vt, reinterpret_cast<int32_t*>(w.side));
-  if (int e = launch_status("attention_u8 prepass_qkv")) return e;
+  PreU8 a{nullptr, k, v, 0, 0, k_ss, k_sh, v_ss, v_sh, S, S, padk(S), padk(S), static_cast<int>(H),
+          static_cast<int>(attn_ws::nchunks(S)), smooth_k, smooth_v, rotate, rk, rk, w, 0, 0};
+  if (int e = prepass_tail<false, false>(a, stream, "attention_u8 prepass_qkv")) return e;
   ptrs[0] = w.q8; ptrs[1] = w.qs; ptrs[2] = w.k8; ptrs[3] = w.ks; ptrs[4] = w.side; ptrs[5] = w.vt;
   ptrs[6] = w.kmean; ptrs[7] = w.vscale; ptrs[8] = w.vmean;
   return RH3_OK;
@@ -1029,7 +1102,7 @@ extern "C" int rh3_int8_attention_u8(const uint16_t* q, int64_t q_ss, int64_t q_
   if (int e = prepass_u8(q, q_ss, q_sh, k, k_ss, k_sh, v, v_ss, v_sh, Sq, Sk, H, rq, rk, smooth_k, smooth_v, rotate,
                          w, stream))
     return e;
-  return forward_u8(w, Sq, Sk, H, scale, nbias, bias, out, o_ss, o_sh, stream);
+  return forward_u8(w, Sq, Sk, H, scale, nbias, bias, out, o_ss, o_sh, stream, true);
 }
 
 extern "C" int rh3_attention_bk_prepass(const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* k,
@@ -1076,7 +1149,7 @@ extern "C" int rh3_int8_attention_bk(const uint16_t* q, int64_t q_ss, int64_t q_
               (long long)w.bytes);
   if (int e = prepass_bk(q, q_ss, q_sh, k, k_ss, k_sh, v, v_ss, v_sh, Sq, Sk, H, smooth_k, smooth_v, rotate, w, stream))
     return e;
-  return forward_bk(w, Sq, Sk, H, scale, out, o_ss, o_sh, stream);
+  return forward_bk(w, Sq, Sk, H, scale, out, o_ss, o_sh, stream, true);
 }
 
 extern "C" int rh3_attention_f8_prepass(const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* k,
