@@ -9,6 +9,7 @@
 //                  bench/attn_emulate.py:10-18) -> codes [H][Spad][128] int8, scales [H][Spad/128]
 //   vt_kernel      V [S][H][128] bf16 -> Vt [H][128][Skpad] bf16, keys permuted inside 32-key groups
 //                  so that the P.V operand of each lane is one 16-byte LDS read
+//   pre_a_kernel, pre_b_kernel: the same parts in two launches for up to 4,096 keys
 // Main kernel: per (384-query block, head) workgroup of 12 waves, 32 queries per wave, 64-key steps.
 //   S^T = K8 . Q8^T on v_mfma_i32_32x32x32_i8 (keys on rows, queries on lanes), one fp32 dequant
 //   multiply per score c = qs[qblock] * ks[kblock] * scale * log2(e) (the 128x128 tile shares both

@@ -3,17 +3,17 @@
 // pre-pass), gfx950, head_dim 128, non-causal.
 //
 // Pre-pass (HBM-bound; attn_int8.cu:2568-2644):
-//   stats_kernel   float64 channel sums of K (after the optional RMSNorm + RoPE), per 256-token chunk
-//   vstats_kernel  float64 channel sums, max and min of V, per 256-token chunk
-//   kmean_kernel   kmean = fp32(sum / Sk)                                      (attn_int8.cu:97-109)
-//   vfinal_kernel  vmean = fp32(sum / Sk) (0 without smooth_v),
+//   stats_chunk    float64 channel sums of K (after the optional RMSNorm + RoPE), per 256-token chunk
+//   vstats_chunk   float64 channel sums, max and min of V, per 256-token chunk
+//   kmean_vfinal_kernel  kmean = fp32(sum / Sk) (attn_int8.cu:97-109), vmean = fp32(sum / Sk) (0 without smooth_v),
 //                  vscale = max(max(vmax - vmean, vmean - vmin), 1e-6) / 127  (attn_int8.cu:97-109)
-//   tokq_kernel    per (token, head) row: [RMSNorm + RoPE] -> [- kmean] -> [normalized H128] -> one scale
+//   tokq_rows      per (token, head) row: [RMSNorm + RoPE] -> [- kmean] -> [normalized H128] -> one scale
 //                  sc = max(amax, 1e-8) / 127, q = rint(x * (1 / sc))         (attn_int8.cu:113-170, :298-340);
 //                  for K also the per-key pair (sc, -1.5*2^23 * sc); padded keys get (0, -inf)
-//   vq_kernel      per (128-key tile, head): int8 V codes rint((v - vmean) / vscale) (attn_int8.cu:452-475),
+//   vq_tile        per (128-key tile, head): int8 V codes rint((v - vmean) / vscale) (attn_int8.cu:452-475),
 //                  transposed to [H][128][Skpad] in the key order of the P.V operand, and the tile's P.V
 //                  accumulator start 1.5*2^23 bits + 128 * (sum of its codes) per channel
+//   In three launches: pre_a_u8_kernel (both statistics and Q), kmean_vfinal_kernel, pre_b_u8_kernel (K and V).
 // Main kernel: per (128-query block, head) workgroup of 4 waves, 32 queries per wave, 128-key tiles.
 //   S^T = K8 . Q8^T on v_mfma_i32_32x32x32_i8 (keys on rows, queries on lanes), the accumulator starting at
 //   the bits of 1.5*2^23 so that t = fma(float bits, s_j, b_j) is the dequantized score in one instruction;
@@ -23,7 +23,7 @@
 //   reference's u8 x s8 product exactly); O = fma(ts, acc bits, fma(O, a, -ts * 1.5*2^23)); out =
 //   bf16(fma(O (1 / l), vscale, vmean)). Text bias (attn_cake.cuh:97-99, :210-240): t += bias*log2(e) / c on
 //   keys [0, nbias).
-// Configs 60-61 (attn_fwd6 :1786-1962): the same kernel with BK = true and blockk_kernel (quant_k_block :404-443)
+// Configs 60-61 (attn_fwd6 :1786-1962): the same kernel with BK = true and blockk_tile (quant_k_block :404-443)
 //   in place of the per-token K quantizer: one K scale per 128-key tile, integer tile max, no per-key dequant.
 #include "attn_common.hpp"
 #include "attn_layout.hpp"
@@ -496,7 +496,7 @@ typedef __attribute__((address_space(3))) const float lds_f32_u8;
 // (64 or 128, the reference's tile) the group max updates the running max m exactly (O and l scaled by
 // 2^((m_old - m) c) when it grows), P = 2^(fma(t, c, fma(-m, c, log2 448))) in e4m3 (v_cvt_pk_fp8_f32: OCP e4m3fn,
 // round to nearest even), l += P unquantized, and O^T += V^T . P^T on v_mfma_scale_f32_32x32x64_f8f6f4 (e4m3 V
-// from vq_kernel<true>) straight into the fp32 accumulators: no per-tile fold.
+// from vq_tile<true>) straight into the fp32 accumulators: no per-tile fold.
 template <int MODE, int MAXG = 128>
 __global__ void __launch_bounds__(U8_NT, 2) attn_u8_kernel(const U8Args a) {
   constexpr bool BK = MODE == 1;

@@ -63,6 +63,32 @@ def test_prepass_rope128_staged_k(dev, s, h):
     _check_prepass(pp, q8, qs, k8, ks, km, v, s)
 
 
+@pytest.mark.parametrize("sq,sk,h,rr,smooth", [
+    (1, 1, 17, False, True),         # one token, an odd number of heads
+    (130, 257, 3, False, True),      # cross lengths, a statistics chunk of one token
+    (300, 128, 2, False, False),     # no smoothing: kmean is 0
+    (4096, 4096, 1, True, True),     # the longest merged pre-pass (16 statistics chunks)
+    (4097, 4097, 1, True, True),     # one more: separate launches, K's rows staged
+    (129, 4097, 2, False, False)])
+def test_prepass_launch_forms(dev, sq, sk, h, rr, smooth):
+    """The per-block pre-pass in two launches (up to 4,096 keys) and in separate ones, on both sides of the line and
+    at ragged ends: codes, scales, kmean and the V^T layout bit-exact against the oracle."""
+    from rapid_h3 import attention
+    rng = np.random.default_rng(sq * 11 + sk * 3 + h)
+    q = _bf(rng.standard_normal((sq, h, 128)))
+    k = _bf(rng.standard_normal((sk, h, 128)) + 2.0 * rng.standard_normal((1, h, 128)))
+    v = _bf(rng.standard_normal((sk, h, 128)))
+    args, dargs = None, ()
+    if rr:
+        tab = _bf(oa.rope_table(np.arange(sq) % 97, rot=96).reshape(sq, 48, 2, 2))
+        qw, kw = (_bf(1.0 + 0.1 * rng.standard_normal(128)) for _ in range(2))
+        args = (tab, qw, kw, 1e-5)
+        dargs = (to_dev(tab, dev).view(1, sq, 1, 48, 2, 2), to_dev(qw, dev), to_dev(kw, dev), 1e-5)
+    pp = attention.prepass(*(to_dev(t, dev) for t in (q, k, v)), *dargs, smooth_k=smooth)
+    q8, qs, k8, ks, km = oa.prepass(q, k, rr=args, smooth_k=smooth)
+    _check_prepass(pp, q8, qs, k8, ks, km, v, sk)
+
+
 def test_attention_golden(dev, golden):
     from rapid_h3 import attention
     g = golden("attention")

@@ -61,6 +61,40 @@ def test_u8_prepass_golden(dev, golden):
     assert np.array_equal(to_np(pc["q8"]), g["q8"]) and np.array_equal(to_np(pc["qs"]), g["qs"])
 
 
+@pytest.mark.parametrize("sq,sk,h,rot,flags", [
+    (1, 1, 17, 0, (True, True, True)),           # one token, an odd number of heads
+    (130, 257, 3, 0, (False, True, True)),       # cross lengths, no K smoothing, a statistics chunk of one token
+    (64, 385, 2, 0, (True, False, False)),       # no V smoothing, no rotation
+    (767, 767, 5, 96, (True, True, True)),       # rows beside the 4-row groups of the per-token quantizer
+    (256, 256, 2, 128, (False, False, True))])
+def test_u8_prepass_merged(dev, sq, sk, h, rot, flags):
+    """The production pre-pass (parts merged into three launches), its per-block-K and e4m3-V forms: every operand
+    bit-exact against the oracle at ragged sizes and with each switch off. V has two channels of one sign, a constant
+    channel and one of zeros (the ends of its code range and an all-zero scale)."""
+    from rapid_h3 import attention
+    rng = np.random.default_rng(sq * 13 + sk + h)
+    q, k, v = (rng.standard_normal((n, h, 128)) for n in (sq, sk, sk))
+    k += 2.0 * rng.standard_normal((1, h, 128))
+    v[:, :, 0], v[:, :, 1] = np.abs(v[:, :, 0]) + 1.0, -np.abs(v[:, :, 1]) - 1.0
+    v[:, :, 2], v[:, :, 3] = 0.75, 0.0
+    q, k, v = (f32_to_bf16(t.astype(np.float32)) for t in (q, k, v))
+    args, dargs = None, ()
+    if rot:
+        tab = f32_to_bf16(oa.rope_table(np.arange(sq) % 97, rot=rot).reshape(sq, rot // 2, 2, 2))
+        qw, kw = (f32_to_bf16((1.0 + 0.1 * rng.standard_normal(128)).astype(np.float32)) for _ in range(2))
+        args = (tab, qw, kw, 1e-5)
+        dargs = (to_dev(tab, dev).view(1, sq, 1, rot // 2, 2, 2), to_dev(qw, dev), to_dev(kw, dev), 1e-5)
+    names = dict(zip(("smooth_k", "smooth_v", "rotate"), flags))
+    dq, dk, dv = (to_dev(t, dev) for t in (q, k, v))
+    exp = oa.prepass_u8(q, k, v, rr=args, **names)
+    _check_pp(attention.prepass_u8(dq, dk, dv, *dargs, **names), exp, "", sk)
+    if not rot:
+        _check_bk(attention.prepass_bk(dq, dk, dv, **names), oa.prepass_blockk(q, k, v, **names), "", sk)
+    pf, ef = attention.prepass_f8(dq, dk, dv, *dargs, **names), oa.prepass_fp8v(q, k, v, args, **names)
+    for n in ("q8", "qs", "k8", "ks", "ksb", "kmean", "vscale", "vmean"):
+        assert np.array_equal(to_np(pf[n]), ef[n]), n
+
+
 def test_ext_int8_prepass_golden(dev, golden):
     """attn_int8.ext().int8_prepass, the reference extension's verification entry (attn_int8.cu:2692-2704, called
     by _rr_check, __init__.py:342-343): the operand list [q8, qs, k8, ks, ksb, vt, vscale, vmean] bit-exact against
