@@ -23,10 +23,9 @@ def _check(xq, wq, dtype, name):
 
 
 def _vec(t, n, name):
-    t = t.reshape(-1)
     if t.numel() != n or t.dtype != torch.float32:
         raise RuntimeError(f"{name}: expected {n} fp32 values, got {t.numel()} {t.dtype}")
-    return t.contiguous()
+    return t if t.is_contiguous() else t.reshape(-1).contiguous()   # only its values in order are used
 
 
 def int8_gemm(xq, xs, wq, ws, bias=None, config=2):
