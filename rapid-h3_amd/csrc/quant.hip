@@ -352,7 +352,7 @@ __global__ void __launch_bounds__(64 * NM_WAVES) quant_normmod_lds_kernel(const 
   }
 }
 
-// Rows wider than 8192: same arithmetic, re-reading the row (from L2) instead of holding it.
+// Rows wider than the other forms take: same arithmetic, re-reading the row (from L2) instead of holding it.
 template <int KIND, bool FP8, typename TabT, bool VEC>
 __global__ void __launch_bounds__(256) quant_rows_wide_kernel(const QuantArgs a) {
   const int lane = threadIdx.x & 63;
@@ -434,35 +434,78 @@ void launch_vec(const QuantArgs& a, hipStream_t st) {
   else if (nch <= 4) hipLaunchKernelGGL((quant_rows_kernel<4, KIND, FP8, TabT, VEC>), grid, block, 0, st, a);
   else if (nch <= 6) hipLaunchKernelGGL((quant_rows_kernel<6, KIND, FP8, TabT, VEC>), grid, block, 0, st, a);
   else if (nch <= 8) hipLaunchKernelGGL((quant_rows_kernel<8, KIND, FP8, TabT, VEC>), grid, block, 0, st, a);
-  else if (nch <= 12) hipLaunchKernelGGL((quant_rows_kernel<12, KIND, FP8, TabT, VEC>), grid, block, 0, st, a);
-  else if (nch <= 16) hipLaunchKernelGGL((quant_rows_kernel<16, KIND, FP8, TabT, VEC>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((quant_rows_wide_kernel<KIND, FP8, TabT, VEC>), grid, block, 0, st, a);
+  else {
+    if constexpr (KIND == KIND_NORMMOD) {  // the others have a form of their own (launch)
+      if (nch <= 12) {
+        hipLaunchKernelGGL((quant_rows_kernel<12, KIND, FP8, TabT, VEC>), grid, block, 0, st, a);
+        return;
+      }
+      if (nch <= 16) {
+        hipLaunchKernelGGL((quant_rows_kernel<16, KIND, FP8, TabT, VEC>), grid, block, 0, st, a);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((quant_rows_wide_kernel<KIND, FP8, TabT, VEC>), grid, block, 0, st, a);
+  }
 }
 
-// Plain rows wider than 4096 columns: one workgroup per row, its 4 wavefronts taking every 4th 512-column
-// chunk (at most 8 each, so the row stays in 32 VGPRs per lane and occupancy stays high); the row absmax
-// goes through LDS. Same arithmetic as quant_rows_kernel<NCH, KIND_PLAIN, FP8> (max is order-free).
-template <int NCHW, bool FP8>
+// One workgroup per row (all but the norm's), its 4 wavefronts taking every 4th 512-column chunk (at most 8 each, so the
+// row stays in 32 VGPRs per lane, or 64 for SwiGLU's fp32 values); the row absmax goes through LDS. Same arithmetic as
+// quant_rows_kernel (max is order-free). A call of few rows is bound by the time one row takes (its loads, then 8 quotients
+// per chunk and lane in series), which this form divides by 4: us, one wavefront per row against this form: 512 x 3072 7.3 /
+// 4.3, 1,560 x 3072 8.5 / 5.7, 512 x 7168 heads 15.2 / 6.5, 512 x 8192 SwiGLU 18.8 / 8.2. A long call of wide rows gains from
+// the lower register count: 22,332 x 7168 heads 99 / 85, 22,332 x 8192 SwiGLU 224 / 150 (3.7 TB/s).
+template <int NCHW, int KIND, bool FP8>
 __global__ void __launch_bounds__(256) quant_rows_split_kernel(const QuantArgs a) {
+  constexpr bool RAW = KIND == KIND_PLAIN || KIND == KIND_HEADS;   // the bf16 words are kept; else the fp32 values
+  // the wavefronts' maxima joined per lane first: a NaN's magnitude bits then hide the same values of its row from the
+  // absmax (those of its lane) as with one wavefront per row
+  constexpr bool JOIN = KIND == KIND_HEADS || (KIND == KIND_PLAIN && NCHW <= 2);
+  __shared__ __attribute__((aligned(16))) uint32_t lmax[JOIN ? 64 : 1][4];
   __shared__ float wmax[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t m = blockIdx.x;
-  uint4 raw[NCHW];
+  uint4 raw[RAW ? NCHW : 1];
+  float v[RAW ? 1 : NCHW][8];
 #pragma unroll
   for (int i = 0; i < NCHW; ++i) {
     const int64_t c = 512 * (4 * i + wave) + 8 * lane;
-    raw[i] = c < a.K ? ld_stream16(a.x + m * a.ldx + c) : make_uint4(0, 0, 0, 0);
+    if constexpr (RAW) {
+      const uint16_t* p = KIND == KIND_HEADS ? a.x + (c >> 7) * a.ld_head + m * a.ldx + (c & 127) : a.x + m * a.ldx + c;
+      raw[i] = c < a.K ? ld_stream16(p) : make_uint4(0, 0, 0, 0);
+    } else if (c < a.K) {
+      load_chunk<KIND, true>(a, m, c, v[i]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[i][e] = 0.0f;
+    }
   }
-  uint32_t m2 = 0;  // on the raw bf16 words: magnitude bits, two per 32-bit lane
+  float amax = 0.0f;
+  uint32_t m2 = 0;  // RAW: on the raw bf16 words: magnitude bits, two per 32-bit lane
+  if constexpr (RAW) {
 #pragma unroll
-  for (int i = 0; i < NCHW; ++i) m2 = absmax8_bf16(m2, raw[i]);
-  float amax = wave_max(amax_of_pair(m2));
-  if (lane == 0) wmax[wave] = amax;
-  // the raw words are unpacked again below rather than kept as floats
+    for (int i = 0; i < NCHW; ++i) m2 = absmax8_bf16(m2, raw[i]);
+    amax = amax_of_pair(m2);
+  } else {
 #pragma unroll
-  for (int i = 0; i < NCHW; ++i) asm volatile("" : "+v"(raw[i].x), "+v"(raw[i].y), "+v"(raw[i].z), "+v"(raw[i].w));
+    for (int i = 0; i < NCHW; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) amax = max3_abs(amax, v[i][e], v[i][e + 1]);
+  }
+  if constexpr (JOIN) {
+    lmax[lane][wave] = m2;
+  } else {
+    amax = wave_max(amax);
+    if (lane == 0) wmax[wave] = amax;
+  }
+  if constexpr (RAW) {
+    // the raw words are unpacked again below rather than kept as floats
+#pragma unroll
+    for (int i = 0; i < NCHW; ++i) asm volatile("" : "+v"(raw[i].x), "+v"(raw[i].y), "+v"(raw[i].z), "+v"(raw[i].w));
+  }
   __syncthreads();
-  amax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+  if constexpr (JOIN) amax = wave_max(amax_of_pair(absmax8_bf16(0, *reinterpret_cast<const uint4*>(lmax[lane]))));
+  else amax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
   const float qmax = FP8 ? 448.0f : 127.0f;
   const float s = fmaxf(amax / qmax, 1e-12f);
   const float inv = 1.0f / s;
@@ -472,7 +515,12 @@ __global__ void __launch_bounds__(256) quant_rows_split_kernel(const QuantArgs a
     const int64_t c = 512 * (4 * i + wave) + 8 * lane;
     if (c >= a.K) continue;
     float x[8];
-    unpack8(raw[i], x);
+    if constexpr (RAW) {
+      unpack8(raw[i], x);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = v[i][e];
+    }
     uint2 out;
     if (FP8) {
       out = quant8_fp8(x, s, inv, fp8_odd_row(amax, s));
@@ -486,14 +534,30 @@ __global__ void __launch_bounds__(256) quant_rows_split_kernel(const QuantArgs a
 template <int KIND, bool FP8, typename TabT>
 int launch(const QuantArgs& a, hipStream_t st, const char* name) {
   if (a.M == 0) return RH3_OK;
-  if (KIND == KIND_PLAIN && a.K > 4096 && a.K <= 16384 && a.M < (1ll << 31)) {
-    const dim3 grid(static_cast<unsigned>(a.M)), block(256);
-    if (a.K <= 8192) hipLaunchKernelGGL((quant_rows_split_kernel<4, FP8>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((quant_rows_split_kernel<8, FP8>), grid, block, 0, st, a);
-    return launch_status(name);
+  if constexpr (KIND != KIND_NORMMOD) {
+    // The workgroup-per-row form for rows of more than 4096 columns, and for narrower ones in calls of up to 2 K rows: there
+    // its per-row costs (the barrier, and idle wavefronts where K is not 4 chunks' multiple) outweigh what it saves on a full
+    // chip. One wavefront / one workgroup per row (us, int8): 2,048 x 1024 4.0 / 4.0, 4,096 x 1024 5.0 / 5.5, 4,096 x 2048
+    // 8.1 / 7.4, 8,192 x 2048 12.2 / 12.2, 4,096 x 3072 11.3 / 10.0, 16,384 x 3072 29.0 / 29.8, 145,152 x 3072 214 / 224.
+    // SwiGLU the same (1,560 x 1024 4.8 / 4.7, 11,000 x 3072 32.7 / 33.1). Plain rows of 8 chunks: always (16,384 x 4096 38.8 /
+    // 35.3; head-major rows 72,216 x 4096 145 / 149). Up to 8,192 columns (plain: 16,384), past which a row is read twice. A
+    // grid of 2^24 workgroups of 256 would pass 2^32 threads.
+    const bool wide = a.K > (KIND == KIND_PLAIN ? 3584 : 4096);
+    if (a.K > 512 && a.K <= (KIND == KIND_PLAIN ? 16384 : 8192) && a.M < (1ll << 24) && (wide || a.M <= 2 * a.K)) {
+      const dim3 grid(static_cast<unsigned>(a.M)), block(256);
+      if (a.K <= 2048) hipLaunchKernelGGL((quant_rows_split_kernel<1, KIND, FP8>), grid, block, 0, st, a);
+      else if (a.K <= 4096) hipLaunchKernelGGL((quant_rows_split_kernel<2, KIND, FP8>), grid, block, 0, st, a);
+      else if (a.K <= 8192) hipLaunchKernelGGL((quant_rows_split_kernel<4, KIND, FP8>), grid, block, 0, st, a);
+      else if constexpr (KIND == KIND_PLAIN) hipLaunchKernelGGL((quant_rows_split_kernel<8, KIND, FP8>), grid, block, 0, st, a);
+      return launch_status(name);
+    }
   }
   // up to 6144 columns the staged table and weight rows fit in 72 KB of LDS
-  if (KIND == KIND_NORMMOD && !FP8 && a.K <= 6144 && a.K % 8 == 0) {
+  // (long calls: a workgroup of 16 rows first copies its table rows, 9 us of which a short call hides nothing; us, one wavefront
+  // per row against this kernel, fp32 tables: 512 x 3072 8.5 / 13.2, 4,096 x 3072 13.2 / 15.3, 5,583 x 3072 21.0 / 17.4, 8,192 x
+  // 1024 9.1 / 10.1, 11,000 x 1024 11.7 / 11.3, 2,816 x 4096 14.1 / 17.4, 2,816 x 5376 18.7 / 22.4, 4,096 x 5376 30.0 / 23.8)
+  const bool shortcall = a.M <= 8192 && a.M * a.K <= (12 << 20);
+  if (KIND == KIND_NORMMOD && !FP8 && a.K <= 6144 && a.K % 8 == 0 && !shortcall) {
     const dim3 grid(static_cast<unsigned>((a.M + NM_WAVES * NM_RPW - 1) / (NM_WAVES * NM_RPW))), block(64 * NM_WAVES);
     const size_t lds = static_cast<size_t>(a.K) * (4 + 4 + 4);
     const int64_t nch = (a.K + 511) / 512;

@@ -5,7 +5,7 @@ import pytest
 
 from conftest import to_dev, to_np
 from oracle import quant as oq
-from oracle.numerics import f32_to_bf16
+from oracle.numerics import bf16_to_f32, f32_to_bf16
 
 pytestmark = pytest.mark.gpu
 
@@ -41,6 +41,51 @@ def test_quant_rows_shapes(dev, m, k):
         eq, es = oq.quantize_rows(x, "fp8_rowwise" if fp8 else "int8_rowwise")
         assert np.array_equal(to_np(q), eq), (m, k, fp8)
         assert np.array_equal(to_np(s), es), (m, k, fp8)
+
+
+@pytest.mark.parametrize("m,k", [
+    (1040, 520), (1041, 520),      # both sides of M = 2 K, a second chunk of one lane
+    (3, 512),                      # one chunk: one wavefront per row
+    (5, 2048), (5, 2056), (2, 3584), (9000, 3592),
+    (3, 4096), (3, 4104), (2, 8192), (2, 8320), (2, 16384), (2, 16392)])
+def test_rows_per_workgroup_forms(dev, m, k):
+    """Plain, head-gathered and SwiGLU rows on one wavefront or one workgroup per row, on both sides of each line of that
+    choice and with idle wavefronts: plain and heads bit-exact against the oracle (a sample of rows where there are
+    many); SwiGLU within one code (its sigmoid), its scale within the few units of the fp32 sigmoid."""
+    from rapid_h3 import quant
+    rng = np.random.default_rng(m * 7 + k)
+    rows = np.unique(np.r_[0, m - 1, rng.integers(0, m, min(m, 60))])
+    x = _bf(rng.standard_normal((m, k)) * np.exp(rng.standard_normal((1, k))))
+    for fp8 in (False, True):
+        q, s = _quant(to_dev(x, dev), fp8)
+        eq, es = oq.quantize_rows(x[rows], "fp8_rowwise" if fp8 else "int8_rowwise")
+        assert np.array_equal(to_np(q)[rows], eq) and np.array_equal(to_np(s)[rows], es), fp8
+    if k % 128 == 0 and k <= 16384:
+        o = np.ascontiguousarray(x.reshape(m, k // 128, 128).transpose(1, 0, 2))
+        q, s = quant.heads_quant_rows_i8(to_dev(o, dev))
+        eq, es = oq.quantize_rows(x[rows], "int8_rowwise")
+        assert np.array_equal(to_np(q)[rows], eq) and np.array_equal(to_np(s)[rows], es)
+    gu = _bf(rng.standard_normal((m, 2 * k)))
+    q, s = quant.swiglu_quant_rows_i8(to_dev(gu, dev))
+    h = oq.silu_mul(*(bf16_to_f32(gu[rows][:, i * k:(i + 1) * k]) for i in (0, 1)))
+    eq, es = oq.quantize_rows(h, "int8_rowwise")
+    assert np.abs(to_np(q)[rows].astype(int) - eq).max() <= 1
+    assert np.allclose(to_np(s)[rows], es, rtol=1e-5)
+
+
+@pytest.mark.parametrize("m,k", [(8192, 1024), (8193, 1024), (4096, 3072), (4097, 3072)])
+def test_norm_mod_forms(dev, m, k):
+    """The norm + modulation quantizer on both sides of the line between one wavefront per row and staged table rows:
+    bit-exact against the oracle on a sample of rows."""
+    from rapid_h3 import quant
+    rng = np.random.default_rng(m + k)
+    rows = np.unique(np.r_[0, 16, 17, m - 1, rng.integers(0, m, 60)])
+    x, w = _bf(rng.standard_normal((m, k))), _bf(1.0 + 0.1 * rng.standard_normal(k))
+    idx = (np.arange(m) >= 17).astype(np.int32)
+    sh, sc = (0.3 * rng.standard_normal((2, k)).astype(np.float32) for _ in range(2))
+    q, s = quant.norm_mod_quant_rows_i8(*(to_dev(t, dev) for t in (x, w)), 1e-6, *(to_dev(t, dev) for t in (idx, sh, sc)))
+    eq, es = oq.norm_mod_quant_rows_i8(x[rows], w, 1e-6, idx[rows], sh, sc)
+    assert np.array_equal(to_np(q)[rows], eq) and np.array_equal(to_np(s)[rows], es)
 
 
 @pytest.mark.parametrize("k", [8, 3072, 8192])
