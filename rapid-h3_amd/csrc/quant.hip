@@ -83,11 +83,15 @@ __device__ __forceinline__ uint32_t fp8_e4m3(float t) {
 // correctly rounded quotient (inv = 1 / s is the correctly rounded reciprocal and no intermediate leaves the normal range
 // where the code depends on it: |x / s| >= 2^-11 with s in [2^-60, 2^60]); the hardware conversion rounds to nearest even.
 // The residual is taken as t s - x, which keeps the sign of a zero.
-// odd: the row's scale is outside that range or its absmax not finite; those rows take the division and the software
-// encoder. With those for every value the kernel ran at 3.5 TB/s, bound by VALU: 145,152 x 3072 387 -> 212 us, the int8 form's time. (A vote on
-// x * inv being near a rounding boundary, as in quant8_i8, does not pay: the quotients of two 8-bit significands are
-// exactly on one so often that two in five votes fail, 422 us.)
-__device__ __forceinline__ bool fp8_odd_row(float amax, float s) { return !(amax < INFINITY && s >= 0x1p-60f && s <= 0x1p60f); }
+// odd: the row's scale is outside that range, its absmax not finite, or the lane holds a NaN, whose magnitude bits may hide
+// infinities and values past 448 s from the absmax; those take the division and the software encoder. With those for every
+// value the kernel ran at 3.5 TB/s, bound by VALU: 145,152 x 3072 387 -> 212 us, the int8 form's time. (A vote on x * inv
+// being near a rounding boundary, as in quant8_i8, does not pay: the quotients of two 8-bit significands are exactly on one
+// so often that two in five votes fail, 422 us.)
+// lane_amax: the absmax of the lane's values, NaN if it holds one
+__device__ __forceinline__ bool fp8_odd(float amax, float lane_amax, float s) {
+  return !(lane_amax <= amax && amax < INFINITY && s >= 0x1p-60f && s <= 0x1p60f);
+}
 __device__ __forceinline__ uint2 quant8_fp8(const float* x, float s, float inv, bool odd) {
   if (odd) {
     uint32_t b[8];
@@ -207,6 +211,7 @@ __global__ void __launch_bounds__(256) quant_rows_kernel(const QuantArgs a) {
 #pragma unroll
       for (int e = 0; e < 8; e += 2) amax = max3_abs(amax, v[j][e], v[j][e + 1]);
   }
+  const float lane_amax = amax;
   amax = wave_max(amax);
   if (RAW) {
     // the raw words are unpacked again below rather than kept as floats (the empty asm hides the first
@@ -226,7 +231,7 @@ __global__ void __launch_bounds__(256) quant_rows_kernel(const QuantArgs a) {
     vals(j, x);
     uint2 out;
     if (FP8) {
-      out = quant8_fp8(x, s, inv, fp8_odd_row(amax, s));
+      out = quant8_fp8(x, s, inv, fp8_odd(amax, lane_amax, s));
     } else {
       out = quant8_i8(x, s, inv);
     }
@@ -492,6 +497,7 @@ __global__ void __launch_bounds__(256) quant_rows_split_kernel(const QuantArgs a
 #pragma unroll
       for (int e = 0; e < 8; e += 2) amax = max3_abs(amax, v[i][e], v[i][e + 1]);
   }
+  float lane_amax = amax;
   if constexpr (JOIN) {
     lmax[lane][wave] = m2;
   } else {
@@ -504,8 +510,10 @@ __global__ void __launch_bounds__(256) quant_rows_split_kernel(const QuantArgs a
     for (int i = 0; i < NCHW; ++i) asm volatile("" : "+v"(raw[i].x), "+v"(raw[i].y), "+v"(raw[i].z), "+v"(raw[i].w));
   }
   __syncthreads();
-  if constexpr (JOIN) amax = wave_max(amax_of_pair(absmax8_bf16(0, *reinterpret_cast<const uint4*>(lmax[lane]))));
-  else amax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+  if constexpr (JOIN) {
+    lane_amax = amax_of_pair(absmax8_bf16(0, *reinterpret_cast<const uint4*>(lmax[lane])));
+    amax = wave_max(lane_amax);
+  } else amax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
   const float qmax = FP8 ? 448.0f : 127.0f;
   const float s = fmaxf(amax / qmax, 1e-12f);
   const float inv = 1.0f / s;
@@ -523,7 +531,7 @@ __global__ void __launch_bounds__(256) quant_rows_split_kernel(const QuantArgs a
     }
     uint2 out;
     if (FP8) {
-      out = quant8_fp8(x, s, inv, fp8_odd_row(amax, s));
+      out = quant8_fp8(x, s, inv, fp8_odd(amax, lane_amax, s));
     } else {
       out = quant8_i8(x, s, inv);
     }

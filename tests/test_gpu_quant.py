@@ -5,7 +5,7 @@ import pytest
 
 from conftest import to_dev, to_np
 from oracle import quant as oq
-from oracle.numerics import bf16_to_f32, f32_to_bf16
+from oracle.numerics import bf16_to_f32, f32_to_bf16, f32_to_fp8_e4m3
 
 pytestmark = pytest.mark.gpu
 
@@ -110,6 +110,29 @@ def test_quant_fp8_quotients(dev, k):
     q = to_np(q)
     assert (q[135, 3], q[136, 3], q[137, 3]) == (0xFE, 0xFE, 0xFE) and (q[138] == 0xFE).all()
     assert np.isinf(to_np(s)[135:137]).all() and (np.delete(q[135], 3) & 0x7F == 0).all()
+
+
+@pytest.mark.parametrize("m,k", [(3, 64), (1100, 520), (3, 1536), (3, 4096), (3, 8192), (3, 16384), (3, 16392)])
+def test_quant_fp8_values_behind_a_nan(dev, m, k):
+    """A NaN's magnitude bits hide the other values of its lane from the row absmax, so infinities and values past 448
+    scales can meet a finite scale: their codes are still those of the clamped IEEE quotient (+-448), in every form (one
+    wavefront per row, one workgroup per row with joined and with separate lanes, rows read twice)."""
+    rng = np.random.default_rng(m + k)
+    x = _bf(rng.standard_normal((m, k)))
+    lane = 8 * 5                                   # the chunk of lane 5; 512 columns on lie the same lane's next chunks
+    x[1, lane] = 0x7FC0                            # NaN
+    x[1, lane + 1:lane + 6] = _bf([np.inf, -np.inf, 3e38, -3e38, 5e3])
+    if k > 1024:                                   # the lane's next chunk: another wavefront's where lanes are joined
+        c = lane + (512 if k <= 4096 else 2048)
+        x[1, c:c + 2] = _bf([-np.inf, 3e38])
+    x[2, 1] = 0xFFC1                               # a NaN with nothing to hide
+    q, s = (to_np(t) for t in _quant(to_dev(x, dev), fp8=True))
+    hidden = k <= 16384                            # the form that reads rows twice skips a NaN alone
+    assert np.isfinite(s[[0, 2]]).all() and np.isfinite(s[1, 0]) == hidden
+    with np.errstate(invalid="ignore", over="ignore"):
+        t = bf16_to_f32(x) / s
+    want = f32_to_fp8_e4m3(np.fmin(np.fmax(t, np.float32(-448)), np.float32(448)))   # a NaN quotient: -448
+    assert np.array_equal(q, want)
 
 
 def test_quant_rows_strided(dev):
