@@ -345,7 +345,19 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, const int bid, int8_t
       if (q >= a.Sq) raw[i] = make_uint4(0, 0, 0, 0);
       m2 = absmax8_bf16(m2, raw[i]);
     }
-    const float am = wave_max(amax_of_pair(m2));
+    float am = amax_of_pair(m2);
+    // a NaN's magnitude bits hide the lane's other values; quant_block's maximum skips the NaN alone
+    if (__builtin_amdgcn_ballot_w64(!(am <= INFINITY)) != 0) {
+      am = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float v[8];
+        unpack8(raw[i], v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(v[e]));
+      }
+    }
+    am = wave_max(am);
     if (lane == 0) wmax[wave] = am;
     __syncthreads();
     const float bm = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));

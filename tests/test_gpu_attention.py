@@ -172,6 +172,27 @@ def test_attention_query_kernels_agree(dev):
     assert torch.equal(attention.attention(q[:1024], k, v), whole[:1024])
 
 
+@pytest.mark.parametrize("sq,sk,h", [(130, 65, 2), (9000, 129, 24)])
+def test_attention_nan_queries(dev, sq, sk, h):
+    """NaNs in queries whose other channels hold their block's largest value, and infinities: the one call (its main
+    kernel quantizes the queries) and the split pair (its pre-pass does) agree bit for bit, and the scale skips the NaN
+    alone: a NaN counts as a zero there, so the other rows of its block are those of the same queries with a zero."""
+    import torch
+    from rapid_h3 import attention
+    g = torch.Generator().manual_seed(sq)
+    q, k, v = (torch.randn(n, h, 128, generator=g).to(torch.bfloat16) for n in (sq, sk, sk))
+    q[3, 0, 33], q[3, 0, 40] = float("nan"), 60.0            # channels 32-47, 64-79, ... of a query share a lane
+    q[129, 1, 0], q[129, 1, 100] = float("nan"), -80.0
+    zero = q.nan_to_num(nan=0.0)
+    if sq > 256:
+        q[200, 1, 7] = zero[200, 1, 7] = float("inf")
+    kt, vt = k.to(dev), v.to(dev)
+    out = attention.attention(q.to(dev), kt, vt)
+    pair = attention.forward(attention.prepass(q.to(dev), kt, vt), sq)
+    assert torch.equal(out.view(torch.int16), pair.view(torch.int16))
+    assert torch.equal(out.view(torch.int16), attention.attention(zero.to(dev), kt, vt).view(torch.int16))
+
+
 def test_attention_strided_out(dev):
     """q/k/v as views of one [S, 3*H*128] qkv buffer; output into a head-major [1, H, S, D] buffer
     through out=o[0].transpose(0, 1) (the _fused_block call, __init__.py:283-291)."""
