@@ -291,6 +291,13 @@ int rh3_attention_forward(int64_t Sq, int64_t Sk, int64_t H, float scale,
                           uint16_t* out, int64_t o_ss, int64_t o_sh,
                           void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
+/* Verification: how the per-block attention runs a call, by the rule its entry points apply (no device access but
+ * the CU count where cus is 0). raw 1: the one call without RMSNorm + RoPE, whose main kernel may quantize the
+ * queries itself; tail 0: rh3_int8_attention_noalloc, which has no room for split partials. RH3_ATTN_SPLIT is read.
+ * plan[0] queries per workgroup (128 or 384), plan[1] 1 when the main kernel quantizes the queries, plan[2] the
+ * 384-query workgroups that run as two key halves. No counterpart in the reference. */
+int rh3_attention_plan(int64_t Sq, int64_t Sk, int64_t H, int raw, int tail, int cus, int64_t* plan /* [3] */);
+
 /* ---------------------------------------------------------------------------------------------
  * INT8 flash attention with the reference's production numerics (attn_int8.cu configs 80-99: attn_fwd8
  * :2250-2511, and the cake configs 90/94 that are bit-identical to it; configs 1xx add the q/k RMSNorm +

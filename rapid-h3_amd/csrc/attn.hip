@@ -789,24 +789,49 @@ int prepass(const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* k, in
 // kernel (us, 384 / 128 queries): 1,024 tokens x 24 heads 39 / 20, 1,560 x 24 54 / 39, 2,816 x 24 86 / 92, 4,096 x 24
 // 186 / 148, 5,583 x 24 290 / 301, 1,560 x 56 92 / 61, 72,216 queries x 512 keys x 24 heads 502 / 402 (qf: it also quantizes
 // the queries itself, which the pre-pass takes 180 us for there), 11,000 x 24 986 / 1,052.
-bool use_small(int64_t Sq, int64_t Sk, int64_t H, bool qf) {
-  const int64_t cus = device_cus();
+// npair: the items of the 384-query grid that would run as two key halves; where they cannot, the half-empty last round
+// costs a whole one (us, 384 / 128 queries, unsplit: 5,583 x 24 325 / 308, 2,600 queries x 5,583 keys x 49 313 / 302).
+bool use_small(int64_t Sq, int64_t Sk, int64_t H, bool qf, int64_t npair, int64_t cus) {
   if (cus <= 0 || pad(Sk) / BLK > SM_KB) return false;
   const double n = static_cast<double>((Sk + STEP - 1) / STEP);
   const int64_t big = (Sq + FWD_BQ - 1) / FWD_BQ * H, small = (Sq + SM_BQ - 1) / SM_BQ * H;
   if (small >= (int64_t{1} << 31)) return false;
   const int64_t bf = big / cus, br = big % cus, sf = small / (3 * cus), sr = (small % (3 * cus) + cus - 1) / cus;
   double tb = static_cast<double>(bf) * (12 + 2.0 * n);
-  if (br > 0) tb += bf == 0 ? 10 + 1.75 * n : 2 * br <= cus && n >= 8 ? 10 + n : 12 + 2.0 * n;
+  if (br > 0) tb += bf == 0 ? 10 + 1.75 * n : npair > 0 ? 10 + n : 12 + 2.0 * n;
   if (qf) tb += 6 + static_cast<double>(Sq * H) * (180.0 / (72216.0 * 24.0));   // the pre-pass over the queries
   const double part[4] = {0, 6 + 0.95 * n, 6 + 1.42 * n, 6 + 2.05 * n};
   const double ts = static_cast<double>(sf) * (8 + 2.15 * n) + part[sr];
   return ts < tb;
 }
 
+// How a call runs: small on the 128-query kernel (raw: which also quantizes the queries), else npair items of the
+// 384-query grid as two key halves
+struct FwdPlan {
+  bool small, raw;
+  int npair;
+};
+
+// raw: the main kernel may read the raw queries; tail: the workspace holds the split partials
+FwdPlan plan_forward(int64_t Sq, int64_t Sk, int64_t H, bool raw, bool tail, int64_t cus) {
+  // One workgroup per CU: the 384-query grid runs in rounds of `cus` workgroups. When the last round is at most half
+  // full, its workgroups run as two key halves each (a round half as long) and a merge kernel combines them.
+  // The split changes how a split workgroup's keys are summed (two fp32 halves merged), so a head's output can
+  // differ in the last bits with the grid (H, Sq, the CU count). RH3_ATTN_SPLIT=0 turns it off for callers that
+  // need the same bits on every grid.
+  const char* env = getenv("RH3_ATTN_SPLIT");
+  const bool split_ok = tail && !(env && env[0] == '0');
+  const int64_t nwg = attn_ws::fwd_blocks(Sq, H), last = cus > 0 ? nwg % cus : 0;
+  const int64_t nsteps = (Sk + STEP - 1) / STEP;
+  const int npair = split_ok && nwg > cus && last > 0 && 2 * last <= cus && last <= attn_ws::TAIL_MAX && nsteps >= 8
+                        ? static_cast<int>(last) : 0;
+  const bool small = use_small(Sq, Sk, H, raw, npair, cus);
+  return {small, small && raw, small ? 0 : npair};
+}
+
 // one-call attention without RMSNorm + RoPE: hand the raw queries to the 128-query kernel where it runs
 void raw_queries(Work& w, const uint16_t* q, int64_t q_ss, int64_t q_sh, int64_t Sq, int64_t Sk, int64_t H) {
-  if (!use_small(Sq, Sk, H, true)) return;
+  if (!plan_forward(Sq, Sk, H, true, w.tail != nullptr, device_cus()).raw) return;
   w.rawq = q;
   w.rq_ss = q_ss;
   w.rq_sh = q_sh;
@@ -814,7 +839,8 @@ void raw_queries(Work& w, const uint16_t* q, int64_t q_ss, int64_t q_sh, int64_t
 
 int forward(const Work& w, int64_t Sq, int64_t Sk, int64_t H, float scale, uint16_t* out, int64_t o_ss,
             int64_t o_sh, hipStream_t st) {
-  if (use_small(Sq, Sk, H, w.rawq != nullptr)) {
+  const FwdPlan plan = plan_forward(Sq, Sk, H, w.rawq != nullptr, w.tail != nullptr, device_cus());
+  if (plan.small || w.rawq) {   // raw queries were left unquantized for this kernel
     const int nqb = static_cast<int>((Sq + SM_BQ - 1) / SM_BQ);
     const FwdArgs f{w.q8, w.qs, w.k8, w.ks, w.kn, w.vt, out, o_ss, o_sh, Sq, Sk, pad(Sq), pad(Sk),
                     scale * 1.4426950408889634f, nqb, 0, 0, nullptr, nullptr, w.rawq, w.rq_ss, w.rq_sh};
@@ -827,19 +853,7 @@ int forward(const Work& w, int64_t Sq, int64_t Sk, int64_t H, float scale, uint1
   RH3_REQUIRE(nwg < (int64_t{1} << 30) / FWD_NT, "attention forward: %lld workgroups exceed the grid limit",
               (long long)nwg);
   const int nqb = static_cast<int>((Sq + FWD_BQ - 1) / FWD_BQ);
-  // One workgroup per CU: the grid runs in rounds of `cus` workgroups. When the last round is at most half
-  // full, its workgroups run as two key halves each (a round half as long) and a merge kernel combines them.
-  const int cus = device_cus();
-  const int64_t last = cus > 0 ? nwg % cus : 0;
-  const int64_t nsteps = (Sk + STEP - 1) / STEP;
-  // The split changes how a split workgroup's keys are summed (two fp32 halves merged), so a head's output can
-  // differ in the last bits with the grid (H, Sq, the CU count). RH3_ATTN_SPLIT=0 turns it off for callers that
-  // need the same bits on every grid.
-  const char* env = getenv("RH3_ATTN_SPLIT");
-  const bool split_ok = !(env && env[0] == '0');
-  const int npair = split_ok && w.tail && nwg > cus && last > 0 && 2 * last <= cus && last <= attn_ws::TAIL_MAX &&
-                            nsteps >= 8
-                        ? static_cast<int>(last) : 0;
+  const int npair = plan.npair;
   const int nmain = static_cast<int>(nwg - npair);
   const FwdArgs f{w.q8, w.qs, w.k8, w.ks, w.kn, w.vt, out, o_ss, o_sh, Sq, Sk, pad(Sq), pad(Sk),
                   scale * 1.4426950408889634f, nqb, nmain, npair, w.tail, w.ctr};
@@ -957,6 +971,16 @@ extern "C" int rh3_int8_attention_noalloc(const uint16_t* q, int64_t q_ss, int64
   if (int e = prepass(q, q_ss, q_sh, k, k_ss, k_sh, v, v_ss, v_sh, Sq, Sk, H, none, none, smooth_k, w, stream))
     return e;
   return forward(w, Sq, Sk, H, scale, out, o_ss, o_sh, stream);
+}
+
+extern "C" int rh3_attention_plan(int64_t Sq, int64_t Sk, int64_t H, int raw, int tail, int cus, int64_t* plan) {
+  clear_error();
+  RH3_REQUIRE(Sq > 0 && Sk > 0 && H > 0 && cus >= 0 && plan, "attention_plan: sizes must be positive, plan set");
+  const FwdPlan p = plan_forward(Sq, Sk, H, raw != 0, tail != 0 && attn_ws::has_tail(Sq, H), cus > 0 ? cus : device_cus());
+  plan[0] = p.small ? SM_BQ : FWD_BQ;
+  plan[1] = p.raw;
+  plan[2] = p.npair;
+  return RH3_OK;
 }
 
 extern "C" int64_t rh3_attention_workspace_bytes(int64_t Sq, int64_t Sk, int64_t H) {

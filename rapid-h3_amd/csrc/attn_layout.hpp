@@ -26,6 +26,10 @@ constexpr int TAIL_ROW = D + 4; // floats per query of a split partial: O[128], 
 // (head, query block) workgroups of the main kernel
 __host__ __device__ inline int64_t fwd_blocks(int64_t Sq, int64_t H) { return (Sq + FWD_BQ - 1) / FWD_BQ * H; }
 
+// whether the workspace reserves the split partials: only a grid larger than TAIL_MAX workgroups can leave a last round
+// worth splitting
+__host__ __device__ inline bool has_tail(int64_t Sq, int64_t H) { return fwd_blocks(Sq, H) > TAIL_MAX; }
+
 struct Work {
   int8_t* q8; float* qs; int8_t* k8; float* ks; float* kmean; double* part; uint16_t* vt;
   float* kn;    // [H][Skpad/128]: per 128-key block, an upper bound of the largest L2 norm of a key's int8 codes
@@ -52,10 +56,8 @@ inline Work layout(void* base, int64_t Sq, int64_t Sk, int64_t H, bool split = t
   w.part = reinterpret_cast<double*>(take(H * nchunk * D * 8));
   w.vt = reinterpret_cast<uint16_t*>(take(H * D * skp * 2));
   w.kn = reinterpret_cast<float*>(take(H * (skp / BLK) * 4));
-  // only a grid larger than TAIL_MAX workgroups can leave a last round worth splitting
-  const int64_t nwg = fwd_blocks(Sq, H);
-  w.tail = split && nwg > TAIL_MAX ? reinterpret_cast<float*>(take(int64_t{2} * TAIL_MAX * FWD_BQ * TAIL_ROW * 4))
-                                   : nullptr;
+  w.tail = split && has_tail(Sq, H) ? reinterpret_cast<float*>(take(int64_t{2} * TAIL_MAX * FWD_BQ * TAIL_ROW * 4))
+                                    : nullptr;
   w.ctr = reinterpret_cast<int*>(take(256));
   w.bytes = off;
   return w;
