@@ -208,7 +208,9 @@ int rh3_gemm_fp8_acc(const uint8_t* xq, int64_t ldx, const uint8_t* wq, int64_t 
  * INT8 flash attention, head_dim 128, non-causal. q [Sq, H, 128], k and v [Sk, H, 128] bf16 with any
  * token / head strides (elements; the 128 channels contiguous). Q and K are quantized per
  * (head, 128-token block); K is first mean-smoothed (kmean over all Sk tokens); Q.K^T runs on int8
- * MFMA, softmax in fp32 (exp2 domain), P.V on bf16 MFMA. out [Sq, H, 128] bf16 with its own strides.
+ * MFMA, softmax in fp32 (exp2 domain), P.V on bf16 MFMA. out [Sq, H, 128] bf16 with its own strides. out may share
+ * storage with q, k or v in any layout (here and in the numerics below): every operand has been read before a row of
+ * out that overlaps it is written.
  * ------------------------------------------------------------------------------------------- */
 
 /* Bytes of workspace the attention entry points need for (Sq, Sk, H). */
@@ -292,11 +294,14 @@ int rh3_attention_forward(int64_t Sq, int64_t Sk, int64_t H, float scale,
                           void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
 /* Verification: how the per-block attention runs a call, by the rule its entry points apply (no device access but
- * the CU count where cus is 0). raw 1: the one call without RMSNorm + RoPE, whose main kernel may quantize the
- * queries itself; tail 0: rh3_int8_attention_noalloc, which has no room for split partials. RH3_ATTN_SPLIT is read.
- * plan[0] queries per workgroup (128 or 384), plan[1] 1 when the main kernel quantizes the queries, plan[2] the
- * 384-query workgroups that run as two key halves. No counterpart in the reference. */
-int rh3_attention_plan(int64_t Sq, int64_t Sk, int64_t H, int raw, int tail, int cus, int64_t* plan /* [3] */);
+ * the CU count where cus is 0). q, out: the operands of the one call without RMSNorm + RoPE, whose main kernel may
+ * quantize the queries itself (only their addresses are used); q NULL: any other call. tail 0:
+ * rh3_int8_attention_noalloc, which has no room for split partials. RH3_ATTN_SPLIT is read. plan[0] queries per
+ * workgroup (128 or 384), plan[1] 1 when the main kernel quantizes the queries, plan[2] the 384-query workgroups
+ * that run as two key halves. No counterpart in the reference. */
+int rh3_attention_plan(const uint16_t* q, int64_t q_ss, int64_t q_sh,
+                       const uint16_t* out, int64_t o_ss, int64_t o_sh,
+                       int64_t Sq, int64_t Sk, int64_t H, int tail, int cus, int64_t* plan /* [3] */);
 
 /* ---------------------------------------------------------------------------------------------
  * INT8 flash attention with the reference's production numerics (attn_int8.cu configs 80-99: attn_fwd8

@@ -829,9 +829,26 @@ FwdPlan plan_forward(int64_t Sq, int64_t Sk, int64_t H, bool raw, bool tail, int
   return {small, small && raw, small ? 0 : npair};
 }
 
-// one-call attention without RMSNorm + RoPE: hand the raw queries to the 128-query kernel where it runs
-void raw_queries(Work& w, const uint16_t* q, int64_t q_ss, int64_t q_sh, int64_t Sq, int64_t Sk, int64_t H) {
-  if (!plan_forward(Sq, Sk, H, true, w.tail != nullptr, device_cus()).raw) return;
+// Whether out [Sq, H, 128] may be written while other workgroups still read q: it lies clear of q (by the ranges their rows
+// span), or is q itself in q's layout (a workgroup reads its own rows before it writes them)
+bool out_clear_of(const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* out, int64_t o_ss, int64_t o_sh, int64_t Sq,
+                  int64_t H) {
+  if (q == out && q_ss == o_ss && q_sh == o_sh) return true;
+  auto lo = [&](const uint16_t* p, int64_t ss, int64_t sh) {
+    return reinterpret_cast<intptr_t>(p) + 2 * (std::min<int64_t>(0, (Sq - 1) * ss) + std::min<int64_t>(0, (H - 1) * sh));
+  };
+  auto hi = [&](const uint16_t* p, int64_t ss, int64_t sh) {
+    return reinterpret_cast<intptr_t>(p) + 2 * (std::max<int64_t>(0, (Sq - 1) * ss) + std::max<int64_t>(0, (H - 1) * sh) + D);
+  };
+  return hi(q, q_ss, q_sh) <= lo(out, o_ss, o_sh) || hi(out, o_ss, o_sh) <= lo(q, q_ss, q_sh);
+}
+
+// One-call attention without RMSNorm + RoPE: hand the raw queries to the 128-query kernel where it runs. Where out overlaps
+// q the pre-pass quantizes them, so that every query is read before the first row of out is written.
+void raw_queries(Work& w, const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* out, int64_t o_ss, int64_t o_sh,
+                 int64_t Sq, int64_t Sk, int64_t H) {
+  const bool clear = out_clear_of(q, q_ss, q_sh, out, o_ss, o_sh, Sq, H);
+  if (!plan_forward(Sq, Sk, H, clear, w.tail != nullptr, device_cus()).raw) return;
   w.rawq = q;
   w.rq_ss = q_ss;
   w.rq_sh = q_sh;
@@ -967,16 +984,18 @@ extern "C" int rh3_int8_attention_noalloc(const uint16_t* q, int64_t q_ss, int64
   if (int e = scratch_of(stream, &base)) return e;
   Work w = layout(base, Sq, Sk, H, false);
   const RR none{nullptr, nullptr, 0.f, 0};
-  raw_queries(w, q, q_ss, q_sh, Sq, Sk, H);
+  raw_queries(w, q, q_ss, q_sh, out, o_ss, o_sh, Sq, Sk, H);
   if (int e = prepass(q, q_ss, q_sh, k, k_ss, k_sh, v, v_ss, v_sh, Sq, Sk, H, none, none, smooth_k, w, stream))
     return e;
   return forward(w, Sq, Sk, H, scale, out, o_ss, o_sh, stream);
 }
 
-extern "C" int rh3_attention_plan(int64_t Sq, int64_t Sk, int64_t H, int raw, int tail, int cus, int64_t* plan) {
+extern "C" int rh3_attention_plan(const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* out, int64_t o_ss,
+                                  int64_t o_sh, int64_t Sq, int64_t Sk, int64_t H, int tail, int cus, int64_t* plan) {
   clear_error();
   RH3_REQUIRE(Sq > 0 && Sk > 0 && H > 0 && cus >= 0 && plan, "attention_plan: sizes must be positive, plan set");
-  const FwdPlan p = plan_forward(Sq, Sk, H, raw != 0, tail != 0 && attn_ws::has_tail(Sq, H), cus > 0 ? cus : device_cus());
+  const bool raw = q != nullptr && out_clear_of(q, q_ss, q_sh, out, o_ss, o_sh, Sq, H);
+  const FwdPlan p = plan_forward(Sq, Sk, H, raw, tail != 0 && attn_ws::has_tail(Sq, H), cus > 0 ? cus : device_cus());
   plan[0] = p.small ? SM_BQ : FWD_BQ;
   plan[1] = p.raw;
   plan[2] = p.npair;
@@ -1077,7 +1096,7 @@ extern "C" int rh3_int8_attention(const uint16_t* q, int64_t q_ss, int64_t q_sh,
   RH3_REQUIRE(workspace && aligned16(workspace) && workspace_bytes >= w.bytes,
               "int8_attention: workspace %lld bytes < required %lld", (long long)workspace_bytes, (long long)w.bytes);
   const RR none{nullptr, nullptr, 0.f, 0};
-  raw_queries(w, q, q_ss, q_sh, Sq, Sk, H);
+  raw_queries(w, q, q_ss, q_sh, out, o_ss, o_sh, Sq, Sk, H);
   if (int e = prepass(q, q_ss, q_sh, k, k_ss, k_sh, v, v_ss, v_sh, Sq, Sk, H, none, none, smooth_k, w, stream))
     return e;
   return forward(w, Sq, Sk, H, scale, out, o_ss, o_sh, stream);

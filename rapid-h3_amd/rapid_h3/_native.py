@@ -50,7 +50,7 @@ SIGNATURES = {
                                _P, _I, _P], _C),
     "rh3_rms_rope_qk": ([_P, _I, _I, _P, _I, _I, _I, _I, _P, _C, _P, _P, _F, _P], _C),
     "rh3_attention_forward": ([_I, _I, _I, _F, _P, _I, _I, _P, _I, _P], _C),
-    "rh3_attention_plan": ([_I, _I, _I, _C, _C, _C, ctypes.POINTER(ctypes.c_int64)], _C),
+    "rh3_attention_plan": ([_P, _I, _I, _P, _I, _I, _I, _I, _I, _C, _C, ctypes.POINTER(ctypes.c_int64)], _C),
     "rh3_attention_prepass": ([_P, _I, _I, _P, _I, _I, _P, _I, _I, _I, _I, _I, _P, _C, _P, _P, _F, _C, _P, _I,
                                ctypes.POINTER(ctypes.c_void_p), _P], _C),
     "rh3_attention_prepass_qkv": ([_P, _I, _I, _P, _I, _I, _I, _I, _P, _C, _P, _F, _C, _P, _I,

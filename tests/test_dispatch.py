@@ -6,11 +6,14 @@ import pytest
 CUS = 256
 
 
-def attention_plan(sq, sk, h, raw=False, tail=True, cus=CUS):
-    """(queries per workgroup, queries quantized by the main kernel, workgroups run as two key halves)"""
+def attention_plan(sq, sk, h, raw=False, tail=True, cus=CUS, q=None, out=None):
+    """(queries per workgroup, queries quantized by the main kernel, workgroups run as two key halves). raw: the one
+    call without RMSNorm + RoPE, its out clear of q; or q and out as (address, token stride, head stride)"""
     from rapid_h3 import _native as nat
     p = (ctypes.c_int64 * 3)()
-    nat.call("rh3_attention_plan", sq, sk, h, int(raw), int(tail), cus, p)
+    if raw:
+        q, out = (1 << 40, h * 128, 128), (1 << 50, h * 128, 128)
+    nat.call("rh3_attention_plan", *(q or (None, 0, 0)), *(out or (None, 0, 0)), sq, sk, h, int(tail), cus, p)
     return tuple(p)
 
 
@@ -34,3 +37,27 @@ def test_attention_plan_short_and_long_items():
     assert attention_plan(2816, 2816, 24, raw=True) == (128, 1, 0)      # it saves the pre-pass over the queries
     assert attention_plan(1024, 65536, 24)[0] == 128
     assert attention_plan(1024, 65537, 24)[0] == 384                    # past the 128-query kernel's scale table
+
+
+def test_attention_plan_out_over_the_queries():
+    """The main kernel quantizes the queries itself only where no other workgroup's out rows can lie on them."""
+    s, h = 1024, 24
+    base, row = 1 << 40, 2 * 128
+    q = (base, h * 128, 128)                                 # [S, H, 128]
+    end = base + s * h * row
+
+    def raw(out, q=q):
+        return attention_plan(s, 512, h, q=q, out=out)[1]
+    assert raw((base, h * 128, 128)) == 1                    # in place
+    assert raw((base, 128, s * 128)) == 0                    # head-major over the same storage
+    assert raw((base + row, h * 128, 128)) == 0              # one head on
+    assert raw((end - row, h * 128, 128)) == 0               # over the last head of the last token
+    assert raw((end, h * 128, 128)) == 1                     # right behind q, and right before it
+    assert raw((base - s * h * row, 128, s * 128)) == 1
+    assert raw((base - s * h * row + row, 128, s * 128)) == 0
+    assert raw((end - row, -h * 128, -128)) == 0             # rows and heads backwards over q
+    assert raw((end + (s * h - 1) * row, -h * 128, -128)) == 1
+    fused = (base, 3 * h * 128, 128)                         # q of a [S, 3, H, 128] buffer, out in its v part
+    assert raw((base + 2 * h * row, 3 * h * 128, 128), q=fused) == 0
+    # the plan without it is that of a call whose pre-pass quantizes the queries
+    assert attention_plan(s, 512, h, q=q, out=(base, 128, s * 128)) == attention_plan(s, 512, h)

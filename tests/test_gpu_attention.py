@@ -193,6 +193,27 @@ def test_attention_nan_queries(dev, sq, sk, h):
     assert torch.equal(out.view(torch.int16), attention.attention(zero.to(dev), kt, vt).view(torch.int16))
 
 
+@pytest.mark.parametrize("where", ["in place", "head-major", "value"])
+def test_attention_out_over_operands(dev, where):
+    """out over the storage of q (its own layout, or head-major: other workgroups' rows) or of v: the bits of a call
+    whose out lies elsewhere, on a grid of several rounds of 128-query workgroups."""
+    import torch
+    from rapid_h3 import attention
+    s, h, sk = 9000, 24, 129
+    g = torch.Generator().manual_seed(8)
+    q, k, v = (torch.randn(n, h, 128, generator=g).to(torch.bfloat16).to(dev) for n in (s, sk, sk))
+    if where == "value":
+        q = q[:sk].contiguous()
+    want = attention.attention(q, k, v)
+    if where == "value":
+        out = v
+    else:
+        out = q if where == "in place" else q.view(h, s, 128).transpose(0, 1)
+    assert out.data_ptr() == (v if where == "value" else q).data_ptr()
+    attention.attention(q, k, v, out=out)
+    assert torch.equal(out.contiguous().view(torch.int16), want.view(torch.int16))
+
+
 def test_attention_strided_out(dev):
     """q/k/v as views of one [S, 3*H*128] qkv buffer; output into a head-major [1, H, S, D] buffer
     through out=o[0].transpose(0, 1) (the _fused_block call, __init__.py:283-291)."""
