@@ -298,10 +298,11 @@ int rh3_attention_forward(int64_t Sq, int64_t Sk, int64_t H, float scale,
  * quantize the queries itself (only their addresses are used); q NULL: any other call. tail 0:
  * rh3_int8_attention_noalloc, which has no room for split partials. RH3_ATTN_SPLIT is read. plan[0] queries per
  * workgroup (128 or 384), plan[1] 1 when the main kernel quantizes the queries, plan[2] the 384-query workgroups
- * that run as two key halves. No counterpart in the reference. */
+ * that run as two key halves, plan[3] 1 when the pre-pass (with smooth_k) runs in two launches. No counterpart in
+ * the reference. */
 int rh3_attention_plan(const uint16_t* q, int64_t q_ss, int64_t q_sh,
                        const uint16_t* out, int64_t o_ss, int64_t o_sh,
-                       int64_t Sq, int64_t Sk, int64_t H, int tail, int cus, int64_t* plan /* [3] */);
+                       int64_t Sq, int64_t Sk, int64_t H, int tail, int cus, int64_t* plan /* [4] */);
 
 /* ---------------------------------------------------------------------------------------------
  * INT8 flash attention with the reference's production numerics (attn_int8.cu configs 80-99: attn_fwd8

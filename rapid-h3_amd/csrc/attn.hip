@@ -740,13 +740,20 @@ int check_qkv(const char* name, const uint16_t* q, int64_t q_ss, int64_t q_sh, c
   return RH3_OK;
 }
 
+// whether the pre-pass runs in two launches (pre_a_kernel, pre_b_kernel): a short call whose parts fit one grid
+bool merged_prepass(int64_t Sq, int64_t Sk, int64_t H, bool smooth_k, bool raw) {
+  const int64_t nchunk = attn_ws::nchunks(Sk);
+  const int64_t blocks = (smooth_k ? nchunk : 0) + (raw ? 0 : pad(Sq) / BLK) + pad(Sk) / 64;
+  return nchunk <= PRE_CHUNKS && blocks * H <= MAX_GRID_256;
+}
+
 int prepass(const uint16_t* q, int64_t q_ss, int64_t q_sh, const uint16_t* k, int64_t k_ss, int64_t k_sh,
             const uint16_t* v, int64_t v_ss, int64_t v_sh, int64_t Sq, int64_t Sk, int64_t H, const RR& rq,
             const RR& rk, int smooth_k, const Work& w, hipStream_t st) {
   const int64_t sqp = pad(Sq), skp = pad(Sk);
   const int nchunk = static_cast<int>((Sk + CHUNK - 1) / CHUNK);
   const float* mean = nullptr;
-  if (nchunk <= PRE_CHUNKS) {
+  if (merged_prepass(Sq, Sk, H, smooth_k, w.rawq != nullptr)) {
     PreArgs a{q, k, v, q_ss, q_sh, k_ss, k_sh, v_ss, v_sh, Sq, Sk, sqp, skp, static_cast<int>(H), nchunk, smooth_k, rq, rk, w,
               0, 0};
     const unsigned heads = static_cast<unsigned>(H);
@@ -795,7 +802,7 @@ bool use_small(int64_t Sq, int64_t Sk, int64_t H, bool qf, int64_t npair, int64_
   if (cus <= 0 || pad(Sk) / BLK > SM_KB) return false;
   const double n = static_cast<double>((Sk + STEP - 1) / STEP);
   const int64_t big = (Sq + FWD_BQ - 1) / FWD_BQ * H, small = (Sq + SM_BQ - 1) / SM_BQ * H;
-  if (small >= (int64_t{1} << 31)) return false;
+  if (small > MAX_GRID_256) return false;
   const int64_t bf = big / cus, br = big % cus, sf = small / (3 * cus), sr = (small % (3 * cus) + cus - 1) / cus;
   double tb = static_cast<double>(bf) * (12 + 2.0 * n);
   if (br > 0) tb += bf == 0 ? 10 + 1.75 * n : npair > 0 ? 10 + n : 12 + 2.0 * n;
@@ -999,6 +1006,7 @@ extern "C" int rh3_attention_plan(const uint16_t* q, int64_t q_ss, int64_t q_sh,
   plan[0] = p.small ? SM_BQ : FWD_BQ;
   plan[1] = p.raw;
   plan[2] = p.npair;
+  plan[3] = merged_prepass(Sq, Sk, H, true, p.raw);
   return RH3_OK;
 }
 

@@ -885,17 +885,33 @@ int check_rr_u8(const char* name, const uint16_t* tab, int rot, const uint16_t* 
   return RH3_OK;
 }
 
+// workgroups of the K quantizer
+template <bool BLK>
+int64_t k_blocks(const PreU8& a) { return BLK ? a.skp / TILE * a.H : tokq_blocks(a.skp, a.H); }
+
+// the merged launches are one-dimensional
+template <bool BLK>
+int check_grids(const PreU8& a, const char* name) {
+  const int64_t ga = static_cast<int64_t>(a.nchunk) * a.H * (a.smooth_k ? 2 : 1) + (a.q ? tokq_blocks(a.sqp, a.H) : 0);
+  const int64_t gb = k_blocks<BLK>(a) + a.skp / TILE * a.H;
+  RH3_REQUIRE(ga <= MAX_GRID_256 && gb <= MAX_GRID_256, "%s: Sq=%lld Sk=%lld H=%d needs %lld workgroups, beyond the grid limit",
+              name, (long long)a.Sq, (long long)a.Sk, a.H, (long long)(ga > gb ? ga : gb));
+  return RH3_OK;
+}
+
 // the second level of the statistics, then the K quantizer and the V codes
 template <bool F8, bool BLK>
 int prepass_tail(PreU8& a, hipStream_t st, const char* name) {
+  if (int e = check_grids<BLK>(a, name)) return e;
   hipLaunchKernelGGL(kmean_vfinal_kernel, dim3(a.H, 2), dim3(KMEAN_NT), 0, st, a.w, a.nchunk, a.Sk, a.smooth_k, a.smooth_v);
   const unsigned tiles = static_cast<unsigned>(a.skp / TILE * a.H);
-  a.nk = BLK ? tiles : tokq_blocks(a.skp, a.H);
+  a.nk = static_cast<unsigned>(k_blocks<BLK>(a));
   hipLaunchKernelGGL((pre_b_u8_kernel<F8, BLK>), dim3(a.nk + tiles), dim3(256), 0, st, a);
   return launch_status(name);
 }
 template <bool F8, bool BLK>
 int prepass_all(PreU8& a, hipStream_t st, const char* name) {
+  if (int e = check_grids<BLK>(a, name)) return e;
   const unsigned chunks = static_cast<unsigned>(a.nchunk) * a.H;
   a.nk = a.smooth_k ? chunks : 0;
   a.nv = chunks;

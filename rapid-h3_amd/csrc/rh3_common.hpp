@@ -30,6 +30,9 @@ int launch_status(const char* what);
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// one-dimensional grids of 256-thread workgroups: a launch holds at most 2^32 - 1 threads per dimension
+constexpr int64_t MAX_GRID_256 = (int64_t{1} << 24) - 1;
+
 // compute units of the current device (0 if the query fails), cached per device
 int device_cus();
 

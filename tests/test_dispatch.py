@@ -6,15 +6,16 @@ import pytest
 CUS = 256
 
 
-def attention_plan(sq, sk, h, raw=False, tail=True, cus=CUS, q=None, out=None):
-    """(queries per workgroup, queries quantized by the main kernel, workgroups run as two key halves). raw: the one
+def attention_plan(sq, sk, h, raw=False, tail=True, cus=CUS, q=None, out=None, full=False):
+    """(queries per workgroup, queries quantized by the main kernel, workgroups run as two key halves[, pre-pass in two
+    launches, with full]). raw: the one
     call without RMSNorm + RoPE, its out clear of q; or q and out as (address, token stride, head stride)"""
     from rapid_h3 import _native as nat
-    p = (ctypes.c_int64 * 3)()
+    p = (ctypes.c_int64 * 4)()
     if raw:
         q, out = (1 << 40, h * 128, 128), (1 << 50, h * 128, 128)
     nat.call("rh3_attention_plan", *(q or (None, 0, 0)), *(out or (None, 0, 0)), sq, sk, h, int(tail), cus, p)
-    return tuple(p)
+    return tuple(p)[:4 if full else 3]
 
 
 @pytest.mark.parametrize("sq,sk,h,npair", [(5583, 5583, 24, 104), (2600, 5583, 49, 87)])
@@ -61,3 +62,26 @@ def test_attention_plan_out_over_the_queries():
     assert raw((base + 2 * h * row, 3 * h * 128, 128), q=fused) == 0
     # the plan without it is that of a call whose pre-pass quantizes the queries
     assert attention_plan(s, 512, h, q=q, out=(base, 128, s * 128)) == attention_plan(s, 512, h)
+
+
+def test_attention_grids_stay_below_the_launch_limit():
+    """A one-dimensional grid holds 2^24 - 1 workgroups of 256 threads: past that the query kernel, or the merged
+    pre-pass, of the other form is taken, and the production pre-passes name the limit before any launch."""
+    from rapid_h3 import _native as nat
+    h = 300
+    most = ((1 << 24) - 1) // h                               # 128-query workgroups per head
+    assert attention_plan(most * 128, 64, h) == (128, 0, 0)
+    assert attention_plan((most + 1) * 128, 64, h)[0] == 384
+    assert attention_plan((most - 3) * 128, 64, h, full=True)[3] == 1   # and a chunk of K statistics, two 64-key V slabs
+    assert attention_plan(most * 128, 64, h, full=True)[3] == 0
+    assert attention_plan(4096, 4096, 24, full=True)[3] == 1
+    assert attention_plan(4096, 4097, 24, full=True)[3] == 0
+    fake = ctypes.c_void_p(0x1000)                            # never dereferenced: refused first
+    big = ctypes.c_int64(1 << 62)
+    s, h = 4_000_000, 200                                     # S H (1/64 + 1/128) = 18.75 M workgroups
+    qkv = [fake, 128, 128] * 3
+    tail = [1, 1, 1, fake, 128, 128, fake, big, None]
+    for name, mid in (("rh3_int8_attention_u8", [None, 0, None, None, 1e-5, 0.1, 0, 0.0]),
+                      ("rh3_int8_attention_bk", [0.1])):
+        st = getattr(nat.lib(), name)(*qkv, s, s, h, *mid, *tail)
+        assert st == 1 and "beyond the grid limit" in nat.last_error(), (name, nat.last_error())
