@@ -454,6 +454,30 @@ void launch_vec(const QuantArgs& a, hipStream_t st) {
   }
 }
 
+// rows that the norm + modulation form of one wavefront per row holds at once: its workgroups of 4 per CU (by its registers),
+// and 0 where they cannot be asked for
+template <int NCH, typename TabT, bool VEC>
+int64_t resident_rows() {
+  static const int per_cu = [] {
+    int n = 0;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, quant_rows_kernel<NCH, KIND_NORMMOD, false, TabT, VEC>, 256, 0) == hipSuccess ? n : 0;
+  }();
+  return int64_t{4} * per_cu * device_cus();
+}
+template <typename TabT, bool VEC>
+int64_t normmod_resident(int64_t K) {   // the kernels of launch_vec up to 6144 columns
+  const int64_t nch = (K + 511) / 512;
+  const int64_t rows = nch <= 1   ? resident_rows<1, TabT, VEC>()
+                       : nch <= 2 ? resident_rows<2, TabT, VEC>()
+                       : nch <= 4 ? resident_rows<4, TabT, VEC>()
+                       : nch <= 6 ? resident_rows<6, TabT, VEC>()
+                       : nch <= 8 ? resident_rows<8, TabT, VEC>()
+                                  : resident_rows<12, TabT, VEC>();
+  // unaligned bf16 tables, read two bytes at a time by every row, cost a full chip more than the staging (4,096 x 4096 17.4 /
+  // 16.0, 4,096 x 3072 13.6 / 13.1)
+  return VEC || sizeof(TabT) == 4 ? rows : rows * 3 / 4;
+}
+
 // One workgroup per row (all but the norm's), its 4 wavefronts taking every 4th 512-column chunk (at most 8 each, so the
 // row stays in 32 VGPRs per lane, or 64 for SwiGLU's fp32 values); the row absmax goes through LDS. Same arithmetic as
 // quant_rows_kernel (max is order-free). A call of few rows is bound by the time one row takes (its loads, then 8 quotients
@@ -560,25 +584,28 @@ int launch(const QuantArgs& a, hipStream_t st, const char* name) {
       return launch_status(name);
     }
   }
-  // up to 6144 columns the staged table and weight rows fit in 72 KB of LDS
-  // (long calls: a workgroup of 16 rows first copies its table rows, 9 us of which a short call hides nothing; us, one wavefront
-  // per row against this kernel, fp32 tables: 512 x 3072 8.5 / 13.2, 4,096 x 3072 13.2 / 15.3, 5,583 x 3072 21.0 / 17.4, 8,192 x
-  // 1024 9.1 / 10.1, 11,000 x 1024 11.7 / 11.3, 2,816 x 4096 14.1 / 17.4, 2,816 x 5376 18.7 / 22.4, 4,096 x 5376 30.0 / 23.8)
-  const bool shortcall = a.M <= 8192 && a.M * a.K <= (12 << 20);
-  if (KIND == KIND_NORMMOD && !FP8 && a.K <= 6144 && a.K % 8 == 0 && !shortcall) {
-    const dim3 grid(static_cast<unsigned>((a.M + NM_WAVES * NM_RPW - 1) / (NM_WAVES * NM_RPW))), block(64 * NM_WAVES);
-    const size_t lds = static_cast<size_t>(a.K) * (4 + 4 + 4);
-    const int64_t nch = (a.K + 511) / 512;
-    if (nch <= 2) hipLaunchKernelGGL((quant_normmod_lds_kernel<2, TabT>), grid, block, lds, st, a);
-    else if (nch <= 4) hipLaunchKernelGGL((quant_normmod_lds_kernel<4, TabT>), grid, block, lds, st, a);
-    else if (nch <= 6) hipLaunchKernelGGL((quant_normmod_lds_kernel<6, TabT>), grid, block, lds, st, a);
-    else if (nch <= 8) hipLaunchKernelGGL((quant_normmod_lds_kernel<8, TabT>), grid, block, lds, st, a);
-    else hipLaunchKernelGGL((quant_normmod_lds_kernel<12, TabT>), grid, block, lds, st, a);
-    return launch_status(name);
-  }
   // 16-byte modulation-table loads when every table row start is 16-byte aligned
   const bool vec = KIND != KIND_NORMMOD || (aligned16(a.shift) && aligned16(a.scale) &&
                                             (a.ld_tab * static_cast<int64_t>(sizeof(TabT))) % 16 == 0);
+  // Up to 6144 columns the staged table and weight rows fit in 72 KB of LDS. A workgroup of 16 rows first copies its table
+  // rows, which a call whose rows all run at once on one wavefront each (normmod_resident) hides nothing of; past that the
+  // second round of wavefronts costs more. us, one wavefront per row / staged, fp32 tables: 2,816 x 5376 15.6 / 20.9,
+  // 3,072 x 5376 16.0 / 21.1, 3,400 x 5376 26.6 / 21.2, 4,096 x 4096 13.4 / 16.7, 4,500 x 4096 21.3 / 18.8, 4,096 x 3072
+  // 11.2 / 13.9, 5,000 x 3072 12.0 / 15.0, 5,583 x 3072 18.7 / 15.6, 8,192 x 2048 11.8 / 12.5, 9,000 x 2048 17.0 / 14.6, 8,192 x
+  // 1024 7.4 / 9.0, 11,000 x 1024 9.5 / 9.9.
+  if constexpr (KIND == KIND_NORMMOD && !FP8) {
+    if (a.K <= 6144 && a.M > (vec ? normmod_resident<TabT, true>(a.K) : normmod_resident<TabT, false>(a.K))) {
+      const dim3 grid(static_cast<unsigned>((a.M + NM_WAVES * NM_RPW - 1) / (NM_WAVES * NM_RPW))), block(64 * NM_WAVES);
+      const size_t lds = static_cast<size_t>(a.K) * (4 + 4 + 4);
+      const int64_t nch = (a.K + 511) / 512;
+      if (nch <= 2) hipLaunchKernelGGL((quant_normmod_lds_kernel<2, TabT>), grid, block, lds, st, a);
+      else if (nch <= 4) hipLaunchKernelGGL((quant_normmod_lds_kernel<4, TabT>), grid, block, lds, st, a);
+      else if (nch <= 6) hipLaunchKernelGGL((quant_normmod_lds_kernel<6, TabT>), grid, block, lds, st, a);
+      else if (nch <= 8) hipLaunchKernelGGL((quant_normmod_lds_kernel<8, TabT>), grid, block, lds, st, a);
+      else hipLaunchKernelGGL((quant_normmod_lds_kernel<12, TabT>), grid, block, lds, st, a);
+      return launch_status(name);
+    }
+  }
   if (vec) launch_vec<KIND, FP8, TabT, true>(a, st);
   else launch_vec<KIND, FP8, TabT, false>(a, st);
   return launch_status(name);

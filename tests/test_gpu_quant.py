@@ -73,10 +73,12 @@ def test_rows_per_workgroup_forms(dev, m, k):
     assert np.allclose(to_np(s)[rows], es, rtol=1e-5)
 
 
-@pytest.mark.parametrize("m,k", [(8192, 1024), (8193, 1024), (4096, 3072), (4097, 3072)])
+@pytest.mark.parametrize("m,k", [(8192, 1024), (8193, 1024), (4096, 3072), (4097, 3072), (5120, 3072), (5121, 3072),
+                                 (4096, 4096), (4097, 4096), (2816, 5376), (3072, 5376), (3073, 5376)])
 def test_norm_mod_forms(dev, m, k):
-    """The norm + modulation quantizer on both sides of the line between one wavefront per row and staged table rows:
-    bit-exact against the oracle on a sample of rows."""
+    """The norm + modulation quantizer on both sides of the line between one wavefront per row and staged table rows (on
+    256 CUs: the rows whose wavefronts are all resident at the kernel's registers, 8, 5, 4 and 3 of them to a SIMD):
+    bit-exact against the oracle on a sample of rows; the same with bf16 tables whose rows are not 16-byte aligned."""
     from rapid_h3 import quant
     rng = np.random.default_rng(m + k)
     rows = np.unique(np.r_[0, 16, 17, m - 1, rng.integers(0, m, 60)])
@@ -85,6 +87,11 @@ def test_norm_mod_forms(dev, m, k):
     sh, sc = (0.3 * rng.standard_normal((2, k)).astype(np.float32) for _ in range(2))
     q, s = quant.norm_mod_quant_rows_i8(*(to_dev(t, dev) for t in (x, w)), 1e-6, *(to_dev(t, dev) for t in (idx, sh, sc)))
     eq, es = oq.norm_mod_quant_rows_i8(x[rows], w, 1e-6, idx[rows], sh, sc)
+    assert np.array_equal(to_np(q)[rows], eq) and np.array_equal(to_np(s)[rows], es)
+    tabs = to_dev(_bf(np.concatenate([np.zeros((2, 1)), sh, sc], 1)), dev)
+    q, s = quant.norm_mod_quant_rows_i8(*(to_dev(t, dev) for t in (x, w)), 1e-6, to_dev(idx, dev), tabs[:, 1:k + 1], tabs[:, k + 1:])
+    assert tabs[:, 1:].data_ptr() % 16 != 0
+    eq, es = oq.norm_mod_quant_rows_i8(x[rows], w, 1e-6, idx[rows], _bf(sh), _bf(sc))
     assert np.array_equal(to_np(q)[rows], eq) and np.array_equal(to_np(s)[rows], es)
 
 
