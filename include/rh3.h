@@ -176,6 +176,12 @@ int rh3_gemm_i8_gated_rows(const int8_t* xq, int64_t ldx, const float* xs, const
 int rh3_gemm_i8_acc(const int8_t* xq, int64_t ldx, const int8_t* wq, int64_t ldw, int32_t* acc, int64_t ldc,
                     int64_t M, int64_t N, int64_t K, int32_t* ctr, hipStream_t stream);
 
+/* Verification: how the GEMMs (but _qkv, which runs on 256 x 256 tiles, a workgroup each) run a call with packed operand
+ * rows, by the rule they apply (no device access but the CU count where cus is 0). plan[0] x plan[1] the tile of the
+ * rows from plan[2] on; the rows before plan[2] run on 256 x 256 tiles in form plan[3]: 1 a workgroup each, 2 one
+ * workgroup per CU in fixed shares, 3 the same with the tile counters where ctr is given; 0 no such rows. */
+int rh3_gemm_plan(int64_t M, int64_t N, int64_t K, int cus, int64_t* plan /* [4] */);
+
 /* The qkv projection with the attention pre-pass partly fused into its epilogue.
  * replaces cutlass_fp8.int8_gemm_qkv_prep -> run_qkv_prep / VisitorQkvPrep (cutlass_fp8.py:42-46,
  * fp8_rowwise.cu:108-272, :635-655): out [M, 3*H*128] = bf16((acc * xs) * ws [+ bias]) for the k and v columns

@@ -878,22 +878,33 @@ GemmArgs rows_from(GemmArgs a, int64_t r0, int64_t out_elem) {
   return a;
 }
 
+// How the 256 x 256 tiles of a call run: a workgroup each, or one workgroup per CU (the LDS use admits no second) over a
+// tile sequence (K a multiple of 256, at least 512), which it walks in fixed shares or claims from the tile counters.
+// The counters pay from four rounds of tiles on: with fewer, the fill kernel before the GEMM costs more than the XCDs'
+// imbalance (us, with / without: 756 tiles of K = 7168 320 / 306, 504 of K = 3072 116 / 98, 1,080 of K = 3072 213 / 217, 1,680
+// of K = 5376 515 / 536).
+enum Form256 { FORM_NONE = 0, FORM_SINGLE = 1, FORM_SHARES = 2, FORM_COUNTED = 3 };
+Form256 form_256(int64_t M, int64_t N, int64_t K, int64_t cus, bool off32) {
+  const int64_t nb = (M + BM - 1) / BM * ((N + BN - 1) / BN), nk = K / BK;
+  if (nk % 4 != 0 || nk < 8 || cus <= 0 || !off32) return FORM_SINGLE;
+  return nb >= 4 * cus ? FORM_COUNTED : FORM_SHARES;
+}
+
+// the 32-bit lane offsets of the persistent and small-tile kernels reach 255 rows of either operand
+bool offsets_fit(int64_t ldx, int64_t ldw) { return 255 * ldx + 64 < (1ll << 32) && 255 * ldw + 64 < (1ll << 32); }
+
 // every row on the 256 x 256 tile
 template <bool FP8, int EPI>
-int run_256(GemmArgs a, hipStream_t st, const char* name, int64_t cus, bool off32) {
+int run_256(GemmArgs a, hipStream_t st, const char* name, int64_t cus) {
   a.tiles_m = static_cast<int>((a.M + BM - 1) / BM);
   a.tiles_n = static_cast<int>((a.N + BN - 1) / BN);
   const int64_t nb = static_cast<int64_t>(a.tiles_m) * a.tiles_n;
   if constexpr (EPI != EPI_QKV) {
-    const int64_t nk = a.K / BK;
-    if (nk % 4 == 0 && nk >= 8 && cus > 0 && off32) {
-      const int64_t grid = nb < cus ? nb : cus;  // one workgroup per CU (the LDS use admits no second)
-      const dim3 g(static_cast<unsigned>(grid));
-      // The tile counters pay from four rounds of tiles on: with fewer, the fill kernel before the GEMM costs more than
-      // the XCDs' imbalance (us, with / without: 756 tiles of K = 7168 320 / 306, 504 of K = 3072 116 / 98, 1,080 of
-      // K = 3072 213 / 217, 1,680 of K = 5376 515 / 536). They are cleared by that fill kernel (no hipMemsetAsync: the
-      // call stays graph-safe).
-      if (a.ctr != nullptr && nb >= 4 * cus) {
+    const Form256 form = form_256(a.M, a.N, a.K, cus, offsets_fit(a.ldx, a.ldw));
+    if (form != FORM_SINGLE) {
+      const dim3 g(static_cast<unsigned>(nb < cus ? nb : cus));
+      // the counters are cleared by a fill kernel (no hipMemsetAsync: the call stays graph-safe)
+      if (a.ctr != nullptr && form == FORM_COUNTED) {
         hipLaunchKernelGGL(zero_ctr_kernel, dim3(1), dim3(64), 0, st, a.ctr);
         hipLaunchKernelGGL((gemm_persistent_kernel<FP8, EPI, true>), g, dim3(512), 0, st, a);
       } else {
@@ -912,23 +923,21 @@ int run(GemmArgs a, hipStream_t st, const char* name) {
   if (a.M == 0 || a.N == 0) return RH3_OK;
   RH3_REQUIRE((a.M + BM - 1) / BM * ((a.N + BN - 1) / BN) < (1ll << 31), "%s: too many tiles", name);
   const int64_t cus = device_cus();
-  // the 32-bit lane offsets of the persistent and small-tile kernels reach 255 rows of either operand
-  const bool off32 = 255 * a.ldx + 64 < (1ll << 32) && 255 * a.ldw + 64 < (1ll << 32);
   if constexpr (EPI != EPI_QKV) {
-    if (off32 && cus > 0) {
+    if (offsets_fit(a.ldx, a.ldw) && cus > 0) {
       const TilePlan p = plan_tiles(a.M, a.N, a.K, cus);
       if (p.tile != TILE_256) {
         if (p.head > 0) {
           GemmArgs h = a;
           h.M = p.head;
-          if (int e = run_256<FP8, EPI>(h, st, name, cus, off32)) return e;
+          if (int e = run_256<FP8, EPI>(h, st, name, cus)) return e;
           a = rows_from(a, p.head, EPI == EPI_ACC ? 4 : 2);
         }
         return run_tile(FP8, EPI, p.tile, a, st, name);
       }
     }
   }
-  return run_256<FP8, EPI>(a, st, name, cus, off32);
+  return run_256<FP8, EPI>(a, st, name, cus);
 }
 
 int check(const char* name, const void* xq, int64_t ldx, const void* wq, int64_t ldw, const void* out, int64_t ldo,
@@ -952,6 +961,21 @@ int check(const char* name, const void* xq, int64_t ldx, const void* wq, int64_t
 }  // namespace rh3
 
 using namespace rh3;
+
+extern "C" int rh3_gemm_plan(int64_t M, int64_t N, int64_t K, int cus, int64_t* plan) {
+  clear_error();
+  RH3_REQUIRE(M > 0 && N > 0 && K > 0 && K % BK == 0 && N % 8 == 0 && cus >= 0 && plan, "gemm_plan: bad sizes");
+  const int64_t c = cus > 0 ? cus : device_cus();
+  const bool fit = offsets_fit(K, K);
+  const TilePlan p = fit && c > 0 ? plan_tiles(M, N, K, c) : TilePlan{TILE_256, 0};
+  const int tm[] = {BM, 128, 128, 256, 256}, tn[] = {BN, 64, 128, 128, 192};   // by TileId
+  const int64_t m256 = p.tile == TILE_256 ? M : p.head;
+  plan[0] = tm[p.tile];
+  plan[1] = tn[p.tile];
+  plan[2] = m256;
+  plan[3] = m256 > 0 ? form_256(m256, N, K, c, fit) : FORM_NONE;
+  return RH3_OK;
+}
 
 extern "C" int rh3_gemm_i8(const int8_t* xq, int64_t ldx, const float* xs, const int8_t* wq, int64_t ldw,
                            const float* ws, const uint16_t* bias, uint16_t* out, int64_t ldo, int64_t M, int64_t N,

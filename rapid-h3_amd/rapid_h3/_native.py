@@ -40,6 +40,7 @@ SIGNATURES = {
     "rh3_gemm_i8_gated": ([_P, _I, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P, _P], _C),
     "rh3_gemm_i8_gated_rows": ([_P, _I, _P, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _P, _P], _C),
     "rh3_gemm_i8_acc": ([_P, _I, _P, _I, _P, _I, _I, _I, _I, _P, _P], _C),
+    "rh3_gemm_plan": ([_I, _I, _I, _C, ctypes.POINTER(ctypes.c_int64)], _C),
     "rh3_gemm_i8_qkv": ([_P, _I, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P, _C, _P, _P, _F, _C, _C, _P, _I, _P], _C),
     "rh3_gemm_fp8": ([_P, _I, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P, _P], _C),
     "rh3_gemm_fp8_acc": ([_P, _I, _P, _I, _P, _I, _I, _I, _I, _P, _P], _C),

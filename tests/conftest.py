@@ -55,3 +55,36 @@ def to_np(t):
     if t.dtype == torch.float8_e4m3fn:
         return t.view(torch.uint8).numpy()
     return t.numpy()
+
+
+def attention_plan(sq, sk, h, raw=False, tail=True, cus=0, q=None, out=None):
+    """How the per-block attention runs a call (rh3_attention_plan): queries per workgroup, 1 where the main kernel
+    quantizes the queries, workgroups run as two key halves, 1 where the pre-pass is two launches. raw: the one call
+    without RMSNorm + RoPE, its out clear of q; or q and out as (address, token stride, head stride). cus 0: the
+    device's."""
+    import ctypes
+    from rapid_h3 import _native as nat
+    p = (ctypes.c_int64 * 4)()
+    if raw:
+        q, out = (1 << 40, h * 128, 128), (1 << 50, h * 128, 128)
+    nat.call("rh3_attention_plan", *(q or (None, 0, 0)), *(out or (None, 0, 0)), sq, sk, h, int(tail), cus, p)
+    return tuple(p)
+
+
+def gemm_plan(m, n, k, cus=0):
+    """How a GEMM runs a call (rh3_gemm_plan): tile rows and columns, rows before them on 256 x 256 tiles, the form of
+    those (GEMM_*)."""
+    import ctypes
+    from rapid_h3 import _native as nat
+    p = (ctypes.c_int64 * 4)()
+    nat.call("rh3_gemm_plan", m, n, k, cus, p)
+    return tuple(p)
+
+
+GEMM_SMALL, GEMM_SINGLE, GEMM_SHARES, GEMM_COUNTED = range(4)   # no 256 x 256 tiles; a workgroup each; per CU: shares, counters
+
+
+def on_256_cus():
+    """The forms that the tests' shapes are chosen for are those of 256 CUs."""
+    import torch
+    return torch.cuda.get_device_properties(0).multi_processor_count == 256

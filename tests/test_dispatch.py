@@ -3,19 +3,12 @@ import ctypes
 
 import pytest
 
-CUS = 256
+from conftest import GEMM_COUNTED, GEMM_SHARES, GEMM_SINGLE, GEMM_SMALL, gemm_plan
+from conftest import attention_plan as device_plan
 
 
-def attention_plan(sq, sk, h, raw=False, tail=True, cus=CUS, q=None, out=None, full=False):
-    """(queries per workgroup, queries quantized by the main kernel, workgroups run as two key halves[, pre-pass in two
-    launches, with full]). raw: the one
-    call without RMSNorm + RoPE, its out clear of q; or q and out as (address, token stride, head stride)"""
-    from rapid_h3 import _native as nat
-    p = (ctypes.c_int64 * 4)()
-    if raw:
-        q, out = (1 << 40, h * 128, 128), (1 << 50, h * 128, 128)
-    nat.call("rh3_attention_plan", *(q or (None, 0, 0)), *(out or (None, 0, 0)), sq, sk, h, int(tail), cus, p)
-    return tuple(p)[:4 if full else 3]
+def attention_plan(*args, full=False, **kw):
+    return device_plan(*args, cus=256, **kw)[:4 if full else 3]
 
 
 @pytest.mark.parametrize("sq,sk,h,npair", [(5583, 5583, 24, 104), (2600, 5583, 49, 87)])
@@ -85,3 +78,22 @@ def test_attention_grids_stay_below_the_launch_limit():
                       ("rh3_int8_attention_bk", [0.1])):
         st = getattr(nat.lib(), name)(*qkv, s, s, h, *mid, *tail)
         assert st == 1 and "beyond the grid limit" in nat.last_error(), (name, nat.last_error())
+
+
+@pytest.mark.parametrize("m,n,k,plan", [
+    (77, 9216, 3072, (128, 64, 0, GEMM_SMALL)), (512, 6144, 3072, (128, 128, 0, GEMM_SMALL)),
+    (700, 784, 1024, (128, 64, 0, GEMM_SMALL)), (129, 16528, 64, (256, 128, 0, GEMM_SMALL)),
+    (1029, 15376, 512, (256, 192, 0, GEMM_SMALL)),
+    (1029, 15376, 1024, (128, 64, 1024, GEMM_SHARES)),           # whole rounds, then the last rows
+    (4096, 3072, 3072, (256, 256, 4096, GEMM_SHARES)),
+    (5300, 6096, 512, (256, 256, 5300, GEMM_SHARES)), (5300, 6096, 320, (256, 256, 5300, GEMM_SINGLE)),
+    (4100, 15616, 512, (256, 256, 4100, GEMM_COUNTED)),
+    (9000, 8200, 256, (256, 256, 9000, GEMM_SINGLE)),            # K below 512
+    (145152, 9216, 3072, (256, 256, 145152, GEMM_COUNTED))])
+def test_gemm_plan(m, n, k, plan):
+    assert gemm_plan(m, n, k, cus=256) == plan
+
+
+def test_gemm_counters_from_four_rounds_on():
+    assert gemm_plan(4 * 256 * 256, 256, 512, cus=256)[3] == GEMM_COUNTED
+    assert gemm_plan(4 * 256 * 256 - 256, 256, 512, cus=256)[3] == GEMM_SHARES

@@ -4,7 +4,7 @@ FP8 within rel-L2 1e-2 of the exact-product emulation."""
 import numpy as np
 import pytest
 
-from conftest import to_dev, to_np
+from conftest import GEMM_COUNTED, GEMM_SHARES, GEMM_SINGLE, GEMM_SMALL, gemm_plan, on_256_cus, to_dev, to_np
 from oracle import gemm as og
 from oracle import quant as oq
 from oracle.numerics import bf16_to_f32, f32_to_bf16
@@ -77,13 +77,22 @@ def test_gemm_shapes(dev, m, n, k):
     assert np.array_equal(to_np(out), og.int8_gemm(xq, xs, wq, ws))
 
 
-@pytest.mark.parametrize("m,n,k", [(4500, 4112, 512), (700, 784, 1024)])
-def test_gemm_persistent_epilogues(dev, m, n, k):
-    """Shapes on the persistent kernel (K a multiple of 256, at least 512): 18 x 17 = 306 tiles give some
-    workgroups two tiles, so a tile boundary falls inside the cross-tile k-loop; ragged last tile row and
-    column. Every epilogue against the oracle: int32 accumulators, plain and bias outputs, the gated residual
-    bit-exact, SwiGLU within one bf16 ulp, FP8 within rel-L2 1e-2."""
+def _reaches(m, n, k, form):
+    """The test's shape runs in the form it is there for (chosen for 256 CUs)."""
+    assert not on_256_cus() or gemm_plan(m, n, k)[3] == form
+
+
+@pytest.mark.parametrize("m,n,k,form", [(5300, 6096, 512, GEMM_SHARES), (4100, 15616, 512, GEMM_COUNTED),
+                                        (5300, 6096, 320, GEMM_SINGLE), (4500, 4112, 512, GEMM_SMALL),
+                                        (700, 784, 1024, GEMM_SMALL)])
+def test_gemm_persistent_epilogues(dev, m, n, k, form):
+    """The persistent kernel (K a multiple of 256, at least 512) in fixed shares (21 x 24 = 504 tiles) and with the tile
+    counters (17 x 61 = 1,037): several tiles per workgroup, so tile boundaries fall inside the cross-tile k-loop. Five
+    k-steps: the same tiles on a workgroup each. Below that the small tiles. Ragged last tile row and column. Every
+    epilogue against the oracle: int32 accumulators, plain and bias outputs, the gated residual bit-exact, SwiGLU within
+    one bf16 ulp, FP8 within rel-L2 1e-2."""
     from rapid_h3 import gemm
+    _reaches(m, n, k, form)
     rng = np.random.default_rng(m + n + k)
     xq = np.clip(np.rint(rng.standard_normal((m, k)) * 30), -127, 127).astype(np.int8)
     wq = np.clip(np.rint(rng.standard_normal((n, k)) * 30), -127, 127).astype(np.int8)
@@ -118,12 +127,15 @@ def test_gemm_persistent_epilogues(dev, m, n, k):
 # shapes of each tile rule on 256 CUs: one round of 128 x 64 (odd k-step counts: the two K halves differ by one), of
 # 128 x 128, of 256 x 128 and of 256 x 192, several rounds of 256 x 192, whole 256 x 256 rounds with the last rows on
 # 128 x 64, and counted 256 x 256 tiles; ragged last rows and columns, a single row, a single k-step
-@pytest.mark.parametrize("m,n,k", [(1, 16, 64), (77, 400, 192), (129, 2064, 320), (130, 8272, 192), (129, 16528, 64),
-                                   (257, 16528, 320), (1029, 15376, 512), (1029, 15376, 1024), (4100, 15616, 512)])
-def test_gemm_tile_rules(dev, m, n, k):
+@pytest.mark.parametrize("m,n,k,tile", [(1, 16, 64, (128, 64)), (77, 400, 192, (128, 64)), (129, 2064, 320, (128, 64)),
+                                        (130, 8272, 192, (128, 128)), (129, 16528, 64, (256, 128)),
+                                        (257, 16528, 320, (256, 192)), (1029, 15376, 512, (256, 192)),
+                                        (1029, 15376, 1024, (128, 64)), (4100, 15616, 512, (256, 256))])
+def test_gemm_tile_rules(dev, m, n, k, tile):
     """Every epilogue on the tile its shape is given: int8 accumulators and outputs bit-exact, SwiGLU within one bf16
     ulp, FP8 accumulators within the fp32 rounding of a K-term sum."""
     from rapid_h3 import gemm
+    assert not on_256_cus() or gemm_plan(m, n, k)[:2] == tile
     rng = np.random.default_rng(m + 3 * n + k)
     xq = np.clip(np.rint(rng.standard_normal((m, k)) * 30), -127, 127).astype(np.int8)
     wq = np.clip(np.rint(rng.standard_normal((n, k)) * 30), -127, 127).astype(np.int8)
@@ -158,16 +170,20 @@ def test_gemm_tile_rules(dev, m, n, k):
     assert np.all(np.abs(got - a @ b.T) <= k * 2.0 ** -24 * (np.abs(a) @ np.abs(b).T))
 
 
-@pytest.mark.parametrize("m,n,k", [(4500, 4112, 512), (9000, 8200, 256), (700, 784, 1024), (300, 264, 512)])
-def test_gemm_tile_counters(dev, m, n, k):
+@pytest.mark.parametrize("m,n,k,form", [(4100, 15616, 512, GEMM_COUNTED), (8200, 8208, 768, GEMM_COUNTED),
+                                        (5300, 6096, 512, GEMM_SHARES), (9000, 8200, 256, GEMM_SINGLE),
+                                        (4500, 4112, 512, GEMM_SMALL), (700, 784, 1024, GEMM_SMALL),
+                                        (300, 264, 512, GEMM_SMALL)])
+def test_gemm_tile_counters(dev, m, n, k, form):
     """The persistent kernel with per-XCD tile counters (ctr, the Python layer's default) and with the fixed tile
     shares (ctr NULL) against the oracle's int32 accumulators, bit-exact; two calls in a row on one counter buffer
-    (each call clears it). 306 and 1155 tiles (more than one per CU, so workgroups claim and steal), 12 tiles
-    (fewer than the CUs: every workgroup's first tile is its last) and 4 tiles (fewer than the 8 XCDs: some XCD
-    ranges are empty and every claim returns none)."""
+    (each call clears it): 1,037 and 1,089 tiles, so that every workgroup claims tiles and the last ones are taken from
+    other XCDs' ranges. In the other forms (fewer than four rounds of tiles, K below 512, small tiles) the counters are
+    left alone and both calls run alike."""
     import ctypes
     import torch
     from rapid_h3 import _native as nat
+    _reaches(m, n, k, form)
     rng = np.random.default_rng(m + n + k)
     xq = np.clip(np.rint(rng.standard_normal((m, k)) * 30), -127, 127).astype(np.int8)
     wq = np.clip(np.rint(rng.standard_normal((n, k)) * 30), -127, 127).astype(np.int8)
@@ -178,14 +194,19 @@ def test_gemm_tile_counters(dev, m, n, k):
         acc = torch.full((m, n), -1, dtype=torch.int32, device=dev)
         nat.call("rh3_gemm_i8_acc", nat.ptr(xt), k, nat.ptr(wt), k, nat.ptr(acc), n, m, n, k, c, nat.stream(dev))
         assert np.array_equal(to_np(acc), want)
+    assert bool((ctr == 12345).all()) == (gemm_plan(m, n, k)[3] != GEMM_COUNTED)
 
 
-@pytest.mark.parametrize("m,n,k", [(4500, 4112, 512), (300, 264, 128)])
-def test_gemm_gated_rows(dev, m, n, k):
+@pytest.mark.parametrize("m,n,k,form", [(5300, 6096, 512, GEMM_SHARES), (4100, 15616, 512, GEMM_COUNTED),
+                                        (5300, 6096, 320, GEMM_SINGLE), (4500, 4112, 512, GEMM_SMALL),
+                                        (300, 264, 128, GEMM_SMALL)])
+def test_gemm_gated_rows(dev, m, n, k, form):
     """The gated residual with a gate row per token (per-token modulation) bit-exact against the oracle, on the
-    persistent kernel (K 512) and on the one-tile-per-workgroup kernel (K 128); rows index a 7-row table."""
+    persistent kernel (fixed shares, tile counters), on the one-tile-per-workgroup kernel and on small tiles; rows index
+    a 7-row table."""
     import torch
     from rapid_h3 import gemm
+    _reaches(m, n, k, form)
     rng = np.random.default_rng(m + k)
     xq = np.clip(np.rint(rng.standard_normal((m, k)) * 30), -127, 127).astype(np.int8)
     wq = np.clip(np.rint(rng.standard_normal((n, k)) * 30), -127, 127).astype(np.int8)
@@ -323,10 +344,12 @@ def test_gemm_counter_buffers_per_stream(dev):
         assert nat.gemm_ctr(dev).data_ptr() == b
     assert a != b
     rng = np.random.default_rng(3)
-    xq = to_dev(np.clip(np.rint(rng.standard_normal((2000, 512)) * 30), -127, 127).astype(np.int8), dev)
-    wq = to_dev(np.clip(np.rint(rng.standard_normal((2048, 512)) * 30), -127, 127).astype(np.int8), dev)
-    xs = to_dev((rng.random((2000, 1)) * 1e-3 + 1e-4).astype(np.float32), dev)
-    ws = to_dev((rng.random((1, 2048)) * 1e-3 + 1e-4).astype(np.float32), dev)
+    m, n, k = 4100, 15616, 512
+    _reaches(m, n, k, GEMM_COUNTED)
+    xq = to_dev(np.clip(np.rint(rng.standard_normal((m, k)) * 30), -127, 127).astype(np.int8), dev)
+    wq = to_dev(np.clip(np.rint(rng.standard_normal((n, k)) * 30), -127, 127).astype(np.int8), dev)
+    xs = to_dev((rng.random((m, 1)) * 1e-3 + 1e-4).astype(np.float32), dev)
+    ws = to_dev((rng.random((1, n)) * 1e-3 + 1e-4).astype(np.float32), dev)
     y0 = gemm.int8_gemm(xq, xs, wq, ws)
     s.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(s):

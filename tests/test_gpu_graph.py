@@ -6,7 +6,7 @@ changes which workgroup computes a tile, not what it computes)."""
 import numpy as np
 import pytest
 
-from conftest import to_dev
+from conftest import GEMM_COUNTED, attention_plan, gemm_plan, on_256_cus, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -55,12 +55,13 @@ def _replays(g, out, want, reset=None, between=None):
 
 
 def test_graph_gemms(dev):
-    """Persistent-kernel shapes (K 512: tiles claimed from the per-XCD counters): plain, SwiGLU and the in-place gated
+    """A shape whose tiles are claimed from the per-XCD counters (1,037 of them): plain, SwiGLU and the in-place gated
     residual, captured together."""
     import torch
     from rapid_h3 import gemm
     rng = np.random.default_rng(5)
-    m, n, k = 4500, 4112, 512
+    m, n, k = 4100, 15616, 512
+    assert not on_256_cus() or gemm_plan(m, n, k)[3] == GEMM_COUNTED
     xq = to_dev(np.clip(np.rint(rng.standard_normal((m, k)) * 30), -127, 127).astype(np.int8), dev)
     wq = to_dev(np.clip(np.rint(rng.standard_normal((n, k)) * 30), -127, 127).astype(np.int8), dev)
     xs = to_dev((rng.random((m, 1)) * 1e-3 + 1e-4).astype(np.float32), dev)
@@ -91,7 +92,8 @@ def test_graph_gemms_two_graphs_at_once(dev):
     import torch
     from rapid_h3 import gemm
     rng = np.random.default_rng(15)
-    m, n, k = 6000, 4096, 1024
+    m, n, k = 4100, 15616, 512
+    assert not on_256_cus() or gemm_plan(m, n, k)[3] == GEMM_COUNTED
     sets = []
     for _ in range(2):
         xq = to_dev(np.clip(np.rint(rng.standard_normal((m, k)) * 30), -127, 127).astype(np.int8), dev)
@@ -136,17 +138,18 @@ def test_graph_gemms_two_graphs_at_once(dev):
             assert torch.equal(sets[i][6].view(torch.int16), r_w.view(torch.int16)), f"graph {i} resid {rep}"
 
 
-@pytest.mark.parametrize("config", [None, 94])
-def test_graph_attention(dev, config):
-    """The per-block recipe (pre-pass, main kernel with its work counter, split last round when the grid has one) and
-    the production numerics (config 94), each captured as one call."""
+@pytest.mark.parametrize("config,s,sk,h,form", [(None, 2600, 2600, 3, (128, 1, 0)), (None, 2600, 5583, 49, (384, 0, 87)),
+                                                (94, 2600, 2600, 3, None)])
+def test_graph_attention(dev, config, s, sk, h, form):
+    """The per-block recipe on its 128-query kernel and on the 384-query one (separate pre-pass launches, work counter,
+    split last round) and the production numerics (config 94), each captured as one call."""
     import torch
     from rapid_h3 import attention
+    assert form is None or not on_256_cus() or attention_plan(s, sk, h, raw=True)[:3] == form
     rng = np.random.default_rng(6)
-    s, h = 2600, 3
     q = to_dev(_bf(rng.standard_normal((s, h, 128))), dev)
-    k = to_dev(_bf(rng.standard_normal((s, h, 128)) + 2.0 * rng.standard_normal((1, h, 128))), dev)
-    v = to_dev(_bf(rng.standard_normal((s, h, 128))), dev)
+    k = to_dev(_bf(rng.standard_normal((sk, h, 128)) + 2.0 * rng.standard_normal((1, h, 128))), dev)
+    v = to_dev(_bf(rng.standard_normal((sk, h, 128))), dev)
 
     def fn():
         return (attention.attention(q, k, v, config=config),)
