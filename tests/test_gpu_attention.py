@@ -4,7 +4,7 @@ tighter than the north star's 1e-2) of the oracle's float64 attention on the sam
 import numpy as np
 import pytest
 
-from conftest import to_dev, to_np
+from conftest import attention_plan, on_256_cus, to_dev, to_np
 from oracle import attn as oa
 from oracle.gemm import rel_l2
 from oracle.numerics import bf16_to_f32, f32_to_bf16
@@ -74,6 +74,7 @@ def test_prepass_launch_forms(dev, sq, sk, h, rr, smooth):
     """The per-block pre-pass in two launches (up to 4,096 keys) and in separate ones, on both sides of the line and
     at ragged ends: codes, scales, kmean and the V^T layout bit-exact against the oracle."""
     from rapid_h3 import attention
+    assert attention_plan(sq, sk, h)[3] == (sk <= 4096)
     rng = np.random.default_rng(sq * 11 + sk * 3 + h)
     q = _bf(rng.standard_normal((sq, h, 128)))
     k = _bf(rng.standard_normal((sk, h, 128)) + 2.0 * rng.standard_normal((1, h, 128)))
@@ -147,6 +148,7 @@ def test_attention_128_query_kernel(dev, sq, sk, h):
     quantizes them) agree bit for bit; sampled rows against the oracle."""
     import torch
     from rapid_h3 import attention
+    assert not on_256_cus() or attention_plan(sq, sk, h, raw=True)[:2] == (128, 1)
     rng = np.random.default_rng(sq + 3 * sk + h)
     q, k, v = (_bf(rng.standard_normal((n, h, 128)) + off) for n, off in
                ((sq, 0.0), (sk, 2.0 * rng.standard_normal((1, h, 128))), (sk, 0.0)))
@@ -162,14 +164,20 @@ def test_attention_128_query_kernel(dev, sq, sk, h):
 
 
 def test_attention_query_kernels_agree(dev):
-    """2,816 queries of 24 heads fill the chip with 384-query workgroups; the first 1,024 of them alone run on the
-    128-query kernel: the same rows, bit for bit (on 256 CUs; elsewhere both may run on one kernel)."""
+    """The three forms of the main kernel agree bit for bit (no split round in any): 2,816 queries of 24 heads on
+    384-query workgroups, their first 1,024 alone on 128-query workgroups, and the one call, whose 128-query workgroups
+    quantize the queries themselves."""
     import torch
     from rapid_h3 import attention
     g = torch.Generator().manual_seed(4)
     q, k, v = (torch.randn(2816, 24, 128, generator=g).to(torch.bfloat16).to(dev) for _ in range(3))
-    whole = attention.attention(q, k, v)
-    assert torch.equal(attention.attention(q[:1024], k, v), whole[:1024])
+    if on_256_cus():
+        assert attention_plan(2816, 2816, 24)[:3] == (384, 0, 0)
+        assert attention_plan(1024, 2816, 24)[:3] == (128, 0, 0)
+        assert attention_plan(2816, 2816, 24, raw=True)[:3] == (128, 1, 0)
+    whole = attention.forward(attention.prepass(q, k, v), 2816)
+    assert torch.equal(attention.forward(attention.prepass(q[:1024], k, v), 1024), whole[:1024])
+    assert torch.equal(attention.attention(q, k, v), whole)
 
 
 @pytest.mark.parametrize("sq,sk,h", [(130, 65, 2), (9000, 129, 24)])
@@ -205,11 +213,10 @@ def test_attention_out_over_operands(dev, where):
     if where == "value":
         q = q[:sk].contiguous()
     want = attention.attention(q, k, v)
-    if where == "value":
-        out = v
-    else:
-        out = q if where == "in place" else q.view(h, s, 128).transpose(0, 1)
-    assert out.data_ptr() == (v if where == "value" else q).data_ptr()
+    out = {"in place": q, "head-major": q.view(h, -1, 128).transpose(0, 1), "value": v}[where]
+    if on_256_cus():   # the main kernel reads raw queries but where other workgroups' rows may lie on them
+        plan = attention_plan(q.shape[0], sk, h, q=(q.data_ptr(), *q.stride()[:2]), out=(out.data_ptr(), *out.stride()[:2]))
+        assert plan[:2] == (128, int(where != "head-major"))
     attention.attention(q, k, v, out=out)
     assert torch.equal(out.contiguous().view(torch.int16), want.view(torch.int16))
 
@@ -233,37 +240,48 @@ def test_attention_strided_out(dev):
     assert rel_l2(got, ref) < GUARD
 
 
-@pytest.mark.parametrize("sk,head_major", [(2600, False), (1100, True), (2600, "padded")])
-def test_attention_split_tail(dev, sk, head_major):
+def _split_heads(sq, sk, raw):
+    """Fewest heads for which this device's 384-query grid leaves at least 16 workgroups for key halves, and how many."""
+    for h in range(1, 1000):
+        bq, _, npair, _ = attention_plan(sq, sk, h, raw=raw)
+        if bq == 384 and npair >= 16:
+            return h, npair
+    raise AssertionError("no such grid")
+
+
+@pytest.mark.parametrize("sk,out_form,one_call", [(5583, "token-major", True), (1100, "head-major", False),
+                                                  (2600, "padded", False)])
+def test_attention_split_tail(dev, sk, out_form, one_call):
     """A grid whose last round (one workgroup of 384 queries per CU) is at most half full: those workgroups
-    run as two key halves, each writing fp32 partials, merged by attn_combine_kernel. H is chosen from the
-    device's CU count so that 7 query blocks x H heads leave 16..cus/2 workgroups in the last round; the
-    heads holding them and head 0 (unsplit) against the oracle. Self-attention with [S, H, D] output, and
-    cross-attention (1,100 keys: 18 steps, the last ragged) into a head-major [1, H, S, D] buffer, and an output
-    view whose head stride is 4 mod 8 elements (132: the merge kernel's stores must not assume 16-byte alignment)."""
-    import torch
+    run as two key halves, each writing fp32 partials, merged by attn_combine_kernel. H is chosen by the device's own
+    plan, so that 7 query blocks x H heads leave at least 16 workgroups in the last round; some of the heads holding them
+    and head 0 (unsplit) against the oracle. The one call with [S, H, D] output (5,583 keys), and the split pair into a
+    head-major [1, H, S, D] buffer (1,100 keys: 18 steps, the last ragged) and into a view whose head stride is 4 mod 8
+    elements (132: the merge kernel's stores must not assume 16-byte alignment)."""
     from rapid_h3 import attention
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    s, nqb = 2600, 7  # 7 query blocks of 384; 2,600 keys = 41 key steps of 64, the last one ragged
-    h = next(hh for hh in range(1, 100000) if nqb * hh > cus and 16 <= (nqb * hh) % cus <= min(cus // 2, 128))
-    last = (nqb * h) % cus
+    import torch
+    s, nqb = 2600, 7  # 7 query blocks of 384
+    h, last = _split_heads(s, sk, one_call)
     tail_heads = sorted({i // nqb for i in range(nqb * h - last, nqb * h)})
+    tail_heads = sorted({tail_heads[0], tail_heads[len(tail_heads) // 2], tail_heads[-1]})
     rng = np.random.default_rng(21 + sk)
     q = _bf(rng.standard_normal((s, h, 128)))
     k = _bf(rng.standard_normal((sk, h, 128)) + 2.0 * rng.standard_normal((1, h, 128)))
     v = _bf(rng.standard_normal((sk, h, 128)))
-    if head_major == "padded":
-        o = torch.empty(s, h, 132, dtype=torch.bfloat16, device=dev)
-        attention.attention(to_dev(q, dev), to_dev(k, dev), to_dev(v, dev), out=o[:, :, :128])
-        out = bf16_to_f32(to_np(o[:, :, :128]))
-    elif head_major:
-        o = torch.empty(1, h, s, 128, dtype=torch.bfloat16, device=dev)
-        attention.attention(to_dev(q, dev), to_dev(k, dev), to_dev(v, dev), out=o[0].transpose(0, 1))
-        out = bf16_to_f32(to_np(o[0].transpose(0, 1)))
+    if out_form == "padded":
+        o = torch.empty(s, h, 132, dtype=torch.bfloat16, device=dev)[:, :, :128]
+    elif out_form == "head-major":
+        o = torch.empty(1, h, s, 128, dtype=torch.bfloat16, device=dev)[0].transpose(0, 1)
     else:
-        out = bf16_to_f32(to_np(attention.attention(to_dev(q, dev), to_dev(k, dev), to_dev(v, dev))))
+        o = torch.empty(s, h, 128, dtype=torch.bfloat16, device=dev)
+    args = (to_dev(q, dev), to_dev(k, dev), to_dev(v, dev))
+    if one_call:
+        attention.attention(*args, out=o)
+    else:
+        attention.forward(attention.prepass(*args), s, out=o)
+    out = bf16_to_f32(to_np(o))
     assert np.isfinite(out).all()
-    for hh in [0] + tail_heads:
+    for hh in sorted({0, *tail_heads}):
         q8, qs, k8, ks, _ = oa.prepass(q[:, hh:hh + 1], k[:, hh:hh + 1])
         ref = oa.attention_from_codes(q8, qs, k8, ks, v[:, hh:hh + 1], 128 ** -0.5)[:s, 0]
         assert rel_l2(out[:, hh], ref) < GUARD, hh
@@ -275,24 +293,28 @@ def test_attention_split_tail(dev, sk, head_major):
 
 
 def test_attention_split_switch(dev, monkeypatch):
-    """RH3_ATTN_SPLIT=0 runs the last round whole: the same grid as test_attention_split_tail with and without the
-    split gives outputs within the tolerance of each other (the split sums each key half in fp32 and merges, so the
-    bits may differ), and the unsplit output also against the oracle."""
-    import torch
+    """RH3_ATTN_SPLIT=0 runs every workgroup whole: the grid of test_attention_split_tail with and without the split gives
+    outputs within the tolerance of each other (the split sums each key half in fp32 and merges, so the bits of the split
+    workgroups differ, and only theirs), and the unsplit output also against the oracle."""
     from rapid_h3 import attention
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    s, nqb = 2600, 7
-    h = next(hh for hh in range(1, 100000) if nqb * hh > cus and 16 <= (nqb * hh) % cus <= min(cus // 2, 128))
+    monkeypatch.delenv("RH3_ATTN_SPLIT", raising=False)
+    s, sk, nqb = 2600, 5583, 7
+    h, last = _split_heads(s, sk, True)
     rng = np.random.default_rng(77)
     q = _bf(rng.standard_normal((s, h, 128)))
-    k = _bf(rng.standard_normal((s, h, 128)) + 2.0 * rng.standard_normal((1, h, 128)))
-    v = _bf(rng.standard_normal((s, h, 128)))
+    k = _bf(rng.standard_normal((sk, h, 128)) + 2.0 * rng.standard_normal((1, h, 128)))
+    v = _bf(rng.standard_normal((sk, h, 128)))
     args = (to_dev(q, dev), to_dev(k, dev), to_dev(v, dev))
-    split = bf16_to_f32(to_np(attention.attention(*args)))
+    split = to_np(attention.attention(*args))
     monkeypatch.setenv("RH3_ATTN_SPLIT", "0")
-    whole = bf16_to_f32(to_np(attention.attention(*args)))
+    assert attention_plan(s, sk, h, raw=True)[2] == 0
+    whole = to_np(attention.attention(*args))
     monkeypatch.delenv("RH3_ATTN_SPLIT")
-    assert rel_l2(split, whole) < GUARD
+    first = (nqb * h - last) // nqb                          # the first head with a split workgroup
+    assert np.array_equal(split[:, :first], whole[:, :first])
+    assert (split[:, first + 1:] != whole[:, first + 1:]).any(axis=(0, 2)).all()
+    split, whole = bf16_to_f32(split), bf16_to_f32(whole)
+    assert rel_l2(split[:, first:], whole[:, first:]) < GUARD
     hh = h - 1                                               # the last head holds split workgroups
     q8, qs, k8, ks, _ = oa.prepass(q[:, hh:hh + 1], k[:, hh:hh + 1])
     ref = oa.attention_from_codes(q8, qs, k8, ks, v[:, hh:hh + 1], 128 ** -0.5)[:s, 0]
@@ -307,8 +329,8 @@ def test_attention_work_counter_reused(dev):
     import torch
     from rapid_h3 import attention
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    s = 1500
-    h = cus // 2 + 3                                         # 4 query blocks per head: more items than CUs
+    s, nqb = 2600, 7                                         # 7 query blocks of 384 per head
+    h = next(hh for hh in range(1, 1000) if nqb * hh > cus and attention_plan(s, s, hh)[0] == 384)
     rng = np.random.default_rng(5)
     q = _bf(rng.standard_normal((s, h, 128)))
     k = _bf(rng.standard_normal((s, h, 128)) + 2.0 * rng.standard_normal((1, h, 128)))
