@@ -236,7 +236,7 @@ __device__ __forceinline__ void wht128_row(float* v, int l16) {
   for (int e = 0; e < 8; ++e) v[e] = v[e] * 0.08838834764831845f;
 }
 
-// absmax of the 16-lane row (lanes of one row group)
+// absmax of the 16-lane row (lanes of one row group); quiet NaNs are skipped, signalling ones must not come here
 __device__ __forceinline__ float row_amax16(const float* v) {
   float amax = 0.0f;
 #pragma unroll

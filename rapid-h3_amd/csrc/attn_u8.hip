@@ -104,6 +104,24 @@ __device__ __forceinline__ void vstats_chunk(const uint16_t* __restrict__ v, int
     if (static_cast<int64_t>(c + 1) * CHUNK <= S) rows(std::true_type{});   // uniform: no row of the chunk past S
     else rows(std::false_type{});
   }
+  // max3 and min3 skip a quiet NaN, but a signalling one replaces what they held: a lane whose sums met any NaN takes its
+  // maxima and minima again, value by value
+  bool nan = false;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) nan |= acc[e] != acc[e];
+  if (nan) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { mx[e] = -INFINITY; mn[e] = INFINITY; }
+    for (int64_t s = static_cast<int64_t>(c) * CHUNK + slot; s < S && s < static_cast<int64_t>(c + 1) * CHUNK; s += 16) {
+      float x[8];
+      unpack8(*reinterpret_cast<const uint4*>(v + s * v_ss + h * v_sh + 8 * l16), x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        mx[e] = fmaxf(mx[e], x[e]);
+        mn[e] = fminf(mn[e], x[e]);
+      }
+    }
+  }
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     red[slot][8 * l16 + e] = acc[e];
@@ -213,6 +231,10 @@ __device__ __forceinline__ void tokq_rows(const uint16_t* __restrict__ x, int64_
       for (int e = 0; e < 8; ++e) v[e] = v[e] - m[e];
     }
     if (rotate) wht128_row(v, l16);
+    if (!rr.tab && !mean && !rotate) {   // the raw values: row_amax16 takes no signalling NaN
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = __builtin_canonicalizef(v[e]);
+    }
     uint2 o;
     const float sc = token_quant_row(v, o);
     *reinterpret_cast<uint2*>(co + u * D) = ok ? o : make_uint2(0, 0);   // padded rows and keys: zero codes

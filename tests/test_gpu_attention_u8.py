@@ -95,6 +95,38 @@ def test_u8_prepass_merged(dev, sq, sk, h, rot, flags):
         assert np.array_equal(to_np(pf[n]), ef[n]), n
 
 
+@pytest.mark.parametrize("s", [300, 512])
+def test_u8_prepass_signalling_nan(dev, s):
+    """A signalling NaN is skipped in the maxima like a quiet one: beside it, a V channel's largest and least value (two
+    tokens apart by 16 sit in one lane, read together) and a token's largest channel still set their scales. Without
+    smoothing and rotation, whose arithmetic would quiet or spread it; full and ragged statistics chunks."""
+    from rapid_h3 import attention
+    h = 2
+    rng = np.random.default_rng(s)
+    f = [(0.5 * rng.standard_normal((s, h, 128))).astype(np.float32) for _ in range(3)]
+    q, k, v = (f32_to_bf16(t) for t in f)
+    big = f32_to_bf16(np.array([40.0, -40.0], np.float32))
+    bad = [np.zeros((s, h, 128), bool) for _ in range(3)]
+    for t in (3, 256 + 3):                                       # both chunks; the second one is ragged at s = 300
+        v[t, :, 8:16], v[t, :, 16:24] = big[0], big[1]
+        bad[2][t + 16, :, 8:24] = True
+    for x, b in ((q, bad[0]), (k, bad[1])):
+        x[5, :, 32] = big[0]
+        b[5, :, 33] = True                                       # the same lane
+        x[9, :, 71], b[9, :, 64:71] = big[1], True
+    runs = []
+    for nan in (0x7FA0, 0x7FE0):                                 # signalling, quiet
+        for x, b in zip((q, k, v), bad):
+            x[b] = nan
+        runs.append(attention.prepass_u8(*(to_dev(t, dev) for t in (q, k, v)), smooth_k=False, smooth_v=False, rotate=False))
+    sn, qn = runs
+    for n in ("q8", "qs", "k8", "ks", "ksb", "vt", "vinit", "vscale"):
+        assert np.array_equal(to_np(sn[n]), to_np(qn[n])), n
+    assert np.array_equal(to_np(sn["vscale"])[:, 8:24], np.full((h, 16), np.float32(40) / np.float32(127)))
+    for n in ("qs", "ks"):
+        assert (to_np(sn[n])[:, [5, 9]] == np.float32(40) / np.float32(127)).all(), n
+
+
 def test_ext_int8_prepass_golden(dev, golden):
     """attn_int8.ext().int8_prepass, the reference extension's verification entry (attn_int8.cu:2692-2704, called
     by _rr_check, __init__.py:342-343): the operand list [q8, qs, k8, ks, ksb, vt, vscale, vmean] bit-exact against
