@@ -1,6 +1,6 @@
 // Small-tile forms of the GEMM (gemm.hip) for calls whose 256 x 256 tiles would leave CUs without work: the same
-// operands, epilogues and arithmetic (int8: the same int32 accumulators and the same rounding steps, so the same bits;
-// e4m3: fp32 sums, split in two halves of K where KG is 2).
+// operands, epilogues and arithmetic, so the same bits: int32 accumulators are exact in any order, and an e4m3 call adds
+// its k-steps one after the other on every tile (KG 1), so a row's result does not depend on the rows beside it.
 #include "gemm_common.hpp"
 
 namespace rh3 {
@@ -8,7 +8,7 @@ namespace gemm {
 namespace {
 
 // TM x TN outputs per workgroup, KG groups of WGM x WGN waves. Group kg runs its share of the k-steps on the whole
-// tile through a ring of its own (NST stages of (TM + TN) x 64 bytes); with KG = 2 the two groups' accumulators are
+// tile through a ring of its own (NST stages of (TM + TN) x 64 bytes); with KG = 2 (int8) the two groups' accumulators are
 // added through LDS before the epilogue, each group finishing half of the tile's rows.
 template <int TM_, int TN_, int WGM_, int WGN_, int KG_, int NST_>
 struct Tile {
@@ -30,10 +30,19 @@ __device__ __forceinline__ void wait_vm_lds() {  // at most N vector memory oper
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
 
+// A 16-pass MFMA (e4m3) needs 20 wait states before its result is read; hipcc (ROCm 7.2) looks back over 19 and can leave a
+// read exactly there, which then finds the register of before. Called after the last MFMAs of a path to the epilogue.
+__device__ __forceinline__ void mfma_settle() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_nop 15\n\ts_nop 3");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 template <bool FP8, int EPI, typename T>
 __global__ void __launch_bounds__(T::NT, T::NT == 256 ? 2 : T::NW / 4) gemm_tile_kernel(const GemmArgs a) {
   using MM = Mma<FP8>;
   using acc_t = typename MM::acc_t;
+  static_assert(!FP8 || T::KG == 1, "an fp32 sum keeps its order");
   constexpr int TM = T::TM, TN = T::TN, TI = T::TI, TJ = T::TJ, WM = T::WM, WN = T::WN, NST = T::NST, LW = T::LW;
   __shared__ __attribute__((aligned(16))) int8_t ring[T::LDS];
   __shared__ __attribute__((aligned(16))) float rec[TM + 2 * TN];  // xs, ws, bias / gate of the tile
@@ -192,21 +201,16 @@ __global__ void __launch_bounds__(T::NT, T::NT == 256 ? 2 : T::NW / 4) gemm_tile
     step(s + 1, cur, ODD);
     cur = next(cur);
   }
+  if constexpr (FP8) mfma_settle();
   if (s < nmin) {
     step(s, cur, EVEN);
     cur = next(cur);
-    ++s;
+    if constexpr (FP8) mfma_settle();
   }
   if (T::KG > 1 && (nk & 1) && kg == 0) {  // the odd step, already landed: no copy and no barrier of its own
-    if constexpr (MM::KSUB == 2) {
-      load_frags(cur, 1, fa1, fb1);
-      mma_all(fa0, fb0);
-      mma_all(fa1, fb1);
-    } else if (s & 1) {
-      mma_all(fa1, fb1);
-    } else {
-      mma_all(fa0, fb0);
-    }
+    load_frags(cur, 1, fa1, fb1);
+    mma_all(fa0, fb0);
+    mma_all(fa1, fb1);
   }
   __builtin_amdgcn_sched_barrier(0);
   wait_vm_lds<0>();  // no copy is in flight and no LDS read pending: the ring is free past the barrier
@@ -232,8 +236,7 @@ __global__ void __launch_bounds__(T::NT, T::NT == 256 ? 2 : T::NW / 4) gemm_tile
 #pragma unroll
         for (int rq = 0; rq < 4; ++rq) {
           const acc_t& c = acc[i][O * TJO + j];
-          *xslot(O, j, i, rq) = make_int4(acc_bits(c[4 * rq]), acc_bits(c[4 * rq + 1]), acc_bits(c[4 * rq + 2]),
-                                          acc_bits(c[4 * rq + 3]));
+          *xslot(O, j, i, rq) = make_int4(c[4 * rq], c[4 * rq + 1], c[4 * rq + 2], c[4 * rq + 3]);
         }
   };
   if constexpr (T::KG == 2) {
@@ -258,11 +261,10 @@ __global__ void __launch_bounds__(T::NT, T::NT == 256 ? 2 : T::NW / 4) gemm_tile
 #pragma unroll
           for (int rq = 0; rq < 4; ++rq) {
             const int4 v = *xslot(O, jo, i, rq);
-            typedef decltype(acc[0][0][0] + acc[0][0][0]) elem_t;
-            acc[i][j][4 * rq] += __builtin_bit_cast(elem_t, v.x);
-            acc[i][j][4 * rq + 1] += __builtin_bit_cast(elem_t, v.y);
-            acc[i][j][4 * rq + 2] += __builtin_bit_cast(elem_t, v.z);
-            acc[i][j][4 * rq + 3] += __builtin_bit_cast(elem_t, v.w);
+            acc[i][j][4 * rq] += v.x;
+            acc[i][j][4 * rq + 1] += v.y;
+            acc[i][j][4 * rq + 2] += v.z;
+            acc[i][j][4 * rq + 3] += v.w;
           }
       }
       if constexpr (EPI == EPI_ACC) {
@@ -373,7 +375,12 @@ int launch(GemmArgs a, hipStream_t st, const char* name) {
 }
 
 // The built tiles, small to large. One workgroup of any of them fills a CU's LDS but for the 128 x 128 one (two fit).
-typedef Tile<128, 64, 2, 2, 2, 5> T128x64;
+// The smallest is bound by its serial k-steps, which two wave groups halve where sums are exact in any order. The e4m3
+// form keeps one chain of 4 waves of 32 x 64 outputs (us, two halves of K / one chain: 77 x 3072 -> 9216 9.1 / 10.7,
+// 77 x 8192 -> 3072 17.8 / 21.5, 226 x 8192 -> 3072 25.1 / 24.6, 512 x 3072 -> 3072 11.8 / 10.8; 64 x 32 outputs a wave
+// 10.8, 23.0, 24.5, 11.1; 8 waves of 32 x 32 12.0, 26.7, 26.7, 12.0).
+template <bool FP8>
+using T128x64 = std::conditional_t<FP8, Tile<128, 64, 4, 1, 1, 8>, Tile<128, 64, 2, 2, 2, 5>>;
 typedef Tile<128, 128, 2, 2, 1, 4> T128x128;
 typedef Tile<256, 128, 4, 2, 1, 6> T256x128;
 typedef Tile<256, 192, 4, 2, 1, 5> T256x192;
@@ -381,7 +388,7 @@ typedef Tile<256, 192, 4, 2, 1, 5> T256x192;
 template <bool FP8, int EPI>
 int launch_cfg(int cfg, const GemmArgs& a, hipStream_t st, const char* name) {
   switch (cfg) {
-    case TILE_128x64: return launch<FP8, EPI, T128x64>(a, st, name);
+    case TILE_128x64: return launch<FP8, EPI, T128x64<FP8>>(a, st, name);
     case TILE_128x128: return launch<FP8, EPI, T128x128>(a, st, name);
     case TILE_256x128: return launch<FP8, EPI, T256x128>(a, st, name);
     default: return launch<FP8, EPI, T256x192>(a, st, name);

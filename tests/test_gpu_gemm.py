@@ -170,6 +170,33 @@ def test_gemm_tile_rules(dev, m, n, k, tile):
     assert np.all(np.abs(got - a @ b.T) <= k * 2.0 ** -24 * (np.abs(a) @ np.abs(b).T))
 
 
+@pytest.mark.parametrize("k,form", [(3072, GEMM_SHARES), (3136, GEMM_SINGLE)])
+def test_fp8_rows_independent_of_the_call(dev, k, form):
+    """A row's FP8 accumulators are the same bits in a call of any number of rows: every tile adds a row's k-steps in
+    the same order (even and odd counts of them). Codes of all exponents, so another order would round differently.
+    Row counts for each tile (on 256 CUs), whole rounds of 256 x 256 with the last rows on a small tile, and 256 x 256
+    alone, against counted 256 x 256 tiles or a workgroup each. The plain epilogue gives bf16((acc xs) ws) bit for bit."""
+    import torch
+    from rapid_h3 import gemm
+    n, most = 3072, 23000
+    rng = np.random.default_rng(k)
+    fq, fwq = (rng.integers(0, 256, size=t, dtype=np.uint8) for t in ((most, k), (n, k)))
+    for c in (fq, fwq):
+        c[(c & 0x7F) == 0x7F] = 0                                # no NaN codes
+    xt, wt = to_dev(fq, dev, "fp8"), to_dev(fwq, dev, "fp8")
+    acc = gemm.fp8_gemm_acc(xt, wt)
+    want = to_np(acc)
+    xs, ws = (to_dev((rng.random(t) + 0.5).astype(np.float32), dev) for t in ((most, 1), (1, n)))
+    out = to_np(((acc * xs) * ws).to(torch.bfloat16))
+    for m, plan in ((1, (128, 64, 0, GEMM_SMALL)), (77, (128, 64, 0, GEMM_SMALL)), (1280, (128, 128, 0, GEMM_SMALL)),
+                    (2560, (256, 128, 0, GEMM_SMALL)), (3000, (256, 192, 0, GEMM_SMALL)), (5442, (128, 64, 5376, form)),
+                    (10752, (256, 256, 10752, form))):
+        assert not on_256_cus() or gemm_plan(m, n, k) == plan
+        assert np.array_equal(to_np(gemm.fp8_gemm_acc(xt[:m], wt)), want[:m]), m
+        assert np.array_equal(to_np(gemm.fp8_gemm(xt[:m], xs[:m], wt, ws)), out[:m]), m
+    assert np.array_equal(to_np(gemm.fp8_gemm(xt, xs, wt, ws)), out)
+
+
 @pytest.mark.parametrize("m,n,k,form", [(4100, 15616, 512, GEMM_COUNTED), (8200, 8208, 768, GEMM_COUNTED),
                                         (5300, 6096, 512, GEMM_SHARES), (9000, 8200, 256, GEMM_SINGLE),
                                         (4500, 4112, 512, GEMM_SMALL), (700, 784, 1024, GEMM_SMALL),
