@@ -429,8 +429,8 @@ __device__ __forceinline__ void vq_tile(const uint16_t* __restrict__ v, int64_t 
 // A: K statistics (smoothing), V statistics and the Q quantizer; kmean_vfinal_kernel: their second level; B: the K quantizer
 // and the V codes. The parts of one launch do not depend on each other; run as eight launches of their own, the small ones cost
 // more in launch gaps than in work and the memory-bound ones ran beside no arithmetic. Whole pre-pass with RMSNorm + RoPE (us,
-// before and now): 1,560 tokens x 24 heads 60 and 42, 5,583 x 56 193 and 168, 22,332 x 56 670 and 611; A is bound by VALU
-// (94 % busy), B by VALU and HBM together.
+// before and now): 1,560 tokens x 24 heads 60 and 42, 5,583 x 56 193 and 168, 22,332 x 56 670 and 611. Both are bound by VALU
+// issue (A 79 %, B 74 % busy at 5,583 x 56, both saturated at 145,152 x 24), with 3.1 to 3.8 waves per SIMD.
 struct PreU8 {
   const uint16_t *q, *k, *v;
   int64_t q_ss, q_sh, k_ss, k_sh, v_ss, v_sh;

@@ -65,8 +65,9 @@ __device__ __forceinline__ void st_stream8(void* p, uint2 v) {
 }
 
 // Buffer-resource accesses: word 3 of a raw (stride 0) gfx9 buffer descriptor (32-bit data format), and the
-// nontemporal cache policy bit. A load whose byte offset (lane offset + immediate) lies at or past the
-// descriptor's size returns 0 and such a store is dropped, so a row's tail needs no branch.
+// nontemporal cache policy bit. A load whose byte offset (lane offset + immediate + scalar offset:
+// without a stride the check is against the size less the scalar offset) lies at or past the descriptor's size returns 0
+// and such a store is dropped, so a row's tail needs no branch.
 constexpr int BUF_RSRC_WORD3 = 0x00020000;
 constexpr int BUF_NT = 2;
 

@@ -117,10 +117,9 @@ __device__ __forceinline__ v4f_t mfma_bf16(const uint4 a, const uint4 b, v4f_t c
 // among them), takes the float64 butterflies instead (h64_slow): about 1 in 50 of the wave's chunks for normal values
 // with 1 % of the channels x20, 1 in 1000 for normal values.
 //
-// What bounds it: VALU issue (72 % busy at 145,152 x 3072 with RMSNorm + modulation, 4 waves per SIMD), then HBM. With the
-// butterflies of all chunks in float64 a row of 3072 took 1,035 VALU instructions per wave (a third of them float64), now
-// about 500. Measured at 145,152 x 3072: RMSNorm + modulation 0.498 -> 0.397 ms; head-major 22,332 x 7168 0.132 ->
-// 0.102 ms = 4.7 TB/s. The operand table stays in LDS: in registers (32 of them) only 3 waves fit a SIMD (0.495 ms), and a
+// What bounds it: VALU issue (70-75 % busy at 145,152 x 3072, 4 waves per SIMD), then HBM. VALU instructions per row of 3072,
+// with the butterflies of all chunks in float64 and now: RMSNorm + modulation 1,777 and 1,187, head-major 1,097 and 708.
+// Measured at 145,152 x 3072: RMSNorm + modulation 0.498 -> 0.397 ms; head-major 22,332 x 7168 0.132 -> 0.102 ms = 4.7 TB/s. The operand table stays in LDS: in registers (32 of them) only 3 waves fit a SIMD (0.495 ms), and a
 // workgroup that walks several tiles spills (0.79 ms).
 //
 // H64 / 8 as that operand: H4[a][b] = -1 where b = 3 - a, +1 elsewhere; row i = 16 T + (l & 15) and column

@@ -2,7 +2,7 @@
 
 Signatures follow the reference's cutlass_fp8 wrappers (/root/reference/custom_nodes/rapid_h3/
 cutlass_fp8.py:32-67): scales may be [M, 1] / [1, N] or 1-D; the `config` tile id is accepted and
-ignored (this backend has one gfx950 schedule per epilogue).
+ignored (the tile of a call follows from its sizes and the CU count).
 """
 import torch
 
