@@ -13,7 +13,7 @@ with 1 % of channels x20, weights N(0, 0.02) random init, modulation and norm we
                     [--recipe int8_rot] [--attn-config 94] [--model h3]
 
 After the timed block (outside the timed region): the C3 FP8 GEMMs at the three C2 shapes and hipBLASLt's int8
-GEMM (torch._int_mm) beside this build's at the four block shapes (fp8_gemm_c3, int8_gemm_vs_hipblaslt), one block
+GEMM (torch._int_mm) beside this library's at the four block shapes (fp8_gemm_c3, int8_gemm_vs_hipblaslt), one block
 at MiniMax-H3's shapes (h3_shapes), one block in the reference's preset numerics (reference_preset: int8_rot
 quantizers, attention config 94), and the CPU baseline (cpu_baseline) on the same block's inputs.
 
@@ -39,7 +39,7 @@ PEAK_HBM_GBS = 8000.0          # MI355X HBM3E
 PEAK_FP8_TFLOPS = 5033.0       # MI355X dense OCP-FP8 MFMA
 D = 128
 MODELS = {  # hidden, heads, FFN width, default tokens
-    "c2": (3072, 24, 8192, 145152),    # BASELINE.json configs C2 / C4: 36 x 48 x 84 latent patches
+    "c2": (3072, 24, 8192, 145152),    # the full-size block: 36 x 48 x 84 latent patches
     "h3": (5376, 56, 14336, 44992),    # MiniMax-H3 (the reference's bench/microbench.py:15, docs/kernels.md:405)
 }
 HIDDEN, HEADS, FFN, _ = MODELS["c2"]
@@ -103,8 +103,8 @@ def setup(m, device, recipe="int8_rowwise"):
 
 
 def _cpu_threads():
-    """Threads for the CPU baseline: every core this process may run on (os.sched_getaffinity; on the GPU box that
-    is the job's share, where os.cpu_count() counts the whole host), set for torch and numpy's BLAS alike."""
+    """Threads for the CPU baseline: every core this process may run on (os.sched_getaffinity: the
+    job's share, where os.cpu_count() counts the whole host), set for torch and numpy's BLAS alike."""
     n = len(os.sched_getaffinity(0)) if hasattr(os, "sched_getaffinity") else os.cpu_count()
     import torch
     torch.set_num_threads(n)
@@ -142,7 +142,7 @@ def _median_time(fn, runs=5, warmup=1):
 def cpu_baseline(m, x, w, mod, segments, tab, trace, ms=4096, rows=1024):
     """The CPU baseline: the build's CPU restatement of the reference's PyTorch path (oracle/, a numpy port:
     kernels.quantize_rows / quantize_weight, the exact int32 product, the (acc * xs) * ws epilogues, the per-block
-    attention emulation), on the host cores of the GPU box, each part the median of 5 runs after 1 warm-up, sampled
+    attention emulation), on the host's cores, each part the median of 5 runs after 1 warm-up, sampled
     as follows:
       * C1 (X [4096, 3072] with 1 % outlier channels, W [3072, 3072] ~ N(0, 0.02), seed 0): measured in full;
       * C2: each of the block's four GEMMs with the quantizer that feeds it, on the first `ms` = 4,096 tokens of the
@@ -163,7 +163,7 @@ def cpu_baseline(m, x, w, mod, segments, tab, trace, ms=4096, rows=1024):
         t = t.detach().cpu()
         return t.view(torch.int16).numpy().view(np.uint16) if t.dtype == torch.bfloat16 else t.numpy()
 
-    # C1 in full, generated on the CPU as BASELINE.json's config C1 (seed 0)
+    # C1 in full, generated on the CPU (seed 0)
     g = torch.Generator().manual_seed(0)
     x1 = torch.randn(4096, 3072, generator=g)
     x1[:, torch.randperm(3072, generator=g)[:31]] *= 20
@@ -507,7 +507,7 @@ def main():
                     help="run only the attention kernel + a 1 GiB copy (workload of the --pmc passes)")
     a = ap.parse_args()
     if a.gpus != 1:
-        print(f"bench.py: this build runs on one GPU; --gpus {a.gpus} is not supported (no multi-GPU path)",
+        print(f"bench.py: runs on one GPU; --gpus {a.gpus} is not supported (no multi-GPU path)",
               file=sys.stderr)
         sys.exit(2)
     global HIDDEN, HEADS, FFN

@@ -11,7 +11,7 @@ Reference semantics followed:
                                    [S, rot/2, 2, 2] = (cos, -sin, sin, cos) from bench/rmsrope_fuse.py:22-33
   * attention                      attn_int8.cu:602-709: softmax(scale * q.k) v, non-causal, D = 128
 
-Orders fixed by this build (both sides use them, so Q/K codes and scales are bit-exact):
+Orders fixed here (both sides use them, so Q/K codes and scales are bit-exact):
   * kmean: float64 sum over all S tokens, divided by S in float64, rounded once to fp32;
   * RMSNorm sum of squares over D = 128: 16 lanes own channels 8*l + e, accumulate x*x in fp32 for
     e = 0..7 from 0, then a butterfly over lane distances 8, 4, 2, 1;
@@ -169,7 +169,7 @@ def rope_table(positions, rot=96, theta=10000.0):
 #     * P = sat_u8(rint(2^(fma(t, c, fma(-tm, c, log2 255))))), rs = sum P, l = fma(ts, rs, l a)
 #     * O = a O + ts * sum_j P_j v8_j; out = bf16(fma(O (1 / l), vscale, vmean))
 #   text bias (attn_cake.cuh:97-99, :210-240): t += bias*log2(e) / c on keys [0, nbias) after the dequant.
-# Orders fixed by this build: kmean / vmean are float64 sums divided by S in float64 and rounded once (the
+# Orders fixed here: kmean / vmean are float64 sums divided by S in float64 and rounded once (the
 # reference sums in fp32 per 256-token chunk); the Walsh-Hadamard stages are the reference's own (strides
 # 1, 2, ..., 64, each stage rounded to fp32), so codes and scales are bit-exact.
 

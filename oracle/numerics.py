@@ -1,7 +1,7 @@
 """Bit-level number formats for the CPU oracle: bf16 and OCP FP8 e4m3fn, stored as integer arrays.
 
 TEST INFRASTRUCTURE ONLY. Nothing under oracle/ is part of the product: only tests/, the smoke check
-in __graft_entry__.py and bench.py's CPU-baseline leg may import it, and only as the checker.
+in __graft_entry__.py and bench.py's CPU-baseline leg may import it, and only as the oracle.
 
 numpy has no bf16 or fp8 dtype, so tensors of those types travel as uint16 / uint8 bit patterns.
 Conversions follow IEEE round-to-nearest-even, the rounding torch uses for `.to(torch.bfloat16)` and

@@ -1,7 +1,7 @@
 """CPU restatement of the reference's activation and weight quantizers (numpy, float32 arithmetic).
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, __graft_entry__.smoke() and bench.py's CPU baseline, as
-the checker. The product path never calls it.
+the oracle. The product path never calls it.
 
 Semantics are the PyTorch path of the reference, which is the parity target:
   * per-token INT8   /root/reference/custom_nodes/rapid_h3/kernels.py:75-80
@@ -228,7 +228,7 @@ def convrot(x, group=256):
 
 
 def convrot_matmul(x, group=256):
-    """The closed form x @ blockdiag(H)^T in float64 (BLAS order), rounded once to fp32 (a checker)."""
+    """The closed form x @ blockdiag(H)^T in float64 (BLAS order), rounded once to fp32 (a cross-check)."""
     v = _as_f32(x).astype(np.float64)
     m, k = v.shape
     h = regular_hadamard(group)

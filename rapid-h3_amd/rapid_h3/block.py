@@ -16,7 +16,7 @@ int8_rowwise (the same chain without rotation, the configuration the benchmark n
     INT8 of h                                      rh3_quant_rows_i8          / rh3_rot_quant_rows_i8
     FFN-down GEMM + gated residual, per segment    rh3_gemm_i8_gated
 
-ComfyUI objects (the block module, adaln_proj, model management) are outside this build: the caller
+ComfyUI objects (the block module, adaln_proj, model management) are outside this package: the caller
 passes the weights and the modulation tables as tensors.
 """
 from dataclasses import dataclass
@@ -100,7 +100,7 @@ def fused_block(x, w: BlockWeights, mod, segments, rope_tab, idx=None, mark=None
     gate_msa, shift_mlp, scale_mlp, gate_mlp), each [R, hidden]; rope_tab [1, S, 1, rot/2, 2, 2] bf16.
     mark: optional callable, called with each name of PHASES after that phase is enqueued (a timer
     records a stream event there); the kernels and their order are the same with or without it.
-    trace: optional dict that receives every intermediate (a checker's view of each stage).
+    trace: optional dict that receives every intermediate (for comparing each stage).
     attn_config: None runs the per-block bf16 P.V attention; an int runs the reference's production
     numerics with that config (its 1xx presets, __init__.py:274-291), 50-56 its FP8 P.V kernel. text_bias = (nbias, bias) adds the
     Jenga text bias (configs 90 / 94 only). fuse_qkv (even head counts): the QKV GEMM's epilogue writes the

@@ -15,7 +15,7 @@ def int8_gemm_qkv_prep(xq, xs, wq, ws, tab, qw, kw, eps, heads, rotate=True):
     cutlass_fp8.py:42-46): returns (qkv [M, 3*heads*128] bf16 with the q columns left unwritten, q8, qs, part)
     for attn_int8.attention_pre, with the reference's production numerics (per-token Q after the H128
     rotation). q8 / qs / part are views of one attention workspace that attention_pre continues on; part
-    holds the float64 K and V statistics of this build (not the reference's fp32 [H, nchunk, 4, 128])."""
+    holds the float64 K and V statistics (not the reference's fp32 [H, nchunk, 4, 128])."""
     from . import attention as _attn
     from .gemm import int8_gemm_qkv
     m = xq.shape[0]

@@ -8,7 +8,7 @@ Behaviour kept from the reference:
   * exact_rows: a comma-separated list of segment kinds; after the INT8 call the query rows of those
     segments (merged [a, b) spans of transformer_options["minimax_h3_layout"].segments, cached per layout)
     are recomputed exactly (:1006-1022, :1035-1037). The reference uses bf16 scaled_dot_product_attention
-    there; this build computes those rows in fp32 and rounds them to bf16;
+    there; here those rows are computed in fp32 and rounded to bf16;
   * config >= 100 (and no exact_rows) tags the override with rapidh3_rmsrope = config % 100 for the fused
     block, config >= 200 with rapidh3_rrcheck (:1000, :1043-1045);
   * a call carrying transformer_options["rapidh3_text_bias"] with S >= 1024 raises (the bias needs the fused

@@ -24,7 +24,7 @@ attention=None). Its attention follows the reference (:277-306):
     skip_reshape=True, skip_output_reshape=True, transformer_options=...), func being the stock attention
     (`attention`, default override.stock_attention), so the override's own config and exact_rows decide the
     numerics; with no override, func itself runs;
-  * with neither an override nor a stock attention given, this build's per-block INT8 recipe (RMSNorm + RoPE fused
+  * with neither an override nor a stock attention given, the per-block INT8 recipe (RMSNorm + RoPE fused
     in its pre-pass), the attention the benchmark measures.
 Inputs the fused path does not take (not bf16, not 2-D, on the CPU, an attention argument, no rope table) go to the
 block's own forward, as in the reference (:255-258).

@@ -4,8 +4,8 @@
 
 Inputs come from numpy's PCG64 (seeded), so they are the same on every machine; expected outputs
 come from the CPU oracle (oracle/), which tests/test_oracle.py pins independently against torch's
-CPU kernels, closed forms and invariants. The GPU tests load these files, so the GPU box needs
-neither the reference nor the oracle's run time to check the fixture cases.
+CPU kernels, closed forms and invariants. The GPU tests load these files, so they need neither
+the reference nor the oracle's run time for the fixture cases.
 """
 import os
 import sys

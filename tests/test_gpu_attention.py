@@ -1,6 +1,6 @@
 """GPU parity of the INT8 attention (librh3 rh3_int8_attention*, rh3_attention_prepass) against the CPU
 oracle: bit-exact Q/K int8 codes, per-block scales and kmean; V^T layout exact; output within rel-L2 4e-3 (GUARD,
-tighter than the north star's 1e-2) of the oracle's float64 attention on the same int8 operands."""
+tighter than the 1e-2 bar) of the oracle's float64 attention on the same int8 operands."""
 import numpy as np
 import pytest
 
@@ -11,7 +11,7 @@ from oracle.numerics import bf16_to_f32, f32_to_bf16
 
 pytestmark = pytest.mark.gpu
 
-TOL = 1e-2     # the north star's bar for the attention output (rel-L2)
+TOL = 1e-2     # the bar for the attention output (rel-L2)
 # The regression guard every output check here asserts: measured errors against the oracle are 2.25e-3 to 2.40e-3
 # on every case (and 6e-4 between the split and whole schedules), so an error that grows by 70 % fails, well before
 # the 1e-2 bar would.
